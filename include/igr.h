@@ -252,11 +252,10 @@ typedef struct igr_tuning {
     int sched_group;    /* lanes per net in the scheduler's claim and viability kernels: 4, 8 or 16 */
     int sched_chunk;    /* scheduler rounds enqueued between host checks, 1..256 */
     int dag_order;      /* workgroup order of a DAG batch: 1 deepest DAG first, 2 routing order */
-    int dag_waves;      /* DAG kernel register budget: 2 (compiler's choice) or 4 waves per SIMD */
+    int dag_waves;      /* waves per net of the DAG kernel, 2 or 4 */
     int track_k;        /* fused track kernel: cells per thread, 4, 8 or 16 */
-    int dag_edges;      /* layer-change costs: 1 a wave per edge with LDS staging, 2 a thread per layer pair */
-    int dag_seq;        /* DAG levels with at least this many nodes run a node per lane, narrower ones 16
-                           lanes per node (1 << 30: always 16 lanes) */
+    int dag_edges;      /* 1 or 2; one kernel prices the DAG edges, the field has no effect */
+    int dag_seq;        /* one kernel runs every DAG level, the field has no effect */
     int sched_kind;     /* scheduler rounds after the first of a batch: 1 active-list (work follows the
                            active nets), 2 release-driven (work follows the released cells); built-in
                            choice 2 from 1.5M scheduled nets */

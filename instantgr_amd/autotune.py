@@ -7,10 +7,8 @@ results (include/igr.h, igr_tuning):
   sched_chunk  scheduler rounds enqueued between host checks
   graph        one hipGraph per pass for the batch sequence, or stream launches
   dag_order    workgroup order of a DAG batch (deepest DAG first, or routing order)
-  dag_waves    register budget of the DAG kernel (2 or 4 waves per SIMD)
+  dag_waves    waves per net of the DAG kernel (2 or 4)
   track_k      cells per thread of the fused track kernel (4, 8, 16)
-  dag_edges    layer-change costs: a wave per edge with LDS staging, or a thread per layer pair
-  dag_seq      node count from which a DAG level runs a node per lane instead of 16 lanes per node
   sched_kind   scheduler rounds: active-list (work follows the active nets) or release-driven
                (work follows the released cells)
   dag_grid     persistent workgroups of the DAG kernel pulling nets from the batch's work queue
@@ -18,9 +16,9 @@ results (include/igr.h, igr_tuning):
                workgroup holds (their layer-range tables)
 
 In the terms of a tile shape: nets per workgroup (lshape_groups, dag_grid),
-LDS slab size (lshape_groups times the node tables of the node-count class),
-and layers per wave (dag_seq: 16 lanes per node, one layer per lane, four
-nodes per wave; or a node per lane holding all its layers, 64 per wave).
+waves per net (dag_waves) and the LDS slab size (lshape_groups times the node
+tables of the node-count class).  dag_edges and dag_seq have no effect and
+keep one value.
 
 `tune` measures them on a design (normally a reduced sample of the production
 design from the same generator) by coordinate descent: each field in turn takes
@@ -44,8 +42,8 @@ CANDIDATES = {
     "dag_order": [1, 2],
     "dag_waves": [2, 4],
     "track_k": [4, 8, 16],
-    "dag_edges": [1, 2],
-    "dag_seq": [4, 8, 16, 32, 1 << 30],
+    "dag_edges": [1],
+    "dag_seq": [16],
     "sched_kind": [1, 2],
     "dag_grid": [1024, 2048, 4096],
     "lshape_groups": [1, 2, 4],

@@ -553,7 +553,7 @@ void pfor(int64_t cnt, const std::function<void(int64_t, int64_t)>& fn) {
 // batch bounds; the device lays the DAGs out (k_dag_layout) and checks them.
 void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const igr_dag_desc* dg_in,
                       const std::function<void(igr_dag_desc&)>& complete, igr_pass_stats* st) {
-    const int XY = c->g.X * c->g.Y, L = c->g.L, LL = L * L, ML = L + 1;
+    const int XY = c->g.X * c->g.Y, L = c->g.L, ML = L + 1;
     igr_dag_desc dgv = *dg_in;
     const igr_dag_desc* dg = &dgv;
     // The scheduler's points are checked here, the DAG structure on the device.
@@ -688,9 +688,10 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
         lbase[r + 1] = lbase[r] + l_nl[i];
         route_slot[r + 1] = route_slot[r] + 8 * nn + 1;
     }
-    const int64_t NS = sbase[n], NL = lbase[n];
+    const int64_t NL = lbase[n];
     std::vector<DagBatch> batches(nb);
     int64_t mx_nodes = 0, mx_edges = 0, mx_slots = 0;
+    bool any_big = false;
     // Per batch, the routed nets in launch order of the workgroup-per-net
     // kernel: deepest DAG first, then most nodes (dag_order 1), or routing
     // order (2).
@@ -713,12 +714,17 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
         B.slot0 = sbase[B.net0];
         B.slot1 = sbase[B.net1];
         int maxl = 1;
+        int64_t lds = 0;
         for (int64_t r = B.net0; r < B.net1; r++) {
             maxl = std::max(maxl, l_nl[rorder[r]]);
+            const int64_t need = dag_net_lds(nbase[r + 1] - nbase[r], sbase[r + 1] - sbase[r], lbase[r + 1] - lbase[r], L);
+            if (need <= DAG_LDS_MAX) lds = std::max(lds, need);
+            else any_big = true;
             B.bytes_edges += l_eb[rorder[r]];
             B.bytes_dp += l_db[rorder[r]];
         }
         B.levels = maxl;
+        B.lds = (int)lds;
         B.index = b;
         B.lvl0 = 0;
         mx_nodes = std::max(mx_nodes, B.node1 - B.node0);
@@ -750,45 +756,32 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     D.sbase.upload(sbase.data(), n + 1, s);
     D.lbase.upload(lbase.data(), n + 1, s);
     D.route_slot.upload(route_slot.data(), n + 1, s);
-    D.node.alloc(NN);
-    D.child_num.alloc(NN);
-    D.loc.alloc(NN);
-    D.csum.alloc(NN + 1);
-    D.par_off.alloc(NN + 1);
-    D.par.alloc(NE);
-    D.slot.alloc(NE);
-    D.enode.alloc(NE);
-    D.nl_off.alloc(n);
-    D.nlevels.alloc(n);
-    D.lvl_node_off.alloc(NL + n);
-    D.lvl_edge_off.alloc(NL + n);
-    D.cur_n.alloc(NL + n);
-    D.cur_e.alloc(NL + n);
-    D.dnode.alloc(NN);
-    D.dedge.alloc(NE);
+    D.nrec.alloc(NN);
+    D.npos.alloc(NN);
+    D.edge.alloc(NE);
+    D.lvl.alloc(NL + n);
+    D.lcur.alloc(NL + n);
+    D.lpos.alloc(NN);
+    D.lslot.alloc(NN);
     D.err.zero(1, s);
-    const int64_t tails[2] = {NE, NS};
-    HIP_OK(hipMemcpyAsync(D.par_off.p + NN, &tails[0], sizeof(int64_t), hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(D.csum.p + NN, &tails[1], sizeof(int64_t), hipMemcpyHostToDevice, s));
     const double t_meta = now_s();
     DagLayoutArgs la{D.r_node_off.p, D.r_nodes.p, D.r_par_off.p, D.r_par.p, D.r_slot.p, D.r_child_num.p, D.r_depth.p,
-                     D.rorder.p, D.node_off.p, D.ebase.p, D.sbase.p, D.lbase.p, (L + 1) * XY,
-                     D.node.p, D.child_num.p, D.loc.p, D.csum.p, D.par_off.p, D.par.p, D.slot.p, D.enode.p,
-                     D.nl_off.p, D.nlevels.p, D.lvl_node_off.p, D.lvl_edge_off.p, D.dnode.p, D.dedge.p,
-                     D.cur_n.p, D.cur_e.p, D.err.p};
+                     D.rorder.p, D.node_off.p, D.ebase.p, D.sbase.p, D.lbase.p, c->g.X, c->g.Y, (L + 1) * XY,
+                     D.nrec.p, D.edge.p, D.npos.p, D.lvl.p, D.lcur.p, D.lpos.p, D.lslot.p, D.err.p};
     launch_dag_layout(c, la, n);
     int err = 0;
     HIP_OK(hipMemcpyAsync(&err, D.err.p, sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
     if (err) throw std::invalid_argument("malformed DAG (node range, slot counts, source, parent order or slots)");
     const double t_up = now_s();
-    D.costs.alloc(mx_nodes * ML);
-    D.lo.alloc(mx_nodes);
-    D.emit.alloc(mx_nodes * 9);
-    D.packed.alloc(std::max<int64_t>(1, mx_slots) * ML);
-    D.best.alloc(std::max<int64_t>(1, mx_slots) * ML);
-    D.cost_edges.alloc(std::max<int64_t>(1, mx_edges) * LL);
-    D.best_change.alloc(std::max<int64_t>(1, mx_edges) * LL);
+    if (any_big) {
+        D.packed.alloc(std::max<int64_t>(1, mx_slots) * ML);
+        D.big_range.alloc(mx_nodes * 16);
+        D.big_dec.alloc(mx_nodes);
+    }
+    const int64_t ND = (L + 1) / 2;   // layers of one direction, at most
+    D.cost_edges.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
+    D.change.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
     NetsDev& N = c->nets;
     N.dag_routes.push_back(new DevBuf<int>());
     N.dag_routes.back()->alloc(route_slot[n]);

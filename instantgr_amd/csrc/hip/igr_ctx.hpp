@@ -115,6 +115,21 @@ struct Sched {
     DevBuf<int> bits;             // per-net state bits (assigned, blocked in this batch)
 };
 
+// Batched form: the records of a DAG's nodes and parent edges, by depth level
+// within the net (16 bytes each, one load).  Positions pack x above y.
+constexpr int DAG_POS_BITS = 13;
+struct alignas(16) DagNode {
+    uint32_t pos;                 // position, the node's layer (L: none) above it
+    uint32_t loc;                 // index in the net's node order
+    uint32_t slots;               // first child slot in the net, slot count in the top four bits
+    uint32_t ebeg;                // first parent edge in the net (the next record's is the end)
+};
+struct alignas(16) DagEdge {
+    uint32_t from, to;            // positions of the child and of the parent
+    uint32_t slot;                // the parent's child slot in the net
+    uint32_t child;               // record of the child in the net
+};
+
 // One rip-up-and-reroute pass on the device: DAGs of the rerouted nets in
 // routing order (batch by batch), with global node/edge/slot numbering.
 struct DagDev {
@@ -126,13 +141,21 @@ struct DagDev {
     DevBuf<int> lo, best_change, emit;
     DevBuf<int> pt;
     DevBuf<int64_t> pt_off;
-    // Batched form: depth levels of every net (nodes and their parent edges).
-    DevBuf<int64_t> nl_off, lvl_node_off, lvl_edge_off, dedge;
-    DevBuf<int> nlevels, dnode;
+    // Batched form: the level-ordered records, the positions in node order,
+    // the level boundaries of every net, the layer-change samples beside
+    // cost_edges, and the tables of nets too large for LDS (keys in packed).
+    DevBuf<DagNode> nrec;
+    DevBuf<DagEdge> edge;
+    DevBuf<uint32_t> npos;
+    DevBuf<int> lvl;
+    DevBuf<uint16_t> change;
+    DevBuf<uint8_t> big_range;
+    DevBuf<uint2> big_dec;
     // Batched form: the DAGs as uploaded (net list order, local parents), the
-    // per-routed-net bases and the level cursors of the device layout.
-    DevBuf<int64_t> r_node_off, r_par_off, ebase, sbase, lbase, cur_n, cur_e;
-    DevBuf<int> r_nodes, r_par, r_slot, r_child_num, r_depth, rorder, err;
+    // per-routed-net bases, and the layout kernel's level cursors, record
+    // positions and slot bases.
+    DevBuf<int64_t> r_node_off, r_par_off, ebase, sbase, lbase;
+    DevBuf<int> r_nodes, r_par, r_slot, r_child_num, r_depth, rorder, err, lcur, lpos, lslot;
     // Batched form: the routed nets of each batch in launch order, and the
     // per-batch work-queue counters.
     DevBuf<int> glist, queue;
@@ -152,23 +175,15 @@ struct DagLayoutArgs {
     const int64_t* ebase;
     const int64_t* sbase;
     const int64_t* lbase;
+    int X, Y;
     int node_limit;               // (L + 1) * X * Y
-    int* node;
-    int* o_child_num;
-    int* loc;
-    int64_t* csum;
-    int64_t* o_par_off;
-    int* o_par;
-    int* o_slot;
-    int* enode;
-    int64_t* nl_off;
-    int* nlevels;
-    int64_t* lvl_node_off;
-    int64_t* lvl_edge_off;
-    int* dnode;
-    int64_t* dedge;
-    int64_t* cur_n;
-    int64_t* cur_e;
+    DagNode* nrec;
+    DagEdge* edge;
+    uint32_t* npos;
+    int* lvl;
+    int* lcur;                    // per level: its fill cursor
+    int* lpos;                    // per node: its record
+    int* lslot;                   // per node: its first child slot in the net
     int* err;
 };
 
@@ -281,7 +296,7 @@ void progress(const char* fmt, ...);
 constexpr int DEF_GRAPH = 1;
 constexpr int DEF_SCHED_CHUNK = 16;
 constexpr int DEF_DAG_ORDER = 1;
-constexpr int DEF_DAG_WAVES = 2;
+constexpr int DEF_DAG_WAVES = 4;
 constexpr int DEF_DAG_SEQ = 16;
 constexpr int DEF_DAG_GRID = 2048;
 // Batched scheduler: release-driven rounds from this many scheduled nets,
@@ -358,6 +373,7 @@ struct DagBatch {
     int levels;
     int index = 0;              // batch number in the pass (work-queue counter)
     int64_t lvl0;               // first entry of this batch in lvl_off
+    int lds = 0;                // batched form: dynamic LDS of the net kernel
     double bytes_edges = 0, bytes_dp = 0;   // algorithmic HBM bytes
 };
 void launch_dag_batch_plain(igr_ctx* c, const DagBatch& b, int stamp, const std::vector<int64_t>& h_lvl_off);
@@ -366,6 +382,10 @@ void launch_dag_compact(igr_ctx* c, const DagBatch& b);
 // queue, all depth levels of a net in one workgroup; the pass's per-batch
 // queue counters are zeroed first.
 void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, int stamp);
+// LDS bytes of a net's tables in that form, and the most a launch takes (a
+// larger net's tables live in global memory).
+int64_t dag_net_lds(int64_t nodes, int64_t slots, int64_t levels, int L);
+constexpr int64_t DAG_LDS_MAX = 60 * 1024;
 void launch_dag_queue_reset(igr_ctx* c, int64_t batches);
 // Batched form: the device layout of a pass's DAGs.
 void launch_dag_layout(igr_ctx* c, const DagLayoutArgs& a, int64_t n);
