@@ -67,6 +67,11 @@ struct EdgeArgs {
     double* cost;             // n blocks of ND * ND
     uint16_t* change;         // the sample of each entry's layer change
     int chunk;                // edges per wave
+    unsigned edge_blocks;     // workgroups from here on rip up
+    const int* rip_nets;      // the next batch's nets
+    int64_t rip_n;
+    int* const* rptr;
+    int* bad;
 };
 
 template <int L>
@@ -76,6 +81,14 @@ __global__ void __launch_bounds__(TPB) k_dag_edge_costs(EdgeArgs a) {
     __shared__ double s_ps[EW_WAVES][EW_SAMPLES * ND];     // prefix sum at (sample, direction layer)
     __shared__ double s_pe[EW_WAVES][2 * ND];              // prefix sum at the child / parent end
     const GridDev& g = a.g;
+    if (blockIdx.x >= a.edge_blocks) {
+        // The rip-up scatter of the next batch: it reads other nets' old
+        // routes and writes only the rip-up difference arrays, so it shares
+        // the launch with the edges of this batch.
+        const int64_t t = ((int64_t)(blockIdx.x - a.edge_blocks) * TPB + threadIdx.x) / RIP_LANES;
+        if (t < a.rip_n) rip_route(g, a.rptr[a.rip_nets[t]], a.bad);
+        return;
+    }
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int64_t w0 = ((int64_t)blockIdx.x * EW_WAVES + wv) * a.chunk;
     if (w0 >= a.n) return;                                 // whole waves; no workgroup barrier below
@@ -649,20 +662,24 @@ __global__ void k_queue_zero(int* p, int64_t n) {
 } // namespace
 
 template <int L>
-static void dag_batch(igr_ctx* c, const DagBatch& b, int stamp) {
+static void dag_batch(igr_ctx* c, const DagBatch& b, const DagBatch* rip, int stamp) {
     DagDev& D = c->dag;
     const int64_t n = b.net1 - b.net0, ne = b.edge1 - b.edge0;
     hipStream_t st = c->stream;
-    if (ne > 0) {
+    const int64_t nr = rip ? rip->net1 - rip->net0 : 0;
+    if (ne > 0 || nr > 0) {
         KScope ks(c, K_DAG_EDGES, b.bytes_edges);
         // edges per wave: enough waves to fill the GPU first, then up to a
         // record per lane
-        const int64_t per = ne / (EDGE_WAVES);
+        const int64_t per = ne / EDGE_WAVES;
         const int chunk = per >= 64 ? 64 : per >= 32 ? 32 : per >= 16 ? 16 : per >= 8 ? 8 : 4;
-        EdgeArgs a{c->g, D.edge.p + b.edge0, ne, D.cost_edges.p, D.change.p, chunk};
-        k_dag_edge_costs<L><<<(unsigned)((ne + (int64_t)chunk * EW_WAVES - 1) / (chunk * EW_WAVES)), TPB, 0, st>>>(a);
+        const unsigned eb = (unsigned)((ne + (int64_t)chunk * EW_WAVES - 1) / (chunk * EW_WAVES));
+        EdgeArgs a{c->g, D.edge.p + b.edge0, ne, D.cost_edges.p, D.change.p, chunk, eb,
+                   rip ? D.nets.p + rip->net0 : nullptr, nr, c->nets.rptr.p, c->bad.p};
+        k_dag_edge_costs<L><<<eb + blocks(nr * RIP_LANES), TPB, 0, st>>>(a);
         HIP_OK(hipGetLastError());
     }
+    if (n == 0) return;
     KScope ks(c, K_DAG_DP, b.bytes_dp);
     const unsigned grid = (unsigned)std::min<int64_t>(n, c->tune.dag_grid ? c->tune.dag_grid : DEF_DAG_GRID);
     NetArgs a{c->g, D.nrec.p, D.edge.p, D.npos.p, D.lvl.p, D.node_off.p, D.ebase.p, D.sbase.p, D.lbase.p,
@@ -676,10 +693,9 @@ static void dag_batch(igr_ctx* c, const DagBatch& b, int stamp) {
 
 int64_t dag_net_lds(int64_t nodes, int64_t slots, int64_t levels, int L) { return net_lds(nodes, slots, levels, L + 1); }
 
-void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, int stamp) {
-    if (b.net1 == b.net0) return;
+void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, const DagBatch* rip, int stamp) {
     switch (c->g.L) {
-#define CASE(LV) case LV: dag_batch<LV>(c, b, stamp); break;
+#define CASE(LV) case LV: dag_batch<LV>(c, b, rip, stamp); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12)
 #undef CASE
     default: throw std::runtime_error("unsupported routing layer count");

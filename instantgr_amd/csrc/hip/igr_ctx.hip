@@ -75,9 +75,6 @@ int igr_create(const igr_grid_desc* d, igr_ctx** out) {
         noalloc_init(c->device);
         HIP_OK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         HIP_OK(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
-        HIP_OK(hipStreamCreateWithFlags(&c->aux_stream, hipStreamNonBlocking));
-        HIP_OK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-        HIP_OK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
         GridDev& g = c->g;
         g.L = d->L; g.X = d->X; g.Y = d->Y; g.DIR = d->DIR & 1;
         g.XYc = (int64_t)d->X * d->Y;
@@ -119,15 +116,10 @@ void igr_destroy(igr_ctx* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
-    if (c->aux_stream) (void)hipStreamSynchronize(c->aux_stream);
-    hipStream_t s = c->stream, cs = c->copy_stream, as = c->aux_stream;
-    hipEvent_t ef = c->ev_fork, ej = c->ev_join;
+    hipStream_t s = c->stream, cs = c->copy_stream;
     delete c;
     if (s) (void)hipStreamDestroy(s);
     if (cs) (void)hipStreamDestroy(cs);
-    if (as) (void)hipStreamDestroy(as);
-    if (ef) (void)hipEventDestroy(ef);
-    if (ej) (void)hipEventDestroy(ej);
 }
 
 static void to_host_ref(igr_ctx* c, const void* dev, void* host, int eb) {
@@ -799,31 +791,20 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
         // (events on the stream) is on.
         StreamGraph sg(s, !c->prof.on && (c->tune.graph ? c->tune.graph : DEF_GRAPH) == 1);
         // The rip-up scatter of batch b+1 (the old routes of other nets, into
-        // the rip-up difference arrays) runs on the side stream beside batch
-        // b's DAG kernels (the new routes, into the commit arrays) and joins
-        // before the fused update that consumes both.  Kernel timing keeps
-        // one stream.
-        const bool side = !c->prof.on;
+        // the rip-up difference arrays) shares the launch of batch b's edge
+        // costs.  Kernel timing gives it a launch of its own.
+        const bool shared = !c->prof.on;
         int s1 = ++c->stamp;
         launch_rip_scatter(c, D.nets.p + batches[0].net0, batches[0].net1 - batches[0].net0);
         launch_track_fused(c, 0, s1, true);
         for (size_t b = 0; b < batches.size(); b++) {
             if (b % 512 == 511) progress("DAG pass: %zu of %zu batches enqueued", b + 1, batches.size());
-            const bool more = b + 1 < batches.size();
-            if (side && more) {
-                const DagBatch& Bn = batches[b + 1];
-                HIP_OK(hipEventRecord(c->ev_fork, s));
-                HIP_OK(hipStreamWaitEvent(c->aux_stream, c->ev_fork, 0));
-                launch_rip_scatter(c, D.nets.p + Bn.net0, Bn.net1 - Bn.net0, c->aux_stream);
-                HIP_OK(hipEventRecord(c->ev_join, c->aux_stream));
-            }
+            const DagBatch* next = b + 1 < batches.size() ? &batches[b + 1] : nullptr;
             const int s2 = ++c->stamp;
-            launch_dag_batch_wave(c, batches[b], s2);
-            if (more) {
-                const DagBatch& Bn = batches[b + 1];
+            launch_dag_batch_wave(c, batches[b], shared ? next : nullptr, s2);
+            if (next) {
                 s1 = ++c->stamp;
-                if (side) HIP_OK(hipStreamWaitEvent(s, c->ev_join, 0));
-                else launch_rip_scatter(c, D.nets.p + Bn.net0, Bn.net1 - Bn.net0);
+                if (!shared) launch_rip_scatter(c, D.nets.p + next->net0, next->net1 - next->net0);
                 launch_track_fused(c, s2, s1, true);
             } else {
                 launch_track_fused(c, s2, 0, false);

@@ -237,8 +237,6 @@ struct igr_ctx {
     igr_dev::GridDev g{};
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;   // uploads that overlap the compute stream
-    hipStream_t aux_stream = nullptr;    // a DAG pass's rip-up scatters beside the DAG kernels
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int device = 0;
     igr_dev::DevBuf<double> w;
     igr_dev::DevBuf<int> xlen, ylen;
@@ -380,8 +378,9 @@ void launch_dag_batch_plain(igr_ctx* c, const DagBatch& b, int stamp, const std:
 void launch_dag_compact(igr_ctx* c, const DagBatch& b);
 // Batched form: persistent workgroups pulling the batch's nets from a work
 // queue, all depth levels of a net in one workgroup; the pass's per-batch
-// queue counters are zeroed first.
-void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, int stamp);
+// queue counters are zeroed first.  The batch to rip up next (or null) is
+// scattered by the same launches.
+void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, const DagBatch* rip, int stamp);
 // LDS bytes of a net's tables in that form, and the most a launch takes (a
 // larger net's tables live in global memory).
 int64_t dag_net_lds(int64_t nodes, int64_t slots, int64_t levels, int L);
@@ -416,5 +415,5 @@ void gather_routes(igr_ctx* c, const int64_t* d_off, int* d_out);
 // The GPU evaluator (eval_kernels.hip).
 void evaluate_routes_dev(igr_ctx* c, const igr_eval_nets* e, const int64_t* h_route_off, const int* h_routes,
                          igr_score* out);
-void launch_rip_scatter(igr_ctx* c, const int* d_nets, int64_t n, hipStream_t s = nullptr);
+void launch_rip_scatter(igr_ctx* c, const int* d_nets, int64_t n);
 } // namespace igr_dev

@@ -18,6 +18,7 @@
 // Demand changes by integers and halves, so the result equals the sequential
 // one.  A track no scatter touched keeps its demand and so its costs: the
 // routing kernels and the rip-up scatter flag every track they write into.
+#include "dag_dev.h"
 #include "igr_ctx.hpp"
 #include "scan.h"
 
@@ -370,42 +371,11 @@ __global__ void __launch_bounds__(1024) k_track_cost(GridDev g, unsigned long lo
     }
 }
 
-// Rip-up footprint of routed nets: +1/-1 wire differences at the two ends of
-// each wire, +1/-1 covered-cell differences at its first cell and one past
-// its last, one count per via cut, and the dirty flag of every track touched.
-// Wires that do not run along their layer's direction set *bad.
+// The rip-up footprint of a list of routed nets (rip_route).
 __global__ void __launch_bounds__(SB) k_rip_scatter(GridDev g, const int* nets, int64_t n, int* const* rptr,
                                                     int* bad) {
-    const int64_t t = (int64_t)blockIdx.x * SB + threadIdx.x;
-    if (t >= n) return;
-    const int* r = rptr[nets[t]];
-    const int XY = g.X * g.Y;
-    for (int i = 1; i < r[0]; i += 2) {
-        const int a = r[i], b = r[i + 1];
-        const int la = a / XY, lb = b / XY;
-        const int x0 = a / g.Y % g.X, y0 = a % g.Y, x1 = b / g.Y % g.X, y1 = b % g.Y;
-        if (la == lb) {
-            const int d = layer_dir(la, g.DIR);
-            if ((d == 0 && y0 != y1) || (d == 1 && x0 != x1)) { atomicOr(bad, 1); continue; }
-            const int lo = d ? min(y0, y1) : min(x0, x1), hi = d ? max(y0, y1) : max(x0, x1);
-            const int len = d ? g.Y : g.X;
-            const int64_t c0 = d ? gidx(g, la, x0, lo) : gidx(g, la, lo, y0);
-            const int64_t c1 = d ? gidx(g, la, x0, hi) : gidx(g, la, hi, y0);
-            if (lo < hi) {
-                atomicAdd(&g.rpre[c0], 1);
-                atomicAdd(&g.rpre[c1], -1);
-            }
-            atomicAdd(&g.rcov[c0], 1);
-            if (hi + 1 < len) atomicAdd(&g.rcov[c1 + 1], -1);
-            g.dirty[track_id(g, la, x0, y0)] = 1;
-        } else {
-            const int lo = min(la, lb), hi = max(la, lb);
-            for (int l = lo; l < hi; l++) {
-                atomicAdd(&g.rvc[gidx(g, l, x0, y0)], 1);
-                g.dirty[track_id(g, l, x0, y0)] = 1;
-            }
-        }
-    }
+    const int64_t t = ((int64_t)blockIdx.x * SB + threadIdx.x) / RIP_LANES;
+    if (t < n) rip_route(g, rptr[nets[t]], bad);
 }
 
 __global__ void k_fill_i(int* p, int64_t n, int v) {
@@ -536,14 +506,10 @@ void launch_track_fused(igr_ctx* c, int s_commit, int s_rip, bool cost) {
     HIP_OK(hipGetLastError());
 }
 
-void launch_rip_scatter(igr_ctx* c, const int* d_nets, int64_t n, hipStream_t s) {
+void launch_rip_scatter(igr_ctx* c, const int* d_nets, int64_t n) {
     if (n == 0) return;
-    if (s == nullptr || s == c->stream) {
-        KScope ks(c, K_RIP);
-        k_rip_scatter<<<blocks(n), SB, 0, c->stream>>>(c->g, d_nets, n, c->nets.rptr.p, c->bad.p);
-    } else {
-        k_rip_scatter<<<blocks(n), SB, 0, s>>>(c->g, d_nets, n, c->nets.rptr.p, c->bad.p);
-    }
+    KScope ks(c, K_RIP);
+    k_rip_scatter<<<blocks(n * RIP_LANES), SB, 0, c->stream>>>(c->g, d_nets, n, c->nets.rptr.p, c->bad.p);
     HIP_OK(hipGetLastError());
 }
 
