@@ -248,7 +248,8 @@ int igr_device_memory(igr_ctx* ctx, size_t* free_bytes, size_t* total_bytes);
  * the autotuner (instantgr_amd/autotune.py) measures and sets them.  Results
  * do not depend on any of them. */
 typedef struct igr_tuning {
-    int graph;          /* 1: each pass's batch sequence captured and launched as one hipGraph; 2: stream launches */
+    int graph;          /* 1: each pass's batch sequence captured and launched as one hipGraph; 2: stream launches
+                           (built-in) */
     int sched_group;    /* lanes per net in the scheduler's claim and viability kernels: 4, 8 or 16 */
     int sched_chunk;    /* scheduler rounds enqueued between host checks, 1..256 */
     int dag_order;      /* workgroup order of a DAG batch: 1 deepest DAG first, 2 routing order */
