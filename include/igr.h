@@ -262,8 +262,7 @@ typedef struct igr_tuning {
                            choice 2 from 1.5M scheduled nets */
     int presum_k;       /* plain form's prefix-sum kernel: cells per thread, 4, 8 or 16 */
     int dag_grid;       /* DAG kernel: persistent workgroups pulling a batch's nets from its work queue */
-    int lshape_groups;  /* pattern DP: nets (16-lane groups) per workgroup, 1, 2 or 4; the workgroup's LDS
-                           slab holds their layer-range tables (0: 4, fewer where the tables need more room) */
+    int lshape_groups;  /* 1, 2 or 4; the pattern DP always takes four nets a wave, the field has no effect */
 } igr_tuning;
 int igr_set_tuning(igr_ctx* ctx, const igr_tuning* t);
 /* The values in force (built-in choices resolved, per-pass choices as 0). */

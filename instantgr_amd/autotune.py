@@ -12,13 +12,10 @@ results (include/igr.h, igr_tuning):
   sched_kind   scheduler rounds: active-list (work follows the active nets) or release-driven
                (work follows the released cells)
   dag_grid     persistent workgroups of the DAG kernel pulling nets from the batch's work queue
-  lshape_groups  nets (16-lane groups) per workgroup of the pattern DP, which sets the LDS slab a
-               workgroup holds (their layer-range tables)
 
-In the terms of a tile shape: nets per workgroup (lshape_groups, dag_grid),
-waves per net (dag_waves) and the LDS slab size (lshape_groups times the node
-tables of the node-count class).  dag_edges and dag_seq have no effect and
-keep one value.
+In the terms of a tile shape: nets per workgroup (dag_grid) and waves per net
+(dag_waves).  dag_edges, dag_seq and lshape_groups have no effect and keep one
+value.
 
 `tune` measures them on a design (normally a reduced sample of the production
 design from the same generator) by coordinate descent: each field in turn takes
@@ -46,7 +43,7 @@ CANDIDATES = {
     "dag_seq": [16],
     "sched_kind": [1, 2],
     "dag_grid": [1024, 2048, 4096],
-    "lshape_groups": [1, 2, 4],
+    "lshape_groups": [4],
 }
 
 # Fields of the plain form only (the tuner measures the batched form).

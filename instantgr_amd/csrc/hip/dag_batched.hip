@@ -6,9 +6,9 @@
 // kernels (dag_kernels.hip), so both forms' routes are identical.
 #include "dag_dev.h"
 #include "igr_ctx.hpp"
+#include "row.h"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace igr_dev {
 
@@ -229,33 +229,6 @@ struct NetArgs {
     int64_t node0, slot0;
 };
 
-// Value of lane N of the caller's 16-lane row.
-template <int N>
-__device__ __forceinline__ int row_bcast(int v) {
-    return __builtin_amdgcn_mov_dpp(v, 0x150 + N, 0xf, 0xf, false);
-}
-template <int N>
-__device__ __forceinline__ float row_bcastf(float v) {
-    return __int_as_float(row_bcast<N>(__float_as_int(v)));
-}
-// Value of the lane D above in the caller's row, +inf past its end.
-template <int D>
-__device__ __forceinline__ double row_above(double v) {
-    const int64_t b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x100 + D, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0x7ff00000, (int)(b >> 32), 0x100 + D, 0xf, 0xf, false);
-    return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
-}
-
-// f(integral_constant 0 .. N - 1), fully unrolled.
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void unrolled(F f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        unrolled<N, I + 1>(f);
-    }
-}
-
 // Key table access: LDS, or global memory for the nets whose tables exceed it
 // (their keys are updated by atomics that complete in L2, so they are read
 // with device-scope loads).
@@ -293,7 +266,7 @@ __device__ __forceinline__ double node_cost(const uint64_t* keys, int nc, int nc
     double vm[L];                                      // via cut t - 2, zero above s
     unrolled<L - 1>([&](auto I) {
         constexpr int t = I + 2;
-        const float v = row_bcastf<I>(vl);
+        const float v = row_bcast<I>(vl);
         vm[I] = t <= s ? (double)v : 0.0;
     });
     unrolled<L>([&](auto I) {
@@ -312,7 +285,7 @@ __device__ __forceinline__ double node_cost(const uint64_t* keys, int nc, int nc
         float m = c;
         unrolled<L>([&](auto I) {
             constexpr int low = L - I;
-            const float below = row_bcastf<low>(c);        // outside the selects: every lane takes part
+            const float below = row_bcast<low>(c);        // outside the selects: every lane takes part
             m = __builtin_amdgcn_fmed3f(m, below, -__builtin_inff());   // their minimum
             m = low >= s ? c : m;
             cost[low - 1] += (double)m;

@@ -403,35 +403,35 @@ int igr_pattern_route(igr_ctx* c, const int* order, int64_t n, int form, igr_pas
                 plain_batch(c, c->scratch.net_list.p + cnt[b], c->scratch.scr_off.p + cnt[b], cnt[b + 1] - cnt[b],
                             lbytes[b]);
         } else {
-            // Each batch's nets grouped by node-count class, one launch per
-            // class: the order of nets inside a batch changes no result (their
-            // footprints are disjoint and their demand updates integer adds).
-            // Nets above the largest class (none under the 12-pin subnet cap)
-            // take the thread-per-net kernel.
-            constexpr int NCLS = 5;
+            // Each batch's nets by decreasing node count, so that the nets of a
+            // wave are alike and the longest start first: the order of nets
+            // inside a batch changes no result (their footprints are disjoint
+            // and their demand updates integer adds).  Nets above
+            // LSWAVE_MAX_NODES (none under the 12-pin subnet cap) come first
+            // and take the thread-per-net kernel.
+            constexpr int NK = LSWAVE_MAX_NODES + 1;   // keys: larger nets, then LSWAVE_MAX_NODES .. 1 nodes
             std::vector<int> wl(n);
-            std::vector<int64_t> co((size_t)nb * NCLS + 1, 0);
-            std::vector<double> cbytes((size_t)nb * NCLS, 0.0);
+            std::vector<int64_t> co((size_t)nb * NK + 1, 0);
+            std::vector<double> bbytes((size_t)nb * 2, 0.0);
             {
-                std::vector<int> cls(n);
-                for (int64_t i = 0; i < n; i++) {
-                    const int k = lshape_wave_class(
-                        (int)(c->nets.h_node_off[list[i] + 1] - c->nets.h_node_off[list[i]]));
-                    cls[i] = k < 0 ? NCLS - 1 : k;
-                }
+                auto key = [&](int64_t i, int b) {
+                    const int64_t k = c->nets.h_node_off[list[i] + 1] - c->nets.h_node_off[list[i]];
+                    return (size_t)b * NK + (k > LSWAVE_MAX_NODES ? 0 : (size_t)(NK - k));
+                };
                 for (int b = 0; b < nb; b++)
                     for (int64_t i = cnt[b]; i < cnt[b + 1]; i++) {
-                        co[(size_t)b * NCLS + cls[i] + 1]++;
-                        cbytes[(size_t)b * NCLS + cls[i]] += c->nets.h_lbytes[list[i]];
+                        const size_t k = key(i, b);
+                        co[k + 1]++;
+                        bbytes[(size_t)b * 2 + (k % NK != 0)] += c->nets.h_lbytes[list[i]];
                     }
                 for (size_t k = 0; k + 1 < co.size(); k++) co[k + 1] += co[k];
                 std::vector<int64_t> pos(co.begin(), co.end() - 1);
                 for (int b = 0; b < nb; b++)
-                    for (int64_t i = cnt[b]; i < cnt[b + 1]; i++) wl[pos[(size_t)b * NCLS + cls[i]]++] = list[i];
+                    for (int64_t i = cnt[b]; i < cnt[b + 1]; i++) wl[pos[key(i, b)]++] = list[i];
             }
             int64_t max_nodes = 0;
             for (int b = 0; b < nb; b++) {
-                const int64_t a = co[(size_t)b * NCLS + NCLS - 1], e = co[(size_t)b * NCLS + NCLS];
+                const int64_t a = cnt[b], e = co[(size_t)b * NK + 1];
                 max_nodes = std::max(max_nodes, scratch_offsets(c, wl.data() + a, e - a, off.data() + a));
             }
             if (max_nodes) ensure_scratch(c, max_nodes);
@@ -445,15 +445,13 @@ int igr_pattern_route(igr_ctx* c, const int* order, int64_t n, int form, igr_pas
             launch_track_fused(c, 0, 0, true);
             for (int b = 0; b < nb; b++) {
                 const int stamp = ++c->stamp;
-                for (int k = 0; k < NCLS; k++) {
-                    const int64_t a = co[(size_t)b * NCLS + k], e = co[(size_t)b * NCLS + k + 1];
-                    if (a == e) continue;
-                    if (k < NCLS - 1)
-                        launch_lshape_wave(c, c->scratch.net_list.p + a, e - a, k, stamp, cbytes[(size_t)b * NCLS + k]);
-                    else
-                        launch_lshape_plain(c, c->scratch.net_list.p + a, c->scratch.scr_off.p + a, e - a, stamp,
-                                            cbytes[(size_t)b * NCLS + k]);
-                }
+                const int64_t a = cnt[b], m = co[(size_t)b * NK + 1], e = cnt[b + 1];
+                launch_lshape_plain(c, c->scratch.net_list.p + a, c->scratch.scr_off.p + a, m - a, stamp,
+                                    bbytes[(size_t)b * 2]);
+                if (e > m)
+                    launch_lshape_wave(c, c->scratch.net_list.p + m, e - m,
+                                       (int)(c->nets.h_node_off[wl[m] + 1] - c->nets.h_node_off[wl[m]]), stamp,
+                                       bbytes[(size_t)b * 2 + 1]);
                 launch_track_fused(c, stamp, 0, b + 1 < nb);
             }
             HIP_OK(hipStreamSynchronize(c->stream));

@@ -340,12 +340,10 @@ void launch_wire_commit(igr_ctx* c, int stamp);
 void launch_via_commit(igr_ctx* c, const int* d_nets, int64_t n, int stamp, int K);
 void launch_lshape_plain(igr_ctx* c, const int* d_nets, const int64_t* d_scr_off, int64_t n, int stamp,
                          double bytes = 0);
-// Batched form: the L-shape DP with a 16-lane group per net and the DP tables
-// in LDS.  Nets of one launch have node counts in one class (lshape_wave_class:
-// up to 4, 8, 16 or LSWAVE_MAX_NODES nodes; -1 above).
+// Batched form: the L-shape DP with a row of 16 lanes per net.  Nets of one
+// launch have at most 'nodes' nodes (up to LSWAVE_MAX_NODES).
 constexpr int LSWAVE_MAX_NODES = 24;
-int lshape_wave_class(int nodes);
-void launch_lshape_wave(igr_ctx* c, const int* d_nets, int64_t n, int cls, int stamp, double bytes = 0);
+void launch_lshape_wave(igr_ctx* c, const int* d_nets, int64_t n, int nodes, int stamp, double bytes = 0);
 void launch_to_ref(igr_ctx* c, const void* src, void* dst, int elem_bytes);
 void launch_from_ref(igr_ctx* c, const void* src, void* dst, int elem_bytes);
 void launch_ripup_mark(igr_ctx* c, int th, uint8_t* d_is_of, int* d_of);

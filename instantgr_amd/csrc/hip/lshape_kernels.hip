@@ -9,6 +9,7 @@
 // sums, children added in decreasing node order), strict '<' keeping the
 // first minimum and '<=' in the layer-range prefix minimum.
 #include "igr_ctx.hpp"
+#include "row.h"
 
 namespace igr_dev {
 
@@ -167,35 +168,57 @@ __global__ void __launch_bounds__(TPB) k_lshape_plain(GridDev g, const int* nets
 
 
 // ---------------------------------------------------------------------------
-// Batched form: a 16-lane group per net, four nets per wave.  The per-node DP
-// tables (cost over layer ranges, back-pointers) live in LDS in triangular
-// form (minl <= maxl); lane l owns layer l: it computes the child's best cost
-// through layer l, the edge costs on layer l, and the prefix minimum of the
-// layer-range row minl = l.  The root's range is the group's min/argmin
-// (first minimum in (minl, maxl) order).  Every value is computed with the
-// same FP64 operations in the same order as the thread-per-net kernel above,
-// so routes and costs are bit-identical.  NC bounds the nodes per net of a
-// launch (the host groups a batch's nets by node count); G groups per block.
+// Batched form: a row of 16 lanes per net, four nets per wave, lane s for
+// layer s - 1.  A node's cost over its layer ranges is never stored: with its
+// children's edge costs per layer in LDS (L doubles a node), lane hi forms the
+// cost of every range [low, hi] (via stack, then the children in decreasing
+// node order, each the running minimum of its edge costs over the range), and
+// the row keeps per layer the smallest range that holds it and its two ends,
+// ties to the smaller low, then the smaller hi.  The same FP64 operations in
+// the same order as the thread-per-net kernel above, so routes and costs are
+// bit-identical.  Which child layers a range used is found again on the way
+// down, for the ranges chosen.
+//
+// Nets are short chains of nodes, so a net's time is the latency of a node:
+// the prefix sums and via costs of the next node and its parent edge are
+// loaded while the current one is worked on.  One launch takes a batch: nets
+// of one wave have similar node counts (the host sorts them), and under 3 KB
+// of LDS a net leaves the waves to the registers.  With the layer-range tables
+// in LDS (450 bytes a node), the grid read inside the chain and a launch per
+// node-count class, a batch took 295 us on 200x200 (20k nets, 40 batches), 252
+// us on 800x800 (500k nets, 58 batches) and 315 us on 1237x989 with 11 layers;
+// this kernel takes 56, 68 and 79 us.
 // ---------------------------------------------------------------------------
-__host__ __device__ constexpr int tri_row(int L, int minl) { return minl * L - minl * (minl - 1) / 2; }
+// What a node's step reads from the grid, by lane.
+struct NodeIn {
+    float vl;                     // via cut of layer lane (lanes 0 .. L - 2) at the node
+    double wc, wp;                // the edge's wire on the lane's layer at the node's side, at the parent's
+    float va, vb;                 // via cut of the lane's layer at the L corners (x, py) and (px, y)
+};
 
-template <int L, int NC, int G>
-__global__ void __launch_bounds__(16 * G) k_lshape_wave(GridDev g, const int* __restrict__ nets, int64_t n,
-                                                         const int64_t* __restrict__ node_off,
-                                                         const int* __restrict__ node,
-                                                         const int* __restrict__ parent,
-                                                         const int64_t* __restrict__ route_off, int* routes,
-                                                         int stamp) {
-    constexpr int LL = L * L, T = L * (L + 1) / 2, LV = L > 1 ? L - 1 : 1;
-    __shared__ double sD[G][NC * T];
-    __shared__ uint16_t sF[G][NC * T];
-    __shared__ int sx[G][NC], sy[G][NC], sl[G][NC], sp[G][NC], slr[G][NC], scode[G][NC];
-    __shared__ float sV[G][NC * LV];
-    __shared__ double smcc[G][L], swc[G][L], sva[G][L], svb[G][L], sdg[G][L];
-    __shared__ int scf[G][L], spv[G][L];
-    __shared__ int snn[G];
-    const int gi = threadIdx.x >> 4, lane = threadIdx.x & 15;
-    const int64_t t = (int64_t)blockIdx.x * G + gi;
+__host__ __device__ constexpr int lswave_net_lds(int L, int cap) { return (cap * (8 * L + 12 + 34) + 15) / 16 * 16; }
+
+template <int L>
+__global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __restrict__ nets, int64_t n, int cap,
+                                                    const int64_t* __restrict__ node_off,
+                                                    const int* __restrict__ node, const int* __restrict__ parent,
+                                                    const int64_t* __restrict__ route_off, int* routes, int stamp) {
+    constexpr int LL = L * L;
+    extern __shared__ __align__(16) double s_dyn[];
+    // per net, cap nodes of: edge cost by parent layer; position, parent, the
+    // choice made on the way down; by layer, the edge's child layer and the
+    // best range's ends; last child and next lower sibling (0: none)
+    const int gi = threadIdx.x >> 4, lane = threadIdx.x & 15, s = lane;
+    unsigned char* base = reinterpret_cast<unsigned char*>(s_dyn) + gi * lswave_net_lds(L, cap);
+    double* mcp = reinterpret_cast<double*>(base);
+    int* pos = reinterpret_cast<int*>(mcp + cap * L);
+    int* par = pos + cap;
+    int* pick = par + cap;
+    uint8_t* curl_of = reinterpret_cast<uint8_t*>(pick + cap);
+    uint8_t* range_of = curl_of + 16 * cap;
+    uint8_t* child_of = range_of + 16 * cap;
+    uint8_t* sib_of = child_of + cap;
+    const int64_t t = (int64_t)blockIdx.x * 4 + gi;
     int nn = 0, net = 0;
     int64_t nb = 0;
     if (t < n) {
@@ -203,287 +226,266 @@ __global__ void __launch_bounds__(16 * G) k_lshape_wave(GridDev g, const int* __
         nb = node_off[net];
         nn = (int)(node_off[net + 1] - nb);
     }
-    if (lane == 0) snn[gi] = nn;
     const int X = g.X, Y = g.Y, XY = X * Y;
     for (int k = lane; k < nn; k += 16) {
-        const int p = node[nb + k];
-        sl[gi][k] = p / XY;
-        sx[gi][k] = p / Y % X;
-        sy[gi][k] = p % Y;
-        sp[gi][k] = parent[nb + k];
+        pos[k] = node[nb + k];
+        par[k] = parent[nb + k];
     }
+    int nmax = nn;
+    nmax = max(nmax, __shfl_xor(nmax, 16, 64));
+    nmax = max(nmax, __shfl_xor(nmax, 32, 64));
     __syncthreads();
-    int nmax = 0;
-    for (int k = 0; k < G; k++) nmax = max(nmax, snn[k]);
-    for (int k = lane; k < nn * (L - 1); k += 16) {
-        const int i = k / (L - 1), l = k - i * (L - 1);
-        sV[gi][k] = g.vcost[gidx(g, l, sx[gi][i], sy[gi][i])];
-    }
-    __syncthreads();
-    double* D = sD[gi];
-    uint16_t* F = sF[gi];
-    // Via-stack cost of every layer range at every node; ranges that miss a
-    // pin's layer are INF (src/Lshape_route.hpp:36-48).
-    if (lane < L) {
-        const int minl = lane, r0 = tri_row(L, minl);
-        for (int i = 0; i < nn; i++) {
-            double* nd = D + i * T + r0;
-            const int pl = sl[gi][i];
-            const bool pin = pl < L;
-            double acc = 0;
-            nd[0] = (pin && minl != pl) ? INF : 0.0;
-            for (int maxl = minl + 1; maxl < L; maxl++) {
-                acc = acc + (double)sV[gi][i * LV + maxl - 1];
-                nd[maxl - minl] = (pin && (minl > pl || maxl < pl)) ? INF : acc;
-            }
+    for (int k = lane; k < nn; k += 16) {
+        const int p = par[k];
+        int c = 0, b = 0;
+        for (int q = 1; q < nn; q++) {
+            const int pq = par[q];
+            if (pq == k) c = q;
+            if (q < k && pq == p) b = q;
         }
+        child_of[k] = (uint8_t)c;
+        sib_of[k] = (uint8_t)b;
     }
     __syncthreads();
-    // Edges bottom-up, children in decreasing node order.
-    for (int i = nmax - 1; i >= 1; i--) {
-        const bool act = i < nn && lane < L;
-        int x = 0, y = 0, px = 0, py = 0, p = 0;
-        if (i < nn) {
-            x = sx[gi][i];
-            y = sy[gi][i];
-            p = sp[gi][i];
-            px = sx[gi][p];
-            py = sy[gi][p];
-        }
-        const bool straight = x == px || y == py;
-        const int minx = min(x, px), maxx = max(x, px), miny = min(y, py), maxy = max(y, py);
-        const int l = lane;
-        double wc = 0, wp = 0, va = 0, vb = 0;
-        if (act) {
-            const int d = layer_dir(l, g.DIR);
-            if (straight) {
-                if ((d == 0 && y == py) || (d == 1 && x == px)) wc = wseg(g, l, minx, maxx, miny, maxy);
+    const int l = s - 1;                               // the lane's layer
+    const bool on = s >= 1 && s <= L;
+    const int dl = layer_dir(l & 15, g.DIR);
+    auto fetch = [&](int i) {
+        NodeIn in{0, 0, 0, 0, 0};
+        if (i >= nn) return in;
+        const int v = pos[i] % XY, x = v / Y, y = v - x * Y;
+        if (lane < L - 1) in.vl = g.vcost[gidx(g, lane, x, y)];
+        if (i > 0 && on) {
+            const int u = pos[par[i]] % XY, px = u / Y, py = u - px * Y;
+            const int minx = min(x, px), maxx = max(x, px), miny = min(y, py), maxy = max(y, py);
+            if (x == px || y == py) {
+                if ((dl == 0 && y == py) || (dl == 1 && x == px)) in.wc = wseg(g, l, minx, maxx, miny, maxy);
             } else {
-                wc = d == 1 ? wseg(g, l, x, x, miny, maxy) : wseg(g, l, minx, maxx, y, y);
-                wp = d == 1 ? wseg(g, l, px, px, miny, maxy) : wseg(g, l, minx, maxx, py, py);
-                va = (double)g.vcost[gidx(g, l, x, py)];
-                vb = (double)g.vcost[gidx(g, l, px, y)];
+                in.wc = dl == 1 ? wseg(g, l, x, x, miny, maxy) : wseg(g, l, minx, maxx, y, y);
+                in.wp = dl == 1 ? wseg(g, l, px, px, miny, maxy) : wseg(g, l, minx, maxx, py, py);
+                in.va = g.vcost[gidx(g, l, x, py)];
+                in.vb = g.vcost[gidx(g, l, px, y)];
             }
-            // Best child range through layer l (first minimum, strict <).
-            const double* nd = D + i * T;
-            double m = INF;
-            int cf = 0;
-            for (int minl = 0; minl <= l; minl++) {
-                const double* row = nd + tri_row(L, minl) - minl;
-                for (int maxl = l; maxl < L; maxl++)
-                    if (row[maxl] < m) {
-                        m = row[maxl];
-                        cf = minl * L + maxl;
+        }
+        return in;
+    };
+    const double PINF = __longlong_as_double(0x7ff0000000000000LL);
+    NodeIn in = fetch(nmax - 1);
+    for (int i = nmax - 1; i >= 0; i--) {
+        const NodeIn next = i > 0 ? fetch(i - 1) : NodeIn{0, 0, 0, 0, 0};
+        const bool act = i < nn;
+        const int v = act ? pos[i] : 0;
+        const int pl = v / XY;                         // the pin's layer, L for none
+        // cost[low - 1] of the range [low, s]
+        double cost[L], vm[L];
+        unrolled<L - 1>([&](auto I) {
+            const float via = row_bcast<I>(in.vl);
+            vm[I] = I + 2 <= s ? (double)via : 0.0;    // zero above the range's top
+        });
+        unrolled<L>([&](auto I) {
+            double acc = 0.0;
+#pragma unroll
+            for (int k = I; k < L - 1; k++) acc += vm[k];
+            cost[I] = acc;
+        });
+        // children, in decreasing node order
+        for (int c = act ? child_of[i] : 0; __ballot(c != 0); c = c ? sib_of[c] : 0) {
+            const double e = c && on ? mcp[c * L + l] : 0.0;
+            double m = e;
+            unrolled<L>([&](auto I) {
+                constexpr int low = L - I;
+                const double below = row_bcast<low>(e);
+                m = below < m ? below : m;
+                m = low >= s ? e : m;
+                cost[low - 1] += m;
+            });
+        }
+        // per layer, the smallest range through it
+        double best = INF;
+        int code = 0;
+        uint64_t at = 0;
+        unrolled<L>([&](auto I) {
+            constexpr int low = I + 1;
+            const bool ok = act & on & (s >= low) & ((pl >= L) | ((low - 1 <= pl) & (pl < s))) & (cost[I] < INF);
+            const double own = ok ? cost[I] : PINF;
+            double c = own;
+            auto lower = [&](double o) { c = o < c ? o : c; };
+            lower(row_above<1>(c));
+            lower(row_above<2>(c));
+            if constexpr (L > 4) lower(row_above<4>(c));
+            if constexpr (L > 8) lower(row_above<8>(c));
+            const uint64_t mine = __ballot(own == c);
+            const bool better = (s >= low) & (c < best);
+            best = better ? c : best;
+            code = better ? low : code;
+            at = better ? mine : at;
+        });
+        if (code) code |= (s + __builtin_ctzll(at >> (threadIdx.x & 63))) << 4;
+        if (act && on) range_of[i * 16 + l] = (uint8_t)code;
+        if (i == 0) {
+            // the root's range: the smallest cost, ties to the smaller low,
+            // then the smaller hi (every range through the best layer is one
+            // of the candidates, so the row's smallest (cost, range) is it)
+            double m = on ? best : PINF;
+            int cd = on && code ? (code & 15) << 4 | code >> 4 : 0x11;
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) {
+                const double om = __shfl_xor(m, o, 16);
+                const int oc = __shfl_xor(cd, o, 16);
+                if (om < m || (om == m && oc < cd)) { m = om; cd = oc; }
+            }
+            if (lane == 0 && nn > 0) pick[0] = (cd >> 4) | (cd & 15) << 4;
+            break;
+        }
+        // edge to the parent: cost by parent layer and the child layer it uses
+        double up = INF;
+        int uc = 0;
+        int u = 0;
+        if (act) u = pos[par[i]] % XY;
+        const int w = v % XY;
+        const bool straight = w / Y == u / Y || w % Y == u % Y;
+        if (__ballot(act && straight)) {
+            const bool along = dl == 0 ? w % Y == u % Y : w / Y == u / Y;
+            if (act && straight && on && along) {
+                up = best + in.wc;
+                uc = l;
+            }
+        }
+        if (__ballot(act && !straight)) {
+            const double from = best + in.wc;
+            double cu = INF;
+            int cc = 0;
+            unrolled<L>([&](auto I) {
+                // child layer I; the corner's vias lie on the layers between,
+                // where the child's direction meets the parent's
+                constexpr int cl = I;
+                const bool vert = layer_dir(cl, g.DIR) == 1;
+                const double cost1 = row_bcast<cl + 1>(from);
+                double cost2 = 0.0;
+                unrolled<L>([&](auto K) {
+                    constexpr int k = K;
+                    if constexpr (k != cl && k != 0) {
+                        const float cut = row_bcast<k + 1>(vert ? in.va : in.vb);
+                        const bool between = k > cl ? k < l : k > l;
+                        cost2 += between ? (double)cut : 0.0;
                     }
-            }
-            smcc[gi][l] = m;
-            scf[gi][l] = cf;
-            swc[gi][l] = wc;
-            sva[gi][l] = va;
-            svb[gi][l] = vb;
+                });
+                cost2 += in.wp;
+                const double sum = cost1 + cost2;
+                const bool take = (((cl ^ l) & 1) != 0) & (sum < cu);
+                cu = take ? sum : cu;
+                cc = take ? cl : cc;
+            });
+            if (!straight) { up = cu; uc = cc; }
+        }
+        if (act && on) {
+            mcp[i * L + l] = up;
+            curl_of[i * 16 + l] = (uint8_t)uc;
         }
         __syncthreads();
-        if (act) {
-            double best = INF;
-            int bp = 0;
-            if (straight) {
-                const int d = layer_dir(l, g.DIR);
-                if (!((d == 0 && y != py) || (d == 1 && x != px))) {
-                    best = smcc[gi][l] + wc;
-                    bp = scf[gi][l] * LL + l * L + l;
-                }
-            } else {
-                // Lane l is the parent-side layer; child-side layers of the
-                // other parity in increasing order, strict < keeps the first.
-                for (int curl = (l & 1) ^ 1; curl < L; curl += 2) {
-                    const double cost = smcc[gi][curl] + swc[gi][curl];
-                    const double* vv = layer_dir(curl, g.DIR) == 1 ? sva[gi] : svb[gi];
-                    double cost2 = 0;
-                    for (int k = min(curl, l) + 1; k < max(curl, l); k++) cost2 += vv[k];
-                    cost2 += wp;
-                    if (cost + cost2 < best) {
-                        best = cost + cost2;
-                        bp = scf[gi][curl] * LL + curl * L + l;
-                    }
-                }
-            }
-            sdg[gi][l] = best;
-            spv[gi][l] = bp;
-        }
-        __syncthreads();
-        if (act) {
-            // Prefix minimum over maxl ('<=' keeps the lower range) added to
-            // the parent's row minl = l; back-pointers of the child.
-            const int r0 = tri_row(L, l);
-            double* pd = D + p * T + r0;
-            uint16_t* fr = F + i * T + r0;
-            double m = sdg[gi][l];
-            int pv = spv[gi][l];
-            pd[0] += m;
-            fr[0] = (uint16_t)pv;
-            for (int maxl = l + 1; maxl < L; maxl++) {
-                const double dm = sdg[gi][maxl];
-                if (!(m <= dm)) {
-                    m = dm;
-                    pv = spv[gi][maxl];
-                }
-                pd[maxl - l] += m;
-                fr[maxl - l] = (uint16_t)pv;
-            }
-        }
-        __syncthreads();
-    }
-    // Root range: min/argmin over the lanes' rows, first in (minl, maxl) order.
-    double m = __builtin_inf();
-    int code = 1 << 30;
-    if (lane < L && nn > 0) {
-        const double* row = D + tri_row(L, lane) - lane;
-        m = row[lane];
-        code = lane * L + lane;
-        for (int maxl = lane + 1; maxl < L; maxl++)
-            if (row[maxl] < m) {
-                m = row[maxl];
-                code = lane * L + maxl;
-            }
-    }
-    for (int off = 8; off >= 1; off >>= 1) {
-        const double om = __shfl_xor(m, off, 16);
-        const int oc = __shfl_xor(code, off, 16);
-        if (om < m || (om == m && oc < code)) {
-            m = om;
-            code = oc;
-        }
-    }
-    // Traceback top-down (node order is pre-order: parents first).
-    if (lane == 0 && nn > 0) {
-        slr[gi][0] = code;
-        scode[gi][0] = 0;
-        for (int i = 1; i < nn; i++) {
-            const int lp = slr[gi][sp[gi][i]];
-            const int c = F[i * T + tri_row(L, lp / L) + lp % L - lp / L];
-            scode[gi][i] = c;
-            slr[gi][i] = c / LL;
-        }
+        in = next;
     }
     __syncthreads();
+    // Top-down (parents first): within the parent's range the lowest of the
+    // cheapest layers, the child layer its edge uses, and that layer's range.
+    for (int i = 1; i < nmax; i++) {
+        const bool act = i < nn;
+        const int up = act ? pick[par[i]] : 0;
+        const int low = up & 15, hi = up >> 4 & 15;
+        double c = act && s >= low && s <= hi ? mcp[i * L + l] : PINF;
+        const double own = c;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            const double oc = __shfl_xor(c, o, 16);
+            c = oc < c ? oc : c;
+        }
+        const uint64_t mine = __ballot(act && own == c) >> (threadIdx.x & 48);
+        if (act) {
+            const int parl = __builtin_ctzll(mine | 1ull << 16) - 1;
+            const int curl = parl < L ? curl_of[i * 16 + parl] : 0;
+            const int code = range_of[i * 16 + curl];
+            if (lane == 0) pick[i] = (code ? code : 0x11) | curl << 8 | (parl & 15) << 12;
+        }
+        __syncthreads();
+    }
     if (t >= n) return;
     // Route pairs in node order: the node's via stack, then the edge to its
     // parent (one piece, or wire-via-wire for an L).
     int* r = routes + route_off[net];
-    int base = 0;
+    int done = 0;
     for (int c0 = 0; c0 < nn; c0 += 16) {
         const int i = c0 + lane;
-        int cntp = 0;
-        int minl = 0, maxl = 0, x = 0, y = 0, px = 0, py = 0, cd = 0;
+        int cnt = 0;
+        int minl = 0, maxl = 0, x = 0, y = 0, px = 0, py = 0, curl = 0, parl = 0;
         if (i < nn) {
-            minl = slr[gi][i] / L;
-            maxl = slr[gi][i] % L;
-            x = sx[gi][i];
-            y = sy[gi][i];
-            cntp = minl < maxl;
+            const int pk = pick[i], v = pos[i] % XY;
+            minl = (pk & 15) - 1;
+            maxl = (pk >> 4 & 15) - 1;
+            x = v / Y;
+            y = v - x * Y;
+            cnt = minl < maxl;
             if (i > 0) {
-                const int p = sp[gi][i];
-                px = sx[gi][p];
-                py = sy[gi][p];
-                cd = scode[gi][i];
-                cntp += (px == x || py == y) ? 1 : 3;
+                const int u = pos[par[i]] % XY;
+                px = u / Y;
+                py = u - px * Y;
+                curl = pk >> 8 & 15;
+                parl = pk >> 12;
+                cnt += (px == x || py == y) ? 1 : 3;
             }
         }
-        int incl = cntp;
+        int incl = cnt;
         for (int off = 1; off < 16; off <<= 1) {
             const int v = __shfl_up(incl, off, 16);
             if (lane >= off) incl += v;
         }
         const int total = __shfl(incl, 15, 16);
         if (i < nn) {
-            int k = 1 + 2 * (base + incl - cntp);
+            int* o = r + 1 + 2 * (done + incl - cnt);
             auto push = [&](int a, int b) {
-                r[k] = a;
-                r[k + 1] = b;
-                k += 2;
+                o[0] = a;
+                o[1] = b;
+                o += 2;
             };
             if (minl < maxl) {
                 push(minl * XY + x * Y + y, maxl * XY + x * Y + y);
-                if (g.vc) emit_via(g, minl, maxl, x, y);
+                emit_via(g, minl, maxl, x, y);
             }
             if (i > 0) {
                 const int minx = min(x, px), maxx = max(x, px), miny = min(y, py), maxy = max(y, py);
-                const int curl = cd / L % L, parl = cd % L;
                 if (px == x || py == y) {
                     push(curl * XY + minx * Y + miny, curl * XY + maxx * Y + maxy);
                     add_segment(g, curl, minx, maxx, miny, maxy, stamp);
-                } else if (layer_dir(curl, g.DIR) == 1) {
-                    push(curl * XY + x * Y + y, curl * XY + x * Y + py);
-                    add_segment(g, curl, x, x, miny, maxy, stamp);
-                    push(curl * XY + x * Y + py, parl * XY + x * Y + py);
-                    if (g.vc) emit_via(g, curl, parl, x, py);
-                    push(parl * XY + x * Y + py, parl * XY + px * Y + py);
-                    add_segment(g, parl, minx, maxx, py, py, stamp);
                 } else {
-                    push(curl * XY + x * Y + y, curl * XY + px * Y + y);
-                    add_segment(g, curl, minx, maxx, y, y, stamp);
-                    push(curl * XY + px * Y + y, parl * XY + px * Y + y);
-                    if (g.vc) emit_via(g, curl, parl, px, y);
-                    push(parl * XY + px * Y + y, parl * XY + px * Y + py);
-                    add_segment(g, parl, px, px, miny, maxy, stamp);
+                    // the corner (x, py) when the child's layer runs along y, else (px, y)
+                    const bool vert = layer_dir(curl, g.DIR) == 1;
+                    const int hx = vert ? x : px, hy = vert ? py : y;
+                    push(curl * XY + x * Y + y, curl * XY + hx * Y + hy);
+                    add_segment(g, curl, min(x, hx), max(x, hx), min(y, hy), max(y, hy), stamp);
+                    push(curl * XY + hx * Y + hy, parl * XY + hx * Y + hy);
+                    emit_via(g, curl, parl, hx, hy);
+                    push(parl * XY + hx * Y + hy, parl * XY + px * Y + py);
+                    add_segment(g, parl, min(px, hx), max(px, hx), min(py, hy), max(py, hy), stamp);
                 }
             }
         }
-        base += total;
+        done += total;
     }
-    if (lane == 0) r[0] = 1 + 2 * base;
-}
-
-
-// LDS bytes of one k_lshape_wave block.
-constexpr int lswave_lds(int L, int NC, int G) {
-    return G * (NC * (L * (L + 1) / 2) * 10 + NC * 24 + NC * (L > 1 ? L - 1 : 1) * 4 + L * 48 + 4);
-}
-constexpr int lswave_groups(int L, int NC) {
-    return lswave_lds(L, NC, 4) <= 60 * 1024 ? 4 : lswave_lds(L, NC, 2) <= 60 * 1024 ? 2 : 1;
-}
-
-template <int L, int NC, int G>
-void lswave_launch_g(igr_ctx* c, const int* d_nets, int64_t n, int stamp) {
-    NetsDev& N = c->nets;
-    const unsigned grid = (unsigned)((n + G - 1) / G);
-    k_lshape_wave<L, NC, G><<<grid, 16 * G, 0, c->stream>>>(c->g, d_nets, n, N.node_off.p, N.node.p, N.parent.p,
-                                                            N.route_off.p, N.routes.p, stamp);
-}
-
-// Nets per workgroup: the tuned count, capped by what the LDS holds, or the
-// largest that fits.
-template <int L, int NC>
-void lswave_launch(igr_ctx* c, const int* d_nets, int64_t n, int stamp) {
-    constexpr int GMAX = lswave_groups(L, NC);
-    const int G = c->tune.lshape_groups ? std::min(c->tune.lshape_groups, GMAX) : GMAX;
-    if (G >= 4 && GMAX >= 4) lswave_launch_g<L, NC, (GMAX >= 4 ? 4 : 1)>(c, d_nets, n, stamp);
-    else if (G >= 2 && GMAX >= 2) lswave_launch_g<L, NC, (GMAX >= 2 ? 2 : 1)>(c, d_nets, n, stamp);
-    else lswave_launch_g<L, NC, 1>(c, d_nets, n, stamp);
-}
-
-template <int L>
-void lswave_launch_l(igr_ctx* c, const int* d_nets, int64_t n, int cls, int stamp) {
-    switch (cls) {
-    case 0: lswave_launch<L, 4>(c, d_nets, n, stamp); break;
-    case 1: lswave_launch<L, 8>(c, d_nets, n, stamp); break;
-    case 2: lswave_launch<L, 16>(c, d_nets, n, stamp); break;
-    default: lswave_launch<L, LSWAVE_MAX_NODES>(c, d_nets, n, stamp); break;
-    }
+    if (lane == 0) r[0] = 1 + 2 * done;
 }
 
 } // namespace
 
-int lshape_wave_class(int nodes) {
-    return nodes <= 4 ? 0 : nodes <= 8 ? 1 : nodes <= 16 ? 2 : nodes <= LSWAVE_MAX_NODES ? 3 : -1;
-}
-
-void launch_lshape_wave(igr_ctx* c, const int* d_nets, int64_t n, int cls, int stamp, double bytes) {
+void launch_lshape_wave(igr_ctx* c, const int* d_nets, int64_t n, int nodes, int stamp, double bytes) {
     if (n == 0) return;
-    if (cls < 0 || cls > 3) throw std::runtime_error("L-shape node-count class out of range");
+    if (nodes < 1 || nodes > LSWAVE_MAX_NODES) throw std::runtime_error("L-shape node count out of range");
     KScope ks(c, K_LSHAPE, bytes);
-#define CASE(LV)                                            \
-    case LV: lswave_launch_l<LV>(c, d_nets, n, cls, stamp); break;
+    NetsDev& N = c->nets;
+    const unsigned grid = (unsigned)((n + 3) / 4);
+#define CASE(LV)                                                                                                    \
+    case LV:                                                                                                        \
+        k_lshape_wave<LV><<<grid, 64, 4 * lswave_net_lds(LV, nodes), c->stream>>>(                                  \
+            c->g, d_nets, n, nodes, N.node_off.p, N.node.p, N.parent.p, N.route_off.p, N.routes.p, stamp);          \
+        break;
     switch (c->g.L) {
         CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12)
     default: throw std::runtime_error("unsupported routing layer count");
