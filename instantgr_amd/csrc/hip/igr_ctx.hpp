@@ -109,9 +109,10 @@ struct Sched {
     // batched form: per-cell net lists, their heads and the round-0 map; the
     // compacted unassigned / active net lists; release-driven rounds: the
     // released cells, new owners, committed nets and their cells, with stamps
-    DevBuf<int> base, cnt, c_net, ctrl, lists, rel, cand, cstamp, comm, hits, hstamp;
+    DevBuf<int> base, cnt, c_net, ctrl, lists, rel, cand, cstamp, hits, hstamp;
     DevBuf<int64_t> head, c_off, c_end, bsum, cur;
     DevBuf<unsigned long long> stat;
+    DevBuf<uint8_t> sn;           // the nets' records
     DevBuf<int> bits;             // per-net state bits (assigned, blocked in this batch)
 };
 

@@ -42,12 +42,20 @@
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 namespace igr_dev {
 
 namespace {
 
 constexpr int TPB = 256;
+// Threads of the kernels that append to a list or count: a workgroup's appends
+// cost one returning atomic on one counter, and those serialise at some 20 ns
+// each, so at most 512 large workgroups.  Average launch on a 1500x1500 grid,
+// 1.6M nets (release-driven), against 256 threads with an atomic per append or
+// per 256-thread workgroup: viability 11 us (76), commit 18 (93), round end 27
+// (46), released-cell claims 22 (28).
+constexpr int LTPB = 1024;
 constexpr int ROUNDS = 30;        // rounds per batch (src/database_cuda.hpp:612)
 
 // control state words (two slots of C_WORDS, then the placed-net counter).
@@ -56,7 +64,7 @@ constexpr int ROUNDS = 30;        // rounds per batch (src/database_cuda.hpp:612
 // active list (C_NA < 0: the unassigned list itself).  Release-driven rounds:
 // the round-0 candidates (below); C_NV0, the nets round 0 found viable (list
 // v0); C_NR, cells the previous round released (list rel); C_NK, new owners
-// of those cells (list cand); C_NC, nets committed in this round (list comm);
+// of those cells (list cand); C_NC, nets committed in this round;
 // C_NH, cells those nets own (list hits).
 // C_LASTC, nets placed when the lists were last compacted.
 enum { C_DONE = 0, C_CUR, C_ROUND, C_COMMIT, C_HAVE, C_NVIABLE, C_NU, C_UL, C_NA, C_AL, C_NR, C_NK, C_NC, C_NH,
@@ -64,11 +72,16 @@ enum { C_DONE = 0, C_CUR, C_ROUND, C_COMMIT, C_HAVE, C_NVIABLE, C_NU, C_UL, C_NA
 constexpr int NLISTS = 3;         // net list buffers of n entries each
 constexpr int COMPACT_DIV = 64;   // release-driven rounds: compact the cell lists every n/64 placed nets
 
+// A net by scheduler index: its points, and its net id for the segments.  One
+// load where the index, the row and two offsets were a chain of three.
+struct alignas(16) SNet {
+    int64_t pt0;
+    int npt, net;
+};
+
 struct BArgs {
     int64_t n;
-    const int* ids;               // scheduler index -> net id (segments)
-    const int* pids;              // scheduler index -> row of the point arrays
-    const int64_t* pt_off;
+    const SNet* sn;
     const int* pt;
     const int64_t* hs_off;
     const int* hs;
@@ -89,7 +102,6 @@ struct BArgs {
     int* cstamp;                  // per net: 1 + the round that listed it in cand, -(1 + g) when the
                                   // end of round g listed it as a round-0 candidate
     int* v0;                      // nets viable in round 0 of the batch
-    int* comm;                    // nets committed this round
     int* hits;                    // X*Y cells owned by the nets committed this round
     int* hstamp;                  // per cell: 1 + the round that listed it in hits
     int64_t* cur;                 // X*Y: no active net before this entry of the cell's list in this batch
@@ -161,13 +173,15 @@ __device__ __forceinline__ bool active(const BArgs& a, int64_t i) { return nstat
 __global__ void k_cell_count(BArgs a, int* cnt) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i >= a.n) return;
-    for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++) atomicAdd(&cnt[a.pt[k]], 1);
+    const SNet s = a.sn[i];
+    for (int64_t k = s.pt0; k < s.pt0 + s.npt; k++) atomicAdd(&cnt[a.pt[k]], 1);
 }
 
 __global__ void k_cell_fill(BArgs a, int* fillc) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i >= a.n) return;
-    for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++) {
+    const SNet s = a.sn[i];
+    for (int64_t k = s.pt0; k < s.pt0 + s.npt; k++) {
         const int p = a.pt[k];
         const int pos = atomicAdd(&fillc[p], 1);
         a.c_net[a.c_off[p] + pos] = (int)i;
@@ -287,9 +301,9 @@ __device__ __forceinline__ uint64_t group_bits(uint64_t m, int G) {
 
 // Appends v to list for every thread with want, one counter atomic per
 // workgroup (a returning atomic per wave on one counter serialises thousands
-// of waves).  Every thread of the workgroup calls it; s holds TPB/64+1 ints.
+// of waves).  Every thread of the workgroup calls it; s holds LTPB/64+1 ints.
 __device__ __forceinline__ void block_append(bool want, int v, int* counter, int* list, int* s) {
-    constexpr int NW = TPB / 64;
+    constexpr int NW = LTPB / 64;
     const uint64_t m = __ballot(want);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) s[wv] = __popcll(m);
@@ -315,7 +329,7 @@ __device__ __forceinline__ void block_append(bool want, int v, int* counter, int
 // lane that takes the offsets is one of them); entries beyond the LDS
 // capacity go out at once.  Every thread of the workgroup calls init() and
 // flush().
-constexpr int GL_CAP = 2048;
+constexpr int GL_CAP = 4096;
 struct GroupList {
     int* buf;                     // LDS, GL_CAP entries
     int* hdr;                     // LDS: count, then the list offset
@@ -358,45 +372,54 @@ template <class F>
 __device__ __forceinline__ void wave_segment_cells(const BArgs& a, int net, F f) {
     const int lane = threadIdx.x & 63;
     const int Y = a.Y, sp = a.sparsity;
-    for (int dir = 0; dir < 2; dir++) {
-        const int64_t s0 = dir ? a.vs_off[net] : a.hs_off[net];
-        const int64_t s1 = dir ? a.vs_off[net + 1] : a.hs_off[net + 1];
-        const int* seg = dir ? a.vs : a.hs;
-        for (int64_t sb = s0; sb < s1; sb += 64) {
-            const int64_t k = sb + lane;
-            int cnt = 0, first = 0, step = 0;
-            if (k < s1) {
-                const int b = seg[2 * k], e = seg[2 * k + 1];
-                if (dir == 0) {          // along x at y = b % Y
-                    const int x0 = b / Y, x1 = e / Y;
-                    cnt = x1 >= x0 ? (x1 - x0) / sp + 1 : 0;
-                    first = x0 * Y + b % Y;
-                    step = sp * Y;
-                } else {                 // along y at x = b / Y
-                    const int y0 = b % Y, y1 = e % Y;
-                    cnt = y1 >= y0 ? (y1 - y0) / sp + 1 : 0;
-                    first = (b / Y) * Y + y0;
-                    step = sp;
-                }
-            }
-            int incl = cnt;              // inclusive scan of the cell counts
-            for (int d = 1; d < 64; d <<= 1) {
-                const int v = __shfl_up(incl, d);
-                if (lane >= d) incl += v;
-            }
-            const int total = __shfl(incl, 63);
-            const int excl = incl - cnt;
-            for (int cb = 0; cb < total; cb += 64) {
-                const int c = cb + lane;
-                int sg = 0;              // the first lane whose inclusive count exceeds c
-                for (int b2 = 32; b2 > 0; b2 >>= 1)
-                    if (__shfl(incl, sg + b2 - 1) <= c) sg += b2;
-                const int f0 = __shfl(first, sg), st0 = __shfl(step, sg), ex = __shfl(excl, sg);
-                const bool valid = c < total;
-                f(valid, valid ? f0 + (c - ex) * st0 : 0);
-            }
+    const int64_t h0 = a.hs_off[net], v0 = a.vs_off[net];
+    const int nh = (int)(a.hs_off[net + 1] - h0), ns = nh + (int)(a.vs_off[net + 1] - v0);
+    for (int sb = 0; sb < ns; sb += 64) {
+        const int k = sb + lane;
+        int cnt = 0, first = 0, step = 0;
+        if (k < ns) {
+            const bool hor = k < nh;
+            const int* seg = hor ? a.hs + 2 * (h0 + k) : a.vs + 2 * (v0 + k - nh);
+            const int b = seg[0], e = seg[1];
+            const int bx = b / Y, by = b - bx * Y, ex = e / Y, ey = e - ex * Y;
+            const int span = hor ? ex - bx : ey - by;   // along x at y = by, or along y at x = bx
+            cnt = span >= 0 ? span / sp + 1 : 0;
+            first = b;
+            step = hor ? sp * Y : sp;
+        }
+        int incl = cnt;                  // inclusive scan of the cell counts
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(incl, d);
+            if (lane >= d) incl += v;
+        }
+        const int total = __shfl(incl, 63);
+        const int excl = incl - cnt;
+        for (int cb = 0; cb < total; cb += 64) {
+            const int c = cb + lane;
+            int sg = 0;                  // the first lane whose inclusive count exceeds c
+            for (int b2 = 32; b2 > 0; b2 >>= 1)
+                if (__shfl(incl, sg + b2 - 1) <= c) sg += b2;
+            const int f0 = __shfl(first, sg), st0 = __shfl(step, sg), ex = __shfl(excl, sg);
+            const bool valid = c < total;
+            f(valid, valid ? f0 + (c - ex) * st0 : 0);
         }
     }
+}
+
+// Calls f(valid, q) for the rest cells of a net: the neighbour cells (0,-1),
+// (-1,0), (1,0) of its points and its sampled segment cells.
+template <class F>
+__device__ __forceinline__ void wave_rest_cells(const BArgs& a, const SNet& s, F f) {
+    const int lane = threadIdx.x & 63;
+    const int X = a.X, Y = a.Y;
+    for (int k = lane; k - lane < s.npt; k += 64) {
+        const bool in = k < s.npt;
+        const int p = in ? a.pt[s.pt0 + k] : 0, x = p / Y, y = p - x * Y;
+        f(in && y > 0, p - 1);
+        f(in && x > 0, p - Y);
+        f(in && x + 1 < X, p + Y);
+    }
+    wave_segment_cells(a, s.net, f);
 }
 
 // 3. (both) a wave per viable net claims the neighbour cells (0,-1), (-1,0),
@@ -405,21 +428,11 @@ __global__ void __launch_bounds__(TPB) k_b_claim_rest(BArgs a, int64_t g, const 
     const int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE]) return;
     const int nv = st[C_NVIABLE];
-    const int lane = threadIdx.x & 63;
-    const int X = a.X, Y = a.Y;
     unsigned long long nb = 0;
-    for (int w = (blockIdx.x * TPB + threadIdx.x) >> 6; w < nv; w += (gridDim.x * TPB) >> 6) {
+    for (int w = (threadIdx.x >> 6) * gridDim.x + blockIdx.x; w < nv; w += (gridDim.x * TPB) >> 6) {
         const int i = vlist[w];
-        const int net = a.ids[i];
-        if (lane == 0) nb += 4 + 4 + 4 + 16 + 32;   // list entry, id, row, point and segment offsets
-        for (int64_t k = a.pt_off[a.pids[i]] + lane; k < a.pt_off[a.pids[i] + 1]; k += 64) {
-            const int p = a.pt[k], x = p / Y, y = p % Y;
-            nb += 4 + 12;   // point, three neighbour claims
-            if (y - 1 >= 0) atomicMax(&a.map[x * Y + y - 1], i);
-            if (x - 1 >= 0) atomicMax(&a.map[(x - 1) * Y + y], i);
-            if (x + 1 < X) atomicMax(&a.map[(x + 1) * Y + y], i);
-        }
-        wave_segment_cells(a, net, [&](bool valid, int q) {
+        if ((threadIdx.x & 63) == 0) nb += 4 + 16 + 32;   // list entry, net record, segment offsets
+        wave_rest_cells(a, a.sn[i], [&](bool valid, int q) {
             if (valid) {
                 atomicMax(&a.map[q], i);
                 nb += 4;
@@ -427,6 +440,14 @@ __global__ void __launch_bounds__(TPB) k_b_claim_rest(BArgs a, int64_t g, const 
         });
     }
     flush_bytes(a, nb);
+}
+
+// A workgroup's commits of the round, counted once (after a barrier).
+__device__ __forceinline__ void count_commits(const BArgs& a, int* st, int won) {
+    if (threadIdx.x != 0 || won == 0) return;
+    atomicAdd(&st[C_NC], won);
+    atomicAdd(&a.ctrl[2 * C_WORDS], won);   // nets placed so far
+    st[C_COMMIT] = 1;
 }
 
 // ---- active-list rounds -----------------------------------------------------
@@ -443,9 +464,9 @@ __global__ void __launch_bounds__(TPB) k_a_claim(BArgs a, int64_t g) {
     for (int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G; t < na; t += nth) {
         const int64_t i = al[t];
         if (!active(a, i)) continue;
-        const int64_t k1 = a.pt_off[a.pids[i] + 1];
-        for (int64_t k = a.pt_off[a.pids[i]] + lg; k < k1; k += G) {
-            int* m = &a.map[a.pt[k]];
+        const SNet s = a.sn[i];
+        for (int k = lg; k < s.npt; k += G) {
+            int* m = &a.map[a.pt[s.pt0 + k]];
             if (*m < (int)i) atomicMax(m, (int)i);
         }
     }
@@ -453,9 +474,12 @@ __global__ void __launch_bounds__(TPB) k_a_claim(BArgs a, int64_t g) {
 
 // 2. active nets owning every point cell go to the viable list
 template <int G>
-__global__ void __launch_bounds__(TPB) k_a_viable(BArgs a, int64_t g, int* vlist) {
+__global__ void __launch_bounds__(LTPB) k_a_viable(BArgs a, int64_t g, int* vlist) {
+    __shared__ int s_buf[GL_CAP], s_hdr[2];
     int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE]) return;
+    GroupList gl{s_buf, s_hdr, &st[C_NVIABLE], vlist};
+    gl.init();
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         // the successor lists' counters, filled by this round's last kernel
         int* nx = a.ctrl + ((g + 1) & 1) * C_WORDS;
@@ -464,42 +488,47 @@ __global__ void __launch_bounds__(TPB) k_a_viable(BArgs a, int64_t g, int* vlist
     }
     int64_t na;
     const int* al = a_list(a, st, na);
-    const int64_t nth = (int64_t)gridDim.x * TPB / G;
+    const int64_t nth = (int64_t)gridDim.x * LTPB / G;
     const int lg = threadIdx.x & (G - 1);
     const int64_t rounds = (na + nth - 1) / nth;   // the same for every lane of the wave
     for (int64_t r = 0; r < rounds; r++) {
-        const int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G + r * nth;
+        const int64_t t = ((int64_t)blockIdx.x * LTPB + threadIdx.x) / G + r * nth;
         const int64_t i = t < na ? al[t] : 0;
         const bool live = t < na && active(a, i);
-        const int64_t k0 = live ? a.pt_off[a.pids[i]] : 0, k1 = live ? a.pt_off[a.pids[i] + 1] : 0;
+        const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
         bool fail = !live;
-        for (int64_t k = k0 + lg;; k += G) {
-            const bool f = !fail && k < k1 && a.map[a.pt[k]] != (int)i;
+        for (int k = lg;; k += G) {
+            const bool f = !fail && k < s.npt && a.map[a.pt[s.pt0 + k]] != (int)i;
             fail = fail || group_bits(__ballot(f), G) != 0;
-            if (__ballot(!fail && k + G < k1) == 0) break;
+            if (__ballot(!fail && k + G < s.npt) == 0) break;
         }
-        if (lg == 0 && !fail) vlist[atomicAdd(&st[C_NVIABLE], 1)] = (int)i;
+        gl.add(lg == 0 && !fail, (int)i);
     }
+    gl.flush();
 }
 
 // 4. a wave per viable net: commit it if it still owns every point cell
-__global__ void __launch_bounds__(TPB) k_a_commit(BArgs a, int64_t g, const int* vlist) {
+__global__ void __launch_bounds__(LTPB) k_a_commit(BArgs a, int64_t g, const int* vlist) {
+    __shared__ int s_won;
     int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE]) return;
+    if (threadIdx.x == 0) s_won = 0;
+    __syncthreads();
     const int nv = st[C_NVIABLE];
     const int lane = threadIdx.x & 63;
-    for (int w = (blockIdx.x * TPB + threadIdx.x) >> 6; w < nv; w += (gridDim.x * TPB) >> 6) {
+    for (int w = (blockIdx.x * LTPB + threadIdx.x) >> 6; w < nv; w += (gridDim.x * LTPB) >> 6) {
         const int i = vlist[w];
+        const SNet s = a.sn[i];
         bool lost = false;
-        for (int64_t k = a.pt_off[a.pids[i]] + lane; k < a.pt_off[a.pids[i] + 1]; k += 64)
-            lost = lost || a.map[a.pt[k]] != i;
+        for (int k = lane; k < s.npt; k += 64) lost = lost || a.map[a.pt[s.pt0 + k]] != i;
         if (__ballot(lost) == 0 && lane == 0) {
             a.batch[i] = st[C_CUR];
             set_assigned(a, i);
-            atomicAdd(&a.ctrl[2 * C_WORDS], 1);   // nets placed so far
-            st[C_COMMIT] = 1;
+            atomicAdd(&s_won, 1);
         }
     }
+    __syncthreads();
+    count_commits(a, st, s_won);
 }
 
 // 5. after a commit: active nets with a point cell owned by a committed net
@@ -517,16 +546,16 @@ __global__ void __launch_bounds__(TPB) k_a_revert(BArgs a, int64_t g) {
         const int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G + r * nth;
         const int64_t i = t < na ? al[t] : 0;
         const bool live = t < na && active(a, i);
-        const int64_t k0 = live ? a.pt_off[a.pids[i]] : 0, k1 = live ? a.pt_off[a.pids[i] + 1] : 0;
+        const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
         bool hit = false;
-        for (int64_t k = k0 + lg;; k += G) {
+        for (int k = lg;; k += G) {
             bool h = false;
-            if (live && !hit && k < k1) {
-                const int pre = a.map[a.pt[k]];
+            if (!hit && k < s.npt) {
+                const int pre = a.map[a.pt[s.pt0 + k]];
                 h = pre != -1 && assigned(a, pre);
             }
             hit = hit || group_bits(__ballot(h), G) != 0;
-            if (__ballot(live && !hit && k + G < k1) == 0) break;
+            if (__ballot(!hit && k + G < s.npt) == 0) break;
         }
         if (lg == 0 && live && hit) {
             set_blocked(a, i);
@@ -540,12 +569,12 @@ __global__ void __launch_bounds__(TPB) k_a_revert(BArgs a, int64_t g) {
 //    the kept map with every unassigned net active.  The successor lists go
 //    to a buffer neither current list uses.  Thread 0 writes the successor
 //    control state.
-__global__ void __launch_bounds__(TPB) k_a_clear_end(BArgs a, int64_t g, int64_t cells) {
-    __shared__ int s_app[TPB / 64 + 1];
+__global__ void __launch_bounds__(LTPB) k_a_clear_end(BArgs a, int64_t g, int64_t cells) {
+    __shared__ int s_app[LTPB / 64 + 1];
     const int* st = a.ctrl + (g & 1) * C_WORDS;
     int* nx = a.ctrl + ((g + 1) & 1) * C_WORDS;
-    const int64_t t = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * TPB;   // grid-stride over cells and list entries
+    const int64_t t = (int64_t)blockIdx.x * LTPB + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * LTPB;   // grid-stride over cells and list entries
     const bool done = st[C_DONE] != 0;
     const bool commit = st[C_COMMIT] != 0;
     const int round = st[C_ROUND];
@@ -651,19 +680,19 @@ __global__ void __launch_bounds__(TPB) k_a_clear_end(BArgs a, int64_t g, int64_t
 //    which joins the viability test.  A group of G lanes scans a cell's list
 //    G entries a step.
 template <int G>
-__global__ void __launch_bounds__(TPB) k_r_claim(BArgs a, int64_t g) {
+__global__ void __launch_bounds__(LTPB) k_r_claim(BArgs a, int64_t g) {
     __shared__ int s_buf[GL_CAP], s_hdr[2];
     int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE] || st[C_ROUND] == 0) return;
     GroupList gl{s_buf, s_hdr, &st[C_NK], a.cand};
     gl.init();
     const int64_t nr = st[C_NR];
-    const int64_t nth = (int64_t)gridDim.x * TPB / G;
+    const int64_t nth = (int64_t)gridDim.x * LTPB / G;
     const int lg = threadIdx.x & (G - 1);
     const int64_t rounds = (nr + nth - 1) / nth;   // the same for every thread
     unsigned long long nb = 0;
     for (int64_t r = 0; r < rounds; r++) {
-        const int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G + r * nth;
+        const int64_t t = ((int64_t)blockIdx.x * LTPB + threadIdx.x) / G + r * nth;
         const bool live = t < nr;
         const int q = live ? a.rel[t] : 0;
         int64_t h = live ? a.cur[q] : 0;
@@ -702,9 +731,12 @@ __global__ void __launch_bounds__(TPB) k_r_claim(BArgs a, int64_t g) {
 // 2. the nets under test (every unassigned net in round 0, the new owners of
 //    released cells later) that own every point cell go to the viable list
 template <int G>
-__global__ void __launch_bounds__(TPB) k_r_viable(BArgs a, int64_t g, int* vlist) {
+__global__ void __launch_bounds__(LTPB) k_r_viable(BArgs a, int64_t g, int* vlist) {
+    __shared__ int s_buf[GL_CAP], s_hdr[2];
     int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE]) return;
+    GroupList gl{s_buf, s_hdr, &st[C_NVIABLE], vlist};
+    gl.init();
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         // the successor lists' counters, filled by this round's last kernel
         int* nx = a.ctrl + ((g + 1) & 1) * C_WORDS;
@@ -713,30 +745,28 @@ __global__ void __launch_bounds__(TPB) k_r_viable(BArgs a, int64_t g, int* vlist
     }
     int64_t na;
     const int* al = r_list(a, st, na);
-    const int64_t nth = (int64_t)gridDim.x * TPB / G;
+    const int64_t nth = (int64_t)gridDim.x * LTPB / G;
     const int lg = threadIdx.x & (G - 1);
     const int64_t rounds = (na + nth - 1) / nth;   // the same for every lane of the wave
     unsigned long long nb = 0;
     for (int64_t r = 0; r < rounds; r++) {
-        const int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G + r * nth;
+        const int64_t t = ((int64_t)blockIdx.x * LTPB + threadIdx.x) / G + r * nth;
         const int64_t i = t < na ? al[t] : 0;
         const bool live = t < na && active(a, i);
-        if (t < na && lg == 0) nb += 4 + 4 + (live ? 4 + 16 : 0);   // entry, state, row, point offsets
-        const int64_t k0 = live ? a.pt_off[a.pids[i]] : 0, k1 = live ? a.pt_off[a.pids[i] + 1] : 0;
+        if (t < na && lg == 0) nb += 4 + 4 + (live ? 16 : 0);   // entry, state, net record
+        const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
         bool fail = !live;
-        for (int64_t k = k0 + lg;; k += G) {
-            const bool chk = !fail && k < k1;
-            const bool f = chk && a.map[a.pt[k]] != (int)i;
+        for (int k = lg;; k += G) {
+            const bool chk = !fail && k < s.npt;
+            const bool f = chk && a.map[a.pt[s.pt0 + k]] != (int)i;
             if (chk) nb += 8;   // point, map cell
             fail = fail || group_bits(__ballot(f), G) != 0;
-            if (__ballot(!fail && k + G < k1) == 0) break;
+            if (__ballot(!fail && k + G < s.npt) == 0) break;
         }
-        if (lg == 0 && !fail) {
-            vlist[atomicAdd(&st[C_NVIABLE], 1)] = (int)i;
-            if (st[C_ROUND] == 0) a.v0[atomicAdd(&st[C_NV0], 1)] = (int)i;
-            nb += st[C_ROUND] == 0 ? 8 : 4;
-        }
+        if (lg == 0 && !fail) nb += 4;
+        gl.add(lg == 0 && !fail, (int)i);
     }
+    gl.flush();
     flush_bytes(a, nb);
 }
 
@@ -745,56 +775,51 @@ __global__ void __launch_bounds__(TPB) k_r_viable(BArgs a, int64_t g, int* vlist
 //    neighbours, sampled segment cells), once each.  Commits do not change
 //    the map, so a net's cells are the same whichever nets of the round
 //    commit around it.
-__global__ void __launch_bounds__(TPB) k_r_commit(BArgs a, int64_t g, const int* vlist) {
-    __shared__ int s_buf[GL_CAP], s_hdr[2];
+__global__ void __launch_bounds__(LTPB) k_r_commit(BArgs a, int64_t g, const int* vlist) {
+    __shared__ int s_buf[GL_CAP], s_hdr[2], s_won;
     int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE]) return;
     GroupList gl{s_buf, s_hdr, &st[C_NH], a.hits};
+    if (threadIdx.x == 0) s_won = 0;
     gl.init();
     const int nv = st[C_NVIABLE];
     const int lane = threadIdx.x & 63;
-    const int X = a.X, Y = a.Y;
     const int stamp = (int)g + 1;
     unsigned long long nb = 0;
-    for (int w = (blockIdx.x * TPB + threadIdx.x) >> 6; w < nv; w += (gridDim.x * TPB) >> 6) {
+    for (int w = (threadIdx.x >> 6) * gridDim.x + blockIdx.x; w < nv; w += (gridDim.x * LTPB) >> 6) {
         const int i = vlist[w];
-        const int64_t k0 = a.pt_off[a.pids[i]], k1 = a.pt_off[a.pids[i] + 1];
-        if (lane == 0) nb += 4 + 4 + 16;   // list entry, row, point offsets
+        const SNet s = a.sn[i];
+        // round 0's viable nets: the batch end lists those still unassigned
+        if (lane == 0 && st[C_ROUND] == 0) a.v0[w] = i;
+        if (lane == 0) nb += 4 + 16 + 32;   // list entry, net record, segment offsets
         bool lost = false;
-        for (int64_t k = k0 + lane; k < k1; k += 64) {
-            lost = lost || a.map[a.pt[k]] != i;
+        for (int k = lane; k < s.npt; k += 64) {
+            lost = lost || a.map[a.pt[s.pt0 + k]] != i;
             nb += 8;   // point, map cell
         }
         if (__ballot(lost) != 0) continue;
         if (lane == 0) {
-            a.comm[atomicAdd(&st[C_NC], 1)] = i;
             a.batch[i] = st[C_CUR];
             set_assigned(a, i);
-            atomicAdd(&a.ctrl[2 * C_WORDS], 1);   // nets placed so far
-            st[C_COMMIT] = 1;
-            nb += 16 + 16;   // committed entry, batch, state word; segment offsets
+            atomicAdd(&s_won, 1);
+            nb += 8;   // batch, state word
         }
-        auto hit = [&](int q) {
-            const bool own = a.map[q] == i;
+        auto hit = [&](bool own, int q) {
             const bool h = own && atomicExch(&a.hstamp[q], stamp) != stamp;
-            nb += 4 + (own ? 8 : 0) + (h ? 4 : 0);   // map cell, stamp, hit entry
+            nb += (own ? 8 : 0) + (h ? 4 : 0);   // stamp, hit entry
             gl.add(h, q);
         };
-        for (int64_t k = k0 + lane; k < k1; k += 64) {
-            const int p = a.pt[k], x = p / Y, y = p % Y;
-            hit(p);
-            if (y - 1 >= 0) hit(x * Y + y - 1);
-            if (x - 1 >= 0) hit((x - 1) * Y + y);
-            if (x + 1 < X) hit((x + 1) * Y + y);
+        for (int k = lane; k - lane < s.npt; k += 64) {
+            const bool in = k < s.npt;
+            hit(in, in ? a.pt[s.pt0 + k] : 0);
         }
-        wave_segment_cells(a, a.ids[i], [&](bool valid, int q) {
-            const bool own = valid && a.map[q] == i;
-            const bool h = own && atomicExch(&a.hstamp[q], stamp) != stamp;
-            if (valid) nb += 4 + (own ? 8 : 0) + (h ? 4 : 0);
-            gl.add(h, q);
+        wave_rest_cells(a, s, [&](bool valid, int q) {
+            if (valid) nb += 4;
+            hit(valid && a.map[q] == i, q);
         });
     }
     gl.flush();
+    count_commits(a, st, s_won);
     flush_bytes(a, nb);
 }
 
@@ -838,12 +863,12 @@ __global__ void __launch_bounds__(TPB) k_r_block(BArgs a, int64_t g) {
 //    the kept map with every unassigned net active.  The successor lists go
 //    to a buffer neither current list uses.  Thread 0 writes the successor
 //    control state.
-__global__ void __launch_bounds__(TPB) k_r_clear_end(BArgs a, int64_t g, int64_t cells) {
+__global__ void __launch_bounds__(LTPB) k_r_clear_end(BArgs a, int64_t g, int64_t cells) {
     __shared__ int s_buf[GL_CAP], s_hdr[2];
     const int* st = a.ctrl + (g & 1) * C_WORDS;
     int* nx = a.ctrl + ((g + 1) & 1) * C_WORDS;
-    const int64_t t = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * TPB;   // grid-stride over cells and list entries
+    const int64_t t = (int64_t)blockIdx.x * LTPB + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * LTPB;   // grid-stride over cells and list entries
     const bool done = st[C_DONE] != 0;
     const bool commit = st[C_COMMIT] != 0;
     const int round = st[C_ROUND];
@@ -930,7 +955,7 @@ __global__ void __launch_bounds__(TPB) k_r_clear_end(BArgs a, int64_t g, int64_t
                     gl.add(want, b);
                 }
             }
-            const int64_t nv0 = st[C_NV0], vpasses = (nv0 + stride - 1) / stride;
+            const int64_t nv0 = round == 0 ? st[C_NVIABLE] : st[C_NV0], vpasses = (nv0 + stride - 1) / stride;
             for (int64_t ps = 0; ps < vpasses; ps++) {
                 const int64_t u = ps * stride + t;
                 const int i = u < nv0 ? a.v0[u] : 0;
@@ -1008,7 +1033,7 @@ __global__ void __launch_bounds__(TPB) k_r_clear_end(BArgs a, int64_t g, int64_t
         nx[C_HAVE] = have;
         nx[C_COMMIT] = 0;
         nx[C_NVIABLE] = 0;
-        nx[C_NV0] = !done && end ? 0 : st[C_NV0];
+        nx[C_NV0] = done ? st[C_NV0] : end ? 0 : round == 0 ? st[C_NVIABLE] : st[C_NV0];
         nx[C_LASTC] = !done && end && (int64_t)(a.ctrl[2 * C_WORDS] - st[C_LASTC]) * COMPACT_DIV >= a.n
                           ? a.ctrl[2 * C_WORDS]
                           : st[C_LASTC];
@@ -1029,15 +1054,24 @@ __global__ void __launch_bounds__(TPB) k_r_clear_end(BArgs a, int64_t g, int64_t
     flush_bytes(a, nb);
 }
 
-__global__ void k_fill_b(int* p, int64_t n, int v) {
+// Net records.  Scheduler index i is entry n - 1 - i of the order (its net
+// 'order' and, where the points come per entry, its row of the point arrays).
+__global__ void k_nets(int64_t n, const int* order, const int64_t* pt_off, bool by_entry, SNet* sn) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i < n) p[i] = v;
+    if (i >= n) return;
+    const int net = order[n - 1 - i];
+    const int64_t row = by_entry ? n - 1 - i : net;
+    const int64_t p0 = pt_off[row];
+    sn[i] = SNet{p0, (int)(pt_off[row + 1] - p0), net};
 }
 
 // Start state: every net unassigned and active, listed in buffer 0.
 __global__ void k_start(BArgs a) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i < a.n) a.lists[i] = (int)i;
+    if (i < a.n) {
+        a.lists[i] = (int)i;
+        a.batch[i] = -1;
+    }
     if (i == 0) {
         a.ctrl[C_NU] = (int)a.n;
         a.ctrl[C_UL] = 0;
@@ -1058,14 +1092,11 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     Sched& S = c->sched;
     NetsDev& N = c->nets;
     hipStream_t st = c->stream;
-    std::vector<int> ids(n);
-    for (int64_t i = 0; i < n; i++) ids[i] = h_order[n - 1 - i];
-    S.ids.upload(ids.data(), n, st);
-    if (d_pt_off) {
-        std::vector<int> pids(n);
-        for (int64_t i = 0; i < n; i++) pids[i] = (int)(n - 1 - i);
-        S.pids.upload(pids.data(), n, st);
-    }
+    S.ids.upload(h_order, n, st);
+    S.sn.alloc(16 * (size_t)n);
+    SNet* sn = reinterpret_cast<SNet*>(S.sn.p);
+    k_nets<<<blocks(n), TPB, 0, st>>>(n, S.ids.p, d_pt_off ? d_pt_off : N.pt_off.p, d_pt_off != nullptr, sn);
+    HIP_OK(hipGetLastError());
     const int64_t XYc = (int64_t)c->g.X * c->g.Y;
     S.map.alloc(XYc);
     S.base.alloc(XYc);
@@ -1082,7 +1113,6 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         S.rel.alloc(XYc);
         S.cand.alloc(n);
         S.cstamp.zero(n, st);
-        S.comm.alloc(n);
         S.hits.alloc(XYc);
         S.hstamp.zero(XYc, st);
         S.cur.alloc(XYc);
@@ -1091,12 +1121,12 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     S.ctrl.zero(2 * C_WORDS + 1, st);
     const int64_t nwords = (n + 15) / 16;
     S.bits.zero(nwords, st);
-    BArgs a{n, S.ids.p, d_pt_off ? S.pids.p : S.ids.p, d_pt_off ? d_pt_off : N.pt_off.p, d_pt_off ? d_pt : N.pt.p,
+    BArgs a{n, sn, d_pt_off ? d_pt : N.pt.p,
             N.hs_off.p, N.hs.p, N.vs_off.p, N.vs.p, S.map.p, S.base.p, S.c_off.p, S.c_end.p, nullptr, S.head.p,
             S.batch.p, S.ctrl.p, S.lists.p,
             release ? S.rel.p : nullptr, release ? S.cand.p : nullptr, release ? S.cstamp.p : nullptr,
             release ? S.lists.p + 2 * n : nullptr,
-            release ? S.comm.p : nullptr, release ? S.hits.p : nullptr, release ? S.hstamp.p : nullptr,
+            release ? S.hits.p : nullptr, release ? S.hstamp.p : nullptr,
             release ? S.cur.p : nullptr, S.stat.p,
             (uint32_t*)S.bits.p, nwords,
             c->g.X, c->g.Y,
@@ -1131,7 +1161,6 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     HIP_OK(hipMemsetAsync(S.cnt.p, 0, sizeof(int) * XYc, st));
     k_cell_fill<<<blocks(n), TPB, 0, st>>>(a, S.cnt.p);
     k_cell_sort<<<blocks(XYc), TPB, 0, st>>>(a, XYc);
-    k_fill_b<<<blocks(n), TPB, 0, st>>>(S.batch.p, n, -1);
     k_start<<<blocks(n), TPB, 0, st>>>(a);
     HIP_OK(hipGetLastError());
     // Lanes per net: about half the average point count, at most 16.
@@ -1140,8 +1169,11 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     const int G = c->tune.sched_group ? c->tune.sched_group : avg <= 6 ? 4 : avg <= 16 ? 8 : 16;
     const int CHUNK = c->tune.sched_chunk ? c->tune.sched_chunk : DEF_SCHED_CHUNK;
     const unsigned ggrid = (unsigned)std::min<int64_t>(2048, blocks(n * G));
-    const unsigned wgrid = 256;   // one wave per viable net
-    const unsigned gm = (unsigned)std::min<int64_t>(2048, blocks(std::max(XYc, n)));   // grid-stride
+    const unsigned vgrid = (unsigned)std::min<int64_t>(512, (n * G + LTPB - 1) / LTPB);
+    // a wave per viable net, as many as a round of this many nets may find
+    const unsigned wgrid = (unsigned)std::min<int64_t>(1024, std::max<int64_t>(16, n / 64));
+    const unsigned cgrid = (wgrid + 3) / 4;
+    const unsigned gm = (unsigned)std::min<int64_t>(512, (std::max(XYc, n) + LTPB - 1) / LTPB);   // grid-stride
     int* h_ctrl = nullptr;
     HIP_OK(hipHostMalloc(&h_ctrl, sizeof(int) * (2 * C_WORDS + 1)));
     const int64_t max_rounds = (int64_t)ROUNDS * (n + 1) + CHUNK;
@@ -1157,50 +1189,28 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
                 progress("scheduler: %d batches after %.1f s", h_ctrl[(g & 1) * C_WORDS + C_CUR],
                          std::chrono::duration<double>(t_now - t_start).count());
             }
-            for (int r = 0; r < CHUNK; r++, g++) {
+            auto round = [&](auto gv) {
+                constexpr int GV = decltype(gv)::value;
                 if (release) {
-                    switch (G) {
-                    case 4:
-                        k_r_claim<4><<<ggrid, TPB, 0, st>>>(a, g);
-                        k_r_viable<4><<<ggrid, TPB, 0, st>>>(a, g, S.viable.p);
-                        break;
-                    case 8:
-                        k_r_claim<8><<<ggrid, TPB, 0, st>>>(a, g);
-                        k_r_viable<8><<<ggrid, TPB, 0, st>>>(a, g, S.viable.p);
-                        break;
-                    default:
-                        k_r_claim<16><<<ggrid, TPB, 0, st>>>(a, g);
-                        k_r_viable<16><<<ggrid, TPB, 0, st>>>(a, g, S.viable.p);
-                        break;
-                    }
+                    k_r_claim<GV><<<vgrid, LTPB, 0, st>>>(a, g);
+                    k_r_viable<GV><<<vgrid, LTPB, 0, st>>>(a, g, S.viable.p);
                     k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
-                    k_r_commit<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
+                    k_r_commit<<<cgrid, LTPB, 0, st>>>(a, g, S.viable.p);
                     k_r_block<64><<<ggrid, TPB, 0, st>>>(a, g);
-                    k_r_clear_end<<<gm, TPB, 0, st>>>(a, g, XYc);
-                } else {
-                    switch (G) {
-                    case 4:
-                        k_a_claim<4><<<ggrid, TPB, 0, st>>>(a, g);
-                        k_a_viable<4><<<ggrid, TPB, 0, st>>>(a, g, S.viable.p);
-                        break;
-                    case 8:
-                        k_a_claim<8><<<ggrid, TPB, 0, st>>>(a, g);
-                        k_a_viable<8><<<ggrid, TPB, 0, st>>>(a, g, S.viable.p);
-                        break;
-                    default:
-                        k_a_claim<16><<<ggrid, TPB, 0, st>>>(a, g);
-                        k_a_viable<16><<<ggrid, TPB, 0, st>>>(a, g, S.viable.p);
-                        break;
-                    }
-                    k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
-                    k_a_commit<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
-                    switch (G) {
-                    case 4: k_a_revert<4><<<ggrid, TPB, 0, st>>>(a, g); break;
-                    case 8: k_a_revert<8><<<ggrid, TPB, 0, st>>>(a, g); break;
-                    default: k_a_revert<16><<<ggrid, TPB, 0, st>>>(a, g); break;
-                    }
-                    k_a_clear_end<<<gm, TPB, 0, st>>>(a, g, XYc);
+                    k_r_clear_end<<<gm, LTPB, 0, st>>>(a, g, XYc);
+                    return;
                 }
+                k_a_claim<GV><<<ggrid, TPB, 0, st>>>(a, g);
+                k_a_viable<GV><<<vgrid, LTPB, 0, st>>>(a, g, S.viable.p);
+                k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
+                k_a_commit<<<cgrid, LTPB, 0, st>>>(a, g, S.viable.p);
+                k_a_revert<GV><<<ggrid, TPB, 0, st>>>(a, g);
+                k_a_clear_end<<<gm, LTPB, 0, st>>>(a, g, XYc);
+            };
+            for (int r = 0; r < CHUNK; r++, g++) {
+                if (G == 4) round(std::integral_constant<int, 4>{});
+                else if (G == 8) round(std::integral_constant<int, 8>{});
+                else round(std::integral_constant<int, 16>{});
             }
             HIP_OK(hipGetLastError());
             HIP_OK(hipMemcpyAsync(h_ctrl, S.ctrl.p, sizeof(int) * (2 * C_WORDS + 1), hipMemcpyDeviceToHost, st));
