@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(1024) k_presum(GridDev g) {
         const int p = p0 + j;
         s[j] = (p >= 1 && p < len) ? (double)(j ? w[j - 1] : before) : 0.0;
     }
-    block_sklansky_rt<double, K, 16>(s, lds, nw);
+    block_sklansky_rt<double, K>(s, lds, nw);
     if constexpr (K % 2 == 0) {
         if ((len & 1) == 0) {
 #pragma unroll
@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(TPB) k_scan_int(GridDev g, int* a) {
         int p = threadIdx.x * K + j;
         s[j] = (p >= 1 && p < len) ? a[base + p - 1] : 0;
     }
-    block_sklansky<int, K, TPB / 64>(s, lds);
+    block_sklansky_rt<int, K>(s, lds, TPB / 64);
 #pragma unroll
     for (int j = 0; j < K; j++) {
         int p = threadIdx.x * K + j;
@@ -375,7 +375,7 @@ __global__ void __launch_bounds__(TPB) k_view_scan(const float* v, float* out, i
         int p = threadIdx.x * K + j;
         s[j] = (p >= 1 && p < len) ? v[base + (int64_t)(p - 1) * stride_pos] : 0.0f;
     }
-    block_sklansky<float, K, TPB / 64>(s, lds);
+    block_sklansky_rt<float, K>(s, lds, TPB / 64);
 #pragma unroll
     for (int j = 0; j < K; j++) {
         int p = threadIdx.x * K + j;

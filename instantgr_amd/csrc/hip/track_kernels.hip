@@ -28,21 +28,54 @@ namespace {
 
 constexpr int SB = 256;   // block size of the scatter and fill kernels
 
-// Value of the first element of the next thread (0 past the last thread).
-template <typename T>
-__device__ __forceinline__ T next_first(T first, T* sh) {
-    __syncthreads();
-    sh[threadIdx.x] = first;
-    __syncthreads();
-    return threadIdx.x + 1 < blockDim.x ? sh[threadIdx.x + 1] : T(0);
+// Inclusive sums of a wave's lanes (integers: any order).
+__device__ __forceinline__ int wave_sum(int v) {
+    v += dpp_move<0x111, 0xf, 0xf>(0, v);
+    v += dpp_move<0x112, 0xf, 0xf>(0, v);
+    v += dpp_move<0x114, 0xf, 0xf>(0, v);
+    v += dpp_move<0x118, 0xf, 0xf>(0, v);
+    v += dpp_move<0x142, 0xa, 0xf>(0, v);
+    v += dpp_move<0x143, 0xc, 0xf>(0, v);
+    return v;
 }
-// Value of the last element of the previous thread (0 for thread 0).
-template <typename T>
-__device__ __forceinline__ T prev_last(T last, T* sh) {
-    __syncthreads();
-    sh[threadIdx.x] = last;
-    __syncthreads();
-    return threadIdx.x > 0 ? sh[threadIdx.x - 1] : T(0);
+__device__ __forceinline__ int row_sum(int v) {
+    v += dpp_move<0x111, 0xf, 0xf>(0, v);
+    v += dpp_move<0x112, 0xf, 0xf>(0, v);
+    v += dpp_move<0x114, 0xf, 0xf>(0, v);
+    v += dpp_move<0x118, 0xf, 0xf>(0, v);
+    return v;
+}
+
+// Inclusive prefix sums of three integer arrays over the workgroup, with one
+// barrier (tot: the waves' totals).
+template <int K>
+__device__ __forceinline__ void block_sums(int (&a)[K], int (&b)[K], int (&c)[K], int4* tot, int nw) {
+#pragma unroll
+    for (int j = 1; j < K; j++) {
+        a[j] += a[j - 1];
+        b[j] += b[j - 1];
+        c[j] += c[j - 1];
+    }
+    const int ta = a[K - 1], tb = b[K - 1], tc = c[K - 1];
+    int pa = wave_sum(ta), pb = wave_sum(tb), pc = wave_sum(tc);
+    if (nw > 1) {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (lane == 63) tot[wave] = make_int4(pa, pb, pc, 0);
+        __syncthreads();
+        const int4 t = (lane & 15) < nw ? tot[lane & 15] : make_int4(0, 0, 0, 0);
+        const int sa = row_sum(t.x), sb = row_sum(t.y), sc = row_sum(t.z);
+        if (wave > 0) {
+            pa += lane_read(sa, wave - 1);
+            pb += lane_read(sb, wave - 1);
+            pc += lane_read(sc, wave - 1);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        a[j] += pa - ta;
+        b[j] += pb - tb;
+        c[j] += pc - tc;
+    }
 }
 
 // K consecutive elements of a track per thread.  With K a multiple of 4 and
@@ -116,58 +149,85 @@ __device__ __forceinline__ void apply_vias(float (&dem)[K], const int (&gv)[K], 
     }
 }
 
-// Wire cost, via cost and the exclusive prefix input (the predecessor's wire
-// cost) of a thread's K cells from their demand and capacity, with pdc the
-// predecessor cell's (demand, capacity).
+// Wire costs, via costs and the exclusive prefix inputs (the predecessor's
+// wire cost) of a thread's K cells from their demand and capacity.  The
+// increments are formed once per cell; those of the cell before the thread's
+// first come from the thread before (sh: one entry per wave, one barrier).
+struct CellCost {
+    double a1, ah;                // increments of one and of half a track
+    float wc;
+};
 template <int K, bool TAB>
-__device__ __forceinline__ void track_costs(const GridDev& g, int l, int dir, int len, int p0, const float (&dem)[K],
-                                            const float (&cap)[K], float2 pdc, const float* tab, float (&wc)[K],
-                                            float (&vc)[K], double (&s)[K]) {
+__device__ __forceinline__ void own_costs(const GridDev& g, int l, int len, int p0, const float (&dem)[K],
+                                          const float (&cap)[K], const int (&el)[K], const float* tab,
+                                          double (&a1)[K], double (&ah)[K], float (&wc)[K]) {
     const double w = g.w[l];
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        inc_pair<TAB>(cap[j], dem[j], w, tab, a1[j], ah[j]);
+        const float x = (float)a1[j];
+        const float y = (float)((double)x + g.unit_wire * (double)el[j]);
+        wc[j] = p0 + j < len - 1 ? y : x;
+    }
+}
+template <int K>
+__device__ __forceinline__ void track_costs(const GridDev& g, int l, int dir, int len, int p0, const float (&dem)[K],
+                                            const float (&cap)[K], const float* tab, CellCost* sh, float (&wc)[K],
+                                            float (&vc)[K], double (&s)[K]) {
     const int* elen = dir ? g.ylen : g.xlen;
-    // edge lengths of the cells p0 - 1 .. p0 + K - 1 (0 from the last cell on)
-    int el[K + 1];
-    el[0] = p0 >= 1 && p0 - 1 < len - 1 ? elen[p0 - 1] : 0;
+    int el[K];                    // edge lengths, 0 from the last cell on
     if (K % 4 == 0 && p0 + K <= len - 1) {
 #pragma unroll
         for (int j = 0; j < K; j += 4) {
             const int4 q = *reinterpret_cast<const int4*>(elen + p0 + j);
-            el[j + 1] = q.x; el[j + 2] = q.y; el[j + 3] = q.z; el[j + 4] = q.w;
+            el[j] = q.x; el[j + 1] = q.y; el[j + 2] = q.z; el[j + 3] = q.w;
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < K; j++) el[j + 1] = p0 + j < len - 1 ? elen[p0 + j] : 0;
+        for (int j = 0; j < K; j++) el[j] = p0 + j < len - 1 ? elen[p0 + j] : 0;
     }
-    auto wire = [&](double a1, int p, int e) {
-        const float x = (float)a1;
-        const float y = (float)((double)x + g.unit_wire * (double)e);
-        return p < len - 1 ? y : x;
-    };
-    double a1p = 0.0, ahp = 0.0;
-    float wcp = 0.0f;
-    if (p0 >= 1 && p0 - 1 < len) {
-        inc_pair<TAB>(pdc.y, pdc.x, w, tab, a1p, ahp);
-        wcp = wire(a1p, p0 - 1, el[0]);
+    bool q = true;
+#pragma unroll
+    for (int j = 0; j < K; j++) q = q && quarter_grid(cap[j], dem[j]);
+    double a1[K], ah[K];
+    // the exponents come from the table when every element of the wave allows
+    // it, else they are computed; the values are the same either way
+    if (__all(q)) own_costs<K, true>(g, l, len, p0, dem, cap, el, tab, a1, ah, wc);
+    else own_costs<K, false>(g, l, len, p0, dem, cap, el, tab, a1, ah, wc);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 63) sh[wave] = CellCost{a1[K - 1], ah[K - 1], wc[K - 1]};
+    __syncthreads();
+    double a1p = __shfl_up(a1[K - 1], 1), ahp = __shfl_up(ah[K - 1], 1);
+    float wcp = __shfl_up(wc[K - 1], 1);
+    if (lane == 0 && wave > 0) {
+        const CellCost c = sh[wave - 1];
+        a1p = c.a1;
+        ahp = c.ah;
+        wcp = c.wc;
     }
 #pragma unroll
     for (int j = 0; j < K; j++) {
         const int p = p0 + j;
-        if (p >= len) { wc[j] = vc[j] = 0.0f; s[j] = 0.0; continue; }
-        double a1, ah;
-        inc_pair<TAB>(cap[j], dem[j], w, tab, a1, ah);
-        wc[j] = wire(a1, p, el[j + 1]);
         float v;
-        if (p == 0) v = (float)a1;
+        if (p == 0) v = (float)a1[j];
         else if (p == len - 1) v = (float)a1p;
-        else v = (float)(ah + ahp);
-        vc[j] = (float)((double)v + g.unit_via);
-        s[j] = p >= 1 ? (double)wcp : 0.0;   // exclusive prefix input
-        a1p = a1;
-        ahp = ah;
+        else v = (float)(ah[j] + ahp);
+        const bool in = p < len;
+        vc[j] = in ? (float)((double)v + g.unit_via) : 0.0f;
+        s[j] = in && p >= 1 ? (double)wcp : 0.0;   // exclusive prefix input
+        a1p = a1[j];
+        ahp = ah[j];
         wcp = wc[j];
     }
 }
 
+// Bound by the loads and stores of its ten arrays (52 bytes a cell where both
+// stamps are set); every load is issued before the first use, the three integer
+// scans share one barrier, and the whole update takes four.  800x800x9, every
+// track dirty: 48 us a launch (54 us at the copy rate for all arrays); with a
+// scan each, fourteen barriers and two counter atomics a track on shared
+// addresses, 128 us.  Cost and prefix sums alone, 2500x2500x11: 429 us (542).
+//
 // s_c: commit stamp (0 = nothing to commit); s_r: rip-up stamp (0 = no
 // rip-up); cost: recompute costs and prefix sums (and clear the dirty flag).
 // stats[0] += cells of the tracks processed, stats[1] += those with rip-up.
@@ -178,9 +238,9 @@ __global__ void __launch_bounds__(1024) k_track_fused(GridDev g, int s_c, int s_
                                                       unsigned long long* stats) {
     constexpr int NWMAX = 16;
     const int nw = blockDim.x >> 6;
-    __shared__ int sh_i[NWMAX * 64];
-    __shared__ float2 sh_f2[NWMAX * 64];
-    __shared__ int lds_i[NWMAX];
+    __shared__ int4 sh_tot[NWMAX];
+    __shared__ int2 sh_via[NWMAX];
+    __shared__ CellCost sh_c[NWMAX];
     __shared__ double lds_d[NWMAX];
     __shared__ float s_exp[EXPTAB_N];
     int t = blockIdx.x;
@@ -194,68 +254,65 @@ __global__ void __launch_bounds__(1024) k_track_fused(GridDev g, int s_c, int s_
     const bool v4 = (len & 3) == 0;
     const int p0 = threadIdx.x * K;
     float dem[K], cap[K];
-    int ts[K];
+    int ts[K], inc[K], gv[K], dec[K], cov[K], gr[K];
     uint32_t wr_dem = 0, wr_ts = 0, clr = 0;   // per-element bit masks
+    // every load before the first use
     load_k<K, float, float4>(g.demand, base, p0, len, v4, dem);
     load_k<K, float, float4>(g.cap, base, p0, len, v4, cap);
-    if (s_c || s_r) load_k<K, int, int4>(g.ts, base, p0, len, v4, ts);
-    else
-#pragma unroll
-        for (int j = 0; j < K; j++) ts[j] = 0;
+    load_k<K, int, int4>(g.ts, base, p0, len, v4, ts);
     if (s_c) {
-        int inc[K], gv[K];
         load_k<K, int, int4>(g.pre, base, p0, len, v4, inc);
         load_k<K, int, int4>(g.vc, base, p0, len, v4, gv);
+    } else {
 #pragma unroll
-        for (int j = 0; j < K; j++)
-            if (inc[j] | gv[j]) clr |= 1u << j;
-        block_sklansky_rt<int, K, NWMAX>(inc, lds_i, nw);
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            const int p = threadIdx.x * K + j;
-            if (p <= len - 2 && inc[j] > 0) {
-                dem[j] += (float)inc[j];
-                wr_dem |= 1u << j;
-                if (ts[j] != s_c) { ts[j] = s_c; wr_ts |= 1u << j; }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            if (ts[j] >= s_c) gv[j] = 0;
-            if (gv[j]) wr_dem |= (3u << j) >> 1;  // edges j-1 and j of this thread
-        }
-        const int gn = next_first<int>(gv[0], sh_i);
-        if (gn) wr_dem |= 1u << (K - 1);
-        apply_vias<K>(dem, gv, gn, len, 1.0f);
+        for (int j = 0; j < K; j++) inc[j] = gv[j] = 0;
     }
     if (s_r) {
-        int dec[K], cov[K], gr[K];
         load_k<K, int, int4>(g.rpre, base, p0, len, v4, dec);
         load_k<K, int, int4>(g.rcov, base, p0, len, v4, cov);
         load_k<K, int, int4>(g.rvc, base, p0, len, v4, gr);
+    } else {
 #pragma unroll
-        for (int j = 0; j < K; j++)
-            if (dec[j] | cov[j] | gr[j]) clr |= 1u << j;
-        block_sklansky_rt<int, K, NWMAX>(dec, lds_i, nw);
-        block_sklansky_rt<int, K, NWMAX>(cov, lds_i, nw);
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            const int p = threadIdx.x * K + j;
-            if (p <= len - 2 && dec[j] > 0) { dem[j] -= (float)dec[j]; wr_dem |= 1u << j; }
-            if (p < len && cov[j] > 0 && ts[j] != s_r) { ts[j] = s_r; wr_ts |= 1u << j; }
-        }
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            if (ts[j] >= s_r) gr[j] = 0;
-            if (gr[j]) wr_dem |= (3u << j) >> 1;
-        }
-        const int gn = next_first<int>(gr[0], sh_i);
-        if (gn) wr_dem |= 1u << (K - 1);
-        apply_vias<K>(dem, gr, gn, len, -1.0f);
+        for (int j = 0; j < K; j++) dec[j] = cov[j] = gr[j] = 0;
     }
+    if (cost)
+        for (int i = threadIdx.x; i < EXPTAB_N; i += blockDim.x) s_exp[i] = g.exptab[i];
+#pragma unroll
+    for (int j = 0; j < K; j++)
+        if (inc[j] | gv[j] | dec[j] | cov[j] | gr[j]) clr |= 1u << j;
+    block_sums<K>(inc, dec, cov, sh_tot, nw);
+    // commit of the wires, gate of the vias (s_c), then the rip-up's (s_r):
+    // the demand changes are integers and halves, so their order is free, but
+    // the timestamps gate in sequence
 #pragma unroll
     for (int j = 0; j < K; j++) {
-        const int p = threadIdx.x * K + j;
+        const int p = p0 + j;
+        if (p <= len - 2 && inc[j] > 0) {
+            dem[j] += (float)inc[j];
+            wr_dem |= 1u << j;
+            if (ts[j] != s_c) { ts[j] = s_c; wr_ts |= 1u << j; }
+        }
+        if (ts[j] >= s_c) gv[j] = 0;
+        if (p <= len - 2 && dec[j] > 0) { dem[j] -= (float)dec[j]; wr_dem |= 1u << j; }
+        if (p < len && cov[j] > 0 && ts[j] != s_r) { ts[j] = s_r; wr_ts |= 1u << j; }
+        if (ts[j] >= s_r) gr[j] = 0;
+        if (gv[j] | gr[j]) wr_dem |= (3u << j) >> 1;   // edges j-1 and j of this thread
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) sh_via[wave] = make_int2(gv[0], gr[0]);
+    __syncthreads();
+    int gvn = __shfl_down(gv[0], 1), grn = __shfl_down(gr[0], 1);
+    if (lane == 63) {
+        const int2 v = wave + 1 < nw ? sh_via[wave + 1] : make_int2(0, 0);
+        gvn = v.x;
+        grn = v.y;
+    }
+    if (gvn | grn) wr_dem |= 1u << (K - 1);
+    apply_vias<K>(dem, gv, gvn, len, 1.0f);
+    apply_vias<K>(dem, gr, grn, len, -1.0f);
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        const int p = p0 + j;
         if (p >= len) continue;
         if (wr_dem >> j & 1) g.demand[base + p] = dem[j];
         if (wr_ts >> j & 1) g.ts[base + p] = ts[j];
@@ -264,33 +321,19 @@ __global__ void __launch_bounds__(1024) k_track_fused(GridDev g, int s_c, int s_
             if (s_r) { g.rpre[base + p] = 0; g.rcov[base + p] = 0; g.rvc[base + p] = 0; }
         }
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && stats) {
         atomicAdd(&stats[0], (unsigned long long)len);
         if (s_r) atomicAdd(&stats[1], (unsigned long long)len);
     }
     if (!cost) return;
-    // Costs from the new demand (src/graph.hpp:40-71).
-    // Per element the increments of one and of half a track (inc_pair, the
-    // shared f(d) term); the via cost takes the element's and its
-    // predecessor's, the prefix input is the predecessor's wire cost.  The
-    // predecessor of a thread's first element is recomputed from the previous
-    // thread's last demand and capacity (one exchange, whose barriers also
-    // publish the LDS exp table).  The exponents come from the table when
-    // every element of the wave allows it, else they are computed; the
-    // values are the same either way.
-    for (int i = threadIdx.x; i < EXPTAB_N; i += blockDim.x) s_exp[i] = g.exptab[i];
-    const float2 pdc = prev_last(make_float2(dem[K - 1], cap[K - 1]), sh_f2);
+    // Costs from the new demand (src/graph.hpp:40-71), then the exclusive FP64
+    // Sklansky prefix of wcost (src/graph.hpp:405-430).
     float wc[K], vc[K];
     double s[K];
-    bool q = quarter_grid(pdc.y, pdc.x);
-#pragma unroll
-    for (int j = 0; j < K; j++) q = q && quarter_grid(cap[j], dem[j]);
-    if (__all(q)) track_costs<K, true>(g, l, dir, len, p0, dem, cap, pdc, s_exp, wc, vc, s);
-    else track_costs<K, false>(g, l, dir, len, p0, dem, cap, pdc, s_exp, wc, vc, s);
+    track_costs<K>(g, l, dir, len, p0, dem, cap, s_exp, sh_c, wc, vc, s);
     store_k<K>(g.wcost, base, p0, len, v4, wc);
     store_k<K>(g.vcost, base, p0, len, v4, vc);
-    // Exclusive FP64 Sklansky prefix of wcost (src/graph.hpp:405-430).
-    block_sklansky_rt<double, K, NWMAX>(s, lds_d, nw);
+    block_sklansky_rt<double, K>(s, lds_d, nw);
     store_k<K>(g.presum, base, p0, len, v4, s);
     if (threadIdx.x == 0) g.dirty[blockIdx.x] = 0;
 }
@@ -306,10 +349,11 @@ template <int K>
 __global__ void __launch_bounds__(1024) k_track_cost(GridDev g, unsigned long long* stats) {
     constexpr int NWMAX = 16;
     const int nw = blockDim.x >> 6;
-    __shared__ float2 sh_f2[NWMAX * 64];
-    __shared__ double lds_d[NWMAX];
+    __shared__ CellCost sh_c[2][NWMAX];
+    __shared__ double lds_d[2][NWMAX];
     __shared__ float s_exp[EXPTAB_N];
     for (int i = threadIdx.x; i < EXPTAB_N; i += blockDim.x) s_exp[i] = g.exptab[i];
+    __syncthreads();
     const int T = g.tbase[g.L];
     const int p0 = threadIdx.x * K;
     auto next_dirty = [&](int t) {
@@ -322,7 +366,7 @@ __global__ void __launch_bounds__(1024) k_track_cost(GridDev g, unsigned long lo
         len = layer_dir(l, g.DIR) ? g.Y : g.X;
         base = (int64_t)l * g.XYc + (int64_t)(t - g.tbase[l]) * len;
     };
-    int t = next_dirty((int)blockIdx.x);
+    int t = next_dirty((int)blockIdx.x), par = 0;
     float dem[K], cap[K];
     int l = 0, len = 0;
     int64_t base = 0;
@@ -343,21 +387,19 @@ __global__ void __launch_bounds__(1024) k_track_cost(GridDev g, unsigned long lo
             load_k<K, float, float4>(g.cap, basen, p0, lenn, (lenn & 3) == 0, capn);
         }
         const bool v4 = (len & 3) == 0;
-        const float2 pdc = prev_last(make_float2(dem[K - 1], cap[K - 1]), sh_f2);
         float wc[K], vc[K];
         double sv[K];
-        bool q = quarter_grid(pdc.y, pdc.x);
-#pragma unroll
-        for (int j = 0; j < K; j++) q = q && quarter_grid(cap[j], dem[j]);
-        if (__all(q)) track_costs<K, true>(g, l, layer_dir(l, g.DIR), len, p0, dem, cap, pdc, s_exp, wc, vc, sv);
-        else track_costs<K, false>(g, l, layer_dir(l, g.DIR), len, p0, dem, cap, pdc, s_exp, wc, vc, sv);
+        // the exchanges alternate between two sets of entries: the next
+        // track's first write comes after this track's barriers
+        track_costs<K>(g, l, layer_dir(l, g.DIR), len, p0, dem, cap, s_exp, sh_c[par], wc, vc, sv);
         store_k<K>(g.wcost, base, p0, len, v4, wc);
         store_k<K>(g.vcost, base, p0, len, v4, vc);
-        block_sklansky_rt<double, K, NWMAX>(sv, lds_d, nw);
+        block_sklansky_rt<double, K>(sv, lds_d[par], nw);
         store_k<K>(g.presum, base, p0, len, v4, sv);
+        par ^= 1;
         if (threadIdx.x == 0) {
             g.dirty[t] = 0;
-            atomicAdd(&stats[0], (unsigned long long)len);
+            if (stats) atomicAdd(&stats[0], (unsigned long long)len);
         }
         t = tn;
         l = ln;
@@ -470,7 +512,9 @@ void launch_track_fused(igr_ctx* c, int s_commit, int s_rip, bool cost) {
     const int T = c->g.tbase[c->g.L];
     const int ml = std::max(c->g.X, c->g.Y);
     const int cs = cost ? 1 : 0;
-    unsigned long long* st = c->track_stats.p;
+    // the processed-cell counters serve the byte counts of kernel timing only:
+    // two atomics a workgroup on two addresses otherwise
+    unsigned long long* st = c->prof.on ? c->track_stats.p : nullptr;
     hipStream_t s = c->stream;
     // Elements per thread: tuned, or 4 up to 4096-cell tracks and 8 above
     // (4 measured fastest on 800-, 1500- and 2500-cell tracks); the workgroup
