@@ -301,10 +301,6 @@ constexpr int DEF_DAG_ORDER = 1;
 constexpr int DEF_DAG_WAVES = 4;
 constexpr int DEF_DAG_SEQ = 16;
 constexpr int DEF_DAG_GRID = 2048;
-// Batched scheduler: release-driven rounds from this many scheduled nets,
-// active-list rounds below.
-constexpr int64_t DEF_SCHED_RELEASE_NETS = 1500000;
-
 // Records the work enqueued on a stream between construction and launch()
 // as one graph, then launches it; inactive, the work runs as it is enqueued.
 // A capture still open when the scope unwinds is ended and dropped.

@@ -57,6 +57,13 @@ constexpr int TPB = 256;
 // (46), released-cell claims 22 (28).
 constexpr int LTPB = 1024;
 constexpr int ROUNDS = 30;        // rounds per batch (src/database_cuda.hpp:612)
+// Release-driven rounds where the cells' lists hold this many nets on average
+// and the nets are this many, active-list rounds elsewhere.  Scheduler time of
+// the active-list rounds against the release-driven ones, by (nets, list
+// length): (24k, 26) 41 / 55 ms, (125k, 20) 268 / 283, (137k, 51) 140 / 141,
+// (199k, 70) 521 / 473, (321k, 29) 429 / 395, (561k, 34) 282 / 263, (1.59M, 16)
+// 111 / 125, (3.0M, 30) 293 / 281.
+constexpr int64_t SCHED_RELEASE_NETS = 150000, SCHED_RELEASE_LIST = 25;
 
 // control state words (two slots of C_WORDS, then the placed-net counter).
 // C_NU / C_UL: length and buffer of the nets round 0 tests.  Active-list
@@ -72,20 +79,24 @@ enum { C_DONE = 0, C_CUR, C_ROUND, C_COMMIT, C_HAVE, C_NVIABLE, C_NU, C_UL, C_NA
 constexpr int NLISTS = 3;         // net list buffers of n entries each
 constexpr int COMPACT_DIV = 64;   // release-driven rounds: compact the cell lists every n/64 placed nets
 
-// A net by scheduler index: its points, and its net id for the segments.  One
-// load where the index, the row and two offsets were a chain of three.
+// A net by scheduler index: its points.  One load where the index, the row and
+// two offsets were a chain of three.
 struct alignas(16) SNet {
     int64_t pt0;
-    int npt, net;
+    int npt, pad;
+};
+// Its segments, read beside it by the kernels that walk a net's rest cells.
+struct alignas(8) SSeg {
+    int64_t h0, v0;
+    int nh, nv;
 };
 
 struct BArgs {
     int64_t n;
     const SNet* sn;
+    const SSeg* sg;
     const int* pt;
-    const int64_t* hs_off;
     const int* hs;
-    const int64_t* vs_off;
     const int* vs;
     int* map;                     // X*Y owner or -1
     int* base;                    // X*Y highest unassigned net listing the cell, or -1
@@ -170,11 +181,11 @@ __device__ __forceinline__ const int* r_list(const BArgs& a, const int* st, int6
 __device__ __forceinline__ bool active(const BArgs& a, int64_t i) { return nstate(a, i) == 0; }
 
 // ---- per-cell lists -------------------------------------------------------
-__global__ void k_cell_count(BArgs a, int* cnt) {
+__global__ void k_cell_count(int64_t n, const SNet* sn, const int* pt, int* cnt) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i >= a.n) return;
-    const SNet s = a.sn[i];
-    for (int64_t k = s.pt0; k < s.pt0 + s.npt; k++) atomicAdd(&cnt[a.pt[k]], 1);
+    if (i >= n) return;
+    const SNet s = sn[i];
+    for (int64_t k = s.pt0; k < s.pt0 + s.npt; k++) atomicAdd(&cnt[pt[k]], 1);
 }
 
 __global__ void k_cell_fill(BArgs a, int* fillc) {
@@ -353,6 +364,33 @@ struct GroupList {
             else list[atomicAdd(counter, 1)] = v;
         }
     }
+    // U candidates a lane with one counter update.
+    template <int U>
+    __device__ __forceinline__ void add(const bool (&want)[U], const int (&v)[U]) {
+        uint64_t m[U];
+        int total = 0;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            m[u] = __ballot(want[u]);
+            total += __popcll(m[u]);
+        }
+        if (total == 0) return;
+        const int lane = threadIdx.x & 63;
+        const uint64_t here = __ballot(true);
+        const int leader = __builtin_ctzll(here);
+        int off = 0;
+        if (lane == leader) off = atomicAdd(&hdr[0], total);
+        off = __shfl(off, leader);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int pos = off + __popcll(m[u] & ((1ull << lane) - 1));
+            if (want[u]) {
+                if (pos < GL_CAP) buf[pos] = v[u];
+                else list[atomicAdd(counter, 1)] = v[u];
+            }
+            off += __popcll(m[u]);
+        }
+    }
     __device__ __forceinline__ void flush() {
         __syncthreads();
         const int nb = hdr[0] < GL_CAP ? hdr[0] : GL_CAP;
@@ -362,24 +400,23 @@ struct GroupList {
     }
 };
 
-// Calls f(valid, q) for the sampled cells q of a net's segments (every
-// sparsity-th cell from each segment's start, src/database_cuda.hpp:320-352),
-// the cells of up to 64 segments at a time spread evenly over the wave's
-// lanes (a lane per segment would walk a long segment alone).  Every lane of
-// the wave calls it together; f sees valid = false on the lanes past the last
-// cell and may use ballots.
-template <class F>
-__device__ __forceinline__ void wave_segment_cells(const BArgs& a, int net, F f) {
+// Calls f(valid, q) with U cells per lane at a time, over the sampled cells of
+// a net's segments (every sparsity-th cell from each segment's start,
+// src/database_cuda.hpp:320-352), the cells of up to 64 segments at a time
+// spread evenly over the wave's lanes (a lane per segment would walk a long
+// segment alone).  Every lane of the wave calls it together; valid is false on
+// the lanes past the last cell, and f may use ballots.
+template <int U, class F>
+__device__ __forceinline__ void wave_segment_cells(const BArgs& a, const SSeg& g, F f) {
     const int lane = threadIdx.x & 63;
     const int Y = a.Y, sp = a.sparsity;
-    const int64_t h0 = a.hs_off[net], v0 = a.vs_off[net];
-    const int nh = (int)(a.hs_off[net + 1] - h0), ns = nh + (int)(a.vs_off[net + 1] - v0);
+    const int ns = g.nh + g.nv;
     for (int sb = 0; sb < ns; sb += 64) {
         const int k = sb + lane;
         int cnt = 0, first = 0, step = 0;
         if (k < ns) {
-            const bool hor = k < nh;
-            const int* seg = hor ? a.hs + 2 * (h0 + k) : a.vs + 2 * (v0 + k - nh);
+            const bool hor = k < g.nh;
+            const int* seg = hor ? a.hs + 2 * (g.h0 + k) : a.vs + 2 * (g.v0 + k - g.nh);
             const int b = seg[0], e = seg[1];
             const int bx = b / Y, by = b - bx * Y, ex = e / Y, ey = e - ex * Y;
             const int span = hor ? ex - bx : ey - by;   // along x at y = by, or along y at x = bx
@@ -394,32 +431,33 @@ __device__ __forceinline__ void wave_segment_cells(const BArgs& a, int net, F f)
         }
         const int total = __shfl(incl, 63);
         const int excl = incl - cnt;
-        for (int cb = 0; cb < total; cb += 64) {
-            const int c = cb + lane;
-            int sg = 0;                  // the first lane whose inclusive count exceeds c
-            for (int b2 = 32; b2 > 0; b2 >>= 1)
-                if (__shfl(incl, sg + b2 - 1) <= c) sg += b2;
-            const int f0 = __shfl(first, sg), st0 = __shfl(step, sg), ex = __shfl(excl, sg);
-            const bool valid = c < total;
-            f(valid, valid ? f0 + (c - ex) * st0 : 0);
+        for (int cb = 0; cb < total; cb += 64 * U) {
+            bool valid[U];
+            int q[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int c = cb + 64 * u + lane;
+                int sg = 0;              // the first lane whose inclusive count exceeds c
+                for (int b2 = 32; b2 > 0; b2 >>= 1)
+                    if (__shfl(incl, sg + b2 - 1) <= c) sg += b2;
+                const int f0 = __shfl(first, sg), st0 = __shfl(step, sg), ex = __shfl(excl, sg);
+                valid[u] = c < total;
+                q[u] = valid[u] ? f0 + (c - ex) * st0 : 0;
+            }
+            f(valid, q);
         }
     }
 }
 
-// Calls f(valid, q) for the rest cells of a net: the neighbour cells (0,-1),
-// (-1,0), (1,0) of its points and its sampled segment cells.
-template <class F>
-__device__ __forceinline__ void wave_rest_cells(const BArgs& a, const SNet& s, F f) {
-    const int lane = threadIdx.x & 63;
-    const int X = a.X, Y = a.Y;
-    for (int k = lane; k - lane < s.npt; k += 64) {
-        const bool in = k < s.npt;
-        const int p = in ? a.pt[s.pt0 + k] : 0, x = p / Y, y = p - x * Y;
-        f(in && y > 0, p - 1);
-        f(in && x > 0, p - Y);
-        f(in && x + 1 < X, p + Y);
-    }
-    wave_segment_cells(a, s.net, f);
+// The neighbour cells (0,-1), (-1,0), (1,0) of a point.
+__device__ __forceinline__ void point_neighbours(const BArgs& a, bool in, int p, bool (&valid)[3], int (&q)[3]) {
+    const int x = p / a.Y, y = p - x * a.Y;
+    valid[0] = in && y > 0;
+    valid[1] = in && x > 0;
+    valid[2] = in && x + 1 < a.X;
+    q[0] = p - 1;
+    q[1] = p - a.Y;
+    q[2] = p + a.Y;
 }
 
 // 3. (both) a wave per viable net claims the neighbour cells (0,-1), (-1,0),
@@ -431,10 +469,23 @@ __global__ void __launch_bounds__(TPB) k_b_claim_rest(BArgs a, int64_t g, const 
     unsigned long long nb = 0;
     for (int w = (threadIdx.x >> 6) * gridDim.x + blockIdx.x; w < nv; w += (gridDim.x * TPB) >> 6) {
         const int i = vlist[w];
-        if ((threadIdx.x & 63) == 0) nb += 4 + 16 + 32;   // list entry, net record, segment offsets
-        wave_rest_cells(a, a.sn[i], [&](bool valid, int q) {
-            if (valid) {
-                atomicMax(&a.map[q], i);
+        const SNet s = a.sn[i];
+        const SSeg sg = a.sg[i];
+        const int lane = threadIdx.x & 63;
+        if (lane == 0) nb += 4 + 16 + 24;   // list entry, net and segment records
+        for (int k = lane; k < s.npt; k += 64) {
+            bool valid[3];
+            int q[3];
+            point_neighbours(a, true, a.pt[s.pt0 + k], valid, q);
+            for (int u = 0; u < 3; u++)
+                if (valid[u]) {
+                    atomicMax(&a.map[q[u]], i);
+                    nb += 4;
+                }
+        }
+        wave_segment_cells<1>(a, sg, [&](bool(&valid)[1], int(&q)[1]) {
+            if (valid[0]) {
+                atomicMax(&a.map[q[0]], i);
                 nb += 4;
             }
         });
@@ -463,8 +514,7 @@ __global__ void __launch_bounds__(TPB) k_a_claim(BArgs a, int64_t g) {
     const int lg = threadIdx.x & (G - 1);
     for (int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G; t < na; t += nth) {
         const int64_t i = al[t];
-        if (!active(a, i)) continue;
-        const SNet s = a.sn[i];
+        const SNet s = a.sn[i];   // every listed net is active
         for (int k = lg; k < s.npt; k += G) {
             int* m = &a.map[a.pt[s.pt0 + k]];
             if (*m < (int)i) atomicMax(m, (int)i);
@@ -494,7 +544,7 @@ __global__ void __launch_bounds__(LTPB) k_a_viable(BArgs a, int64_t g, int* vlis
     for (int64_t r = 0; r < rounds; r++) {
         const int64_t t = ((int64_t)blockIdx.x * LTPB + threadIdx.x) / G + r * nth;
         const int64_t i = t < na ? al[t] : 0;
-        const bool live = t < na && active(a, i);
+        const bool live = t < na;   // every listed net is active
         const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
         bool fail = !live;
         for (int k = lg;; k += G) {
@@ -545,8 +595,9 @@ __global__ void __launch_bounds__(TPB) k_a_revert(BArgs a, int64_t g) {
     for (int64_t r = 0; r < rounds; r++) {
         const int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G + r * nth;
         const int64_t i = t < na ? al[t] : 0;
-        const bool live = t < na && active(a, i);
-        const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
+        SNet s = t < na ? a.sn[i] : SNet{0, 0, 0};
+        const bool live = t < na && !assigned(a, i);
+        if (!live) s.npt = 0;
         bool hit = false;
         for (int k = lg;; k += G) {
             bool h = false;
@@ -753,8 +804,9 @@ __global__ void __launch_bounds__(LTPB) k_r_viable(BArgs a, int64_t g, int* vlis
         const int64_t t = ((int64_t)blockIdx.x * LTPB + threadIdx.x) / G + r * nth;
         const int64_t i = t < na ? al[t] : 0;
         const bool live = t < na && active(a, i);
-        if (t < na && lg == 0) nb += 4 + 4 + (live ? 16 : 0);   // entry, state, net record
-        const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
+        if (t < na && lg == 0) nb += 4 + 4 + 16;   // entry, state, net record
+        SNet s = t < na ? a.sn[i] : SNet{0, 0, 0};   // beside the state word, not after it
+        if (!live) s.npt = 0;
         bool fail = !live;
         for (int k = lg;; k += G) {
             const bool chk = !fail && k < s.npt;
@@ -768,6 +820,18 @@ __global__ void __launch_bounds__(LTPB) k_r_viable(BArgs a, int64_t g, int* vlis
     }
     gl.flush();
     flush_bytes(a, nb);
+}
+
+// Lists the cells not yet listed in the round of this stamp.
+template <int U>
+__device__ __forceinline__ void hit(const BArgs& a, GroupList& gl, int stamp, const bool (&own)[U], const int (&q)[U],
+                                    unsigned long long& nb) {
+    bool h[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) h[u] = own[u] && atomicExch(&a.hstamp[q[u]], stamp) != stamp;
+#pragma unroll
+    for (int u = 0; u < U; u++) nb += (own[u] ? 8 : 0) + (h[u] ? 4 : 0);   // stamp, hit entry
+    gl.add(h, q);
 }
 
 // 4. a wave per viable net: commit it if it still owns every point cell;
@@ -789,9 +853,10 @@ __global__ void __launch_bounds__(LTPB) k_r_commit(BArgs a, int64_t g, const int
     for (int w = (threadIdx.x >> 6) * gridDim.x + blockIdx.x; w < nv; w += (gridDim.x * LTPB) >> 6) {
         const int i = vlist[w];
         const SNet s = a.sn[i];
+        const SSeg sg = a.sg[i];
         // round 0's viable nets: the batch end lists those still unassigned
         if (lane == 0 && st[C_ROUND] == 0) a.v0[w] = i;
-        if (lane == 0) nb += 4 + 16 + 32;   // list entry, net record, segment offsets
+        if (lane == 0) nb += 4 + 16 + 24;   // list entry, net and segment records
         bool lost = false;
         for (int k = lane; k < s.npt; k += 64) {
             lost = lost || a.map[a.pt[s.pt0 + k]] != i;
@@ -804,18 +869,29 @@ __global__ void __launch_bounds__(LTPB) k_r_commit(BArgs a, int64_t g, const int
             atomicAdd(&s_won, 1);
             nb += 8;   // batch, state word
         }
-        auto hit = [&](bool own, int q) {
-            const bool h = own && atomicExch(&a.hstamp[q], stamp) != stamp;
-            nb += (own ? 8 : 0) + (h ? 4 : 0);   // stamp, hit entry
-            gl.add(h, q);
-        };
+        // several cells a lane at a time: their map loads, then their stamp
+        // exchanges, overlap
         for (int k = lane; k - lane < s.npt; k += 64) {
             const bool in = k < s.npt;
-            hit(in, in ? a.pt[s.pt0 + k] : 0);
+            const int p = in ? a.pt[s.pt0 + k] : 0;
+            bool valid[3], own[4];
+            int nq[3], q[4];
+            point_neighbours(a, in, p, valid, nq);
+            own[3] = in;
+            q[3] = p;
+#pragma unroll
+            for (int u = 0; u < 3; u++) {
+                q[u] = nq[u];
+                own[u] = valid[u] && a.map[nq[u]] == i;
+            }
+            hit<4>(a, gl, stamp, own, q, nb);
         }
-        wave_rest_cells(a, s, [&](bool valid, int q) {
-            if (valid) nb += 4;
-            hit(valid && a.map[q] == i, q);
+        wave_segment_cells<2>(a, sg, [&](bool(&valid)[2], int(&q)[2]) {
+            bool own[2];
+#pragma unroll
+            for (int u = 0; u < 2; u++) own[u] = valid[u] && a.map[q[u]] == i;
+            nb += 4 * (valid[0] + valid[1]);
+            hit<2>(a, gl, stamp, own, q, nb);
         });
     }
     gl.flush();
@@ -1056,13 +1132,16 @@ __global__ void __launch_bounds__(LTPB) k_r_clear_end(BArgs a, int64_t g, int64_
 
 // Net records.  Scheduler index i is entry n - 1 - i of the order (its net
 // 'order' and, where the points come per entry, its row of the point arrays).
-__global__ void k_nets(int64_t n, const int* order, const int64_t* pt_off, bool by_entry, SNet* sn) {
+__global__ void k_nets(int64_t n, const int* order, const int64_t* pt_off, bool by_entry, const int64_t* hs_off,
+                       const int64_t* vs_off, SNet* sn, SSeg* sg) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i >= n) return;
     const int net = order[n - 1 - i];
     const int64_t row = by_entry ? n - 1 - i : net;
     const int64_t p0 = pt_off[row];
-    sn[i] = SNet{p0, (int)(pt_off[row + 1] - p0), net};
+    sn[i] = SNet{p0, (int)(pt_off[row + 1] - p0), 0};
+    const int64_t h0 = hs_off[net], v0 = vs_off[net];
+    sg[i] = SSeg{h0, v0, (int)(hs_off[net + 1] - h0), (int)(vs_off[net + 1] - v0)};
 }
 
 // Start state: every net unassigned and active, listed in buffer 0.
@@ -1093,9 +1172,11 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     NetsDev& N = c->nets;
     hipStream_t st = c->stream;
     S.ids.upload(h_order, n, st);
-    S.sn.alloc(16 * (size_t)n);
+    S.sn.alloc((sizeof(SNet) + sizeof(SSeg)) * (size_t)n);
     SNet* sn = reinterpret_cast<SNet*>(S.sn.p);
-    k_nets<<<blocks(n), TPB, 0, st>>>(n, S.ids.p, d_pt_off ? d_pt_off : N.pt_off.p, d_pt_off != nullptr, sn);
+    SSeg* sg = reinterpret_cast<SSeg*>(sn + n);
+    k_nets<<<blocks(n), TPB, 0, st>>>(n, S.ids.p, d_pt_off ? d_pt_off : N.pt_off.p, d_pt_off != nullptr, N.hs_off.p,
+                                      N.vs_off.p, sn, sg);
     HIP_OK(hipGetLastError());
     const int64_t XYc = (int64_t)c->g.X * c->g.Y;
     S.map.alloc(XYc);
@@ -1107,8 +1188,24 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     S.batch.alloc(n);
     S.viable.alloc(n);
     S.lists.alloc(NLISTS * n);
-    // Release-driven rounds from this many nets (active-list rounds below).
-    const bool release = c->tune.sched_kind ? c->tune.sched_kind == 2 : n >= DEF_SCHED_RELEASE_NETS;
+    S.stat.zero(3, st);
+    S.ctrl.zero(2 * C_WORDS + 1, st);
+    const int64_t nwords = (n + 15) / 16;
+    S.bits.zero(nwords, st);
+    // Per-cell lists of the nets' point cells, highest priority first.
+    k_cell_count<<<blocks(n), TPB, 0, st>>>(n, sn, d_pt_off ? d_pt : N.pt.p, S.cnt.p);
+    const int64_t nb = (XYc + SCAN_BLOCK - 1) / SCAN_BLOCK;
+    S.bsum.alloc(nb);
+    k_scan_reduce<<<(unsigned)nb, TPB, 0, st>>>(S.cnt.p, XYc, S.bsum.p);
+    k_scan_bsums<<<1, TPB, 0, st>>>(S.bsum.p, nb);
+    k_scan_apply<<<(unsigned)nb, TPB, 0, st>>>(S.cnt.p, XYc, S.bsum.p, S.c_off.p);
+    HIP_OK(hipGetLastError());
+    int64_t entries = 0;
+    HIP_OK(hipMemcpyAsync(&entries, S.c_off.p + XYc, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    HIP_OK(hipStreamSynchronize(st));
+    S.c_net.alloc(std::max<int64_t>(1, entries));
+    const bool release = c->tune.sched_kind ? c->tune.sched_kind == 2
+                                            : n >= SCHED_RELEASE_NETS && entries >= SCHED_RELEASE_LIST * XYc;
     if (release) {
         S.rel.alloc(XYc);
         S.cand.alloc(n);
@@ -1117,12 +1214,7 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         S.hstamp.zero(XYc, st);
         S.cur.alloc(XYc);
     }
-    S.stat.zero(3, st);
-    S.ctrl.zero(2 * C_WORDS + 1, st);
-    const int64_t nwords = (n + 15) / 16;
-    S.bits.zero(nwords, st);
-    BArgs a{n, sn, d_pt_off ? d_pt : N.pt.p,
-            N.hs_off.p, N.hs.p, N.vs_off.p, N.vs.p, S.map.p, S.base.p, S.c_off.p, S.c_end.p, nullptr, S.head.p,
+    BArgs a{n, sn, sg, d_pt_off ? d_pt : N.pt.p, N.hs.p, N.vs.p, S.map.p, S.base.p, S.c_off.p, S.c_end.p, S.c_net.p, S.head.p,
             S.batch.p, S.ctrl.p, S.lists.p,
             release ? S.rel.p : nullptr, release ? S.cand.p : nullptr, release ? S.cstamp.p : nullptr,
             release ? S.lists.p + 2 * n : nullptr,
@@ -1145,19 +1237,6 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         trace.zero(a.trace_cap * TR_WORDS, st);
         a.trace = trace.p;
     }
-    // Per-cell lists of the nets' point cells, highest priority first.
-    k_cell_count<<<blocks(n), TPB, 0, st>>>(a, S.cnt.p);
-    const int64_t nb = (XYc + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    S.bsum.alloc(nb);
-    k_scan_reduce<<<(unsigned)nb, TPB, 0, st>>>(S.cnt.p, XYc, S.bsum.p);
-    k_scan_bsums<<<1, TPB, 0, st>>>(S.bsum.p, nb);
-    k_scan_apply<<<(unsigned)nb, TPB, 0, st>>>(S.cnt.p, XYc, S.bsum.p, S.c_off.p);
-    HIP_OK(hipGetLastError());
-    int64_t entries = 0;
-    HIP_OK(hipMemcpyAsync(&entries, S.c_off.p + XYc, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
-    S.c_net.alloc(std::max<int64_t>(1, entries));
-    a.c_net = S.c_net.p;
     HIP_OK(hipMemsetAsync(S.cnt.p, 0, sizeof(int) * XYc, st));
     k_cell_fill<<<blocks(n), TPB, 0, st>>>(a, S.cnt.p);
     k_cell_sort<<<blocks(XYc), TPB, 0, st>>>(a, XYc);
