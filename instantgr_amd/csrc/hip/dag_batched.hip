@@ -211,11 +211,13 @@ struct NetArgs {
     const DagEdge* edge;          // per net by child in level order
     const uint32_t* npos;         // per net in node order: position and layer
     const int* lvl;               // per net: nlev + 1 level boundaries
-    const int64_t *nbase, *ebase, *sbase, *lbase, *route_slot;   // by routed net
+    const int64_t *nbase, *ebase, *sbase, *lbase;   // by routed net
+    const int* rorder;            // by routed net: its list entry
+    const int64_t* list_node;     // by list entry: the nodes before it
     const double* cost;           // the batch's edge costs and layer-change samples
     const uint16_t* change;
-    const int *nets, *list;
-    int64_t n, edge0;
+    const int* nets;
+    int64_t net0, n, edge0;       // the batch's nets
     int* queue;
     int* routes;
     int** rptr;
@@ -509,7 +511,8 @@ __device__ void route_net(const NetArgs& a, int64_t r, uint64_t* K, uint8_t* R, 
     // Routes in node order: each node's piece of its parent edge, then its
     // via stack; wires and vias are scattered for the fused track update.
     const int XY = g.X * g.Y;
-    int* rt = a.routes + a.route_slot[r];
+    const int64_t entry = a.rorder[r];
+    int* rt = a.routes + dag_route_slot(a.list_node[entry], entry);
     int base = 1;
     for (int k0 = 0; k0 < nn; k0 += T) {
         const int k = k0 + tid;
@@ -588,13 +591,8 @@ __device__ void route_net(const NetArgs& a, int64_t r, uint64_t* K, uint8_t* R, 
     }
 }
 
-// LDS bytes of one net's tables: keys, layer ranges, decisions, levels.
-__host__ __device__ inline int64_t net_lds(int64_t nodes, int64_t slots, int64_t levels, int ML) {
-    return 8 * slots * ML + 24 * nodes + 4 * (levels + 2);
-}
-
 // Workgroups pull the batch's nets from its queue (one counter per batch,
-// zero at the pass start) in list order, deepest DAG first, and exit when the
+// zero at the pass start) in routing order, deepest DAG first, and exit when the
 // counter passes n.
 template <int L, int NW>
 __global__ void __launch_bounds__(64 * NW) k_dag_net(NetArgs a) {
@@ -607,10 +605,10 @@ __global__ void __launch_bounds__(64 * NW) k_dag_net(NetArgs a) {
         __syncthreads();
         const int qi = s_next;
         if (qi >= a.n) return;
-        const int64_t r = a.list[qi];
+        const int64_t r = a.net0 + qi;
         const int64_t nn = a.nbase[r + 1] - a.nbase[r], ns = a.sbase[r + 1] - a.sbase[r];
         const int64_t nl = a.lbase[r + 1] - a.lbase[r];
-        if (net_lds(nn, ns, nl, ML) <= a.lds_bytes) {
+        if (dag_net_lds_bytes(nn, ns, nl, ML) <= a.lds_bytes) {
             uint64_t* K = reinterpret_cast<uint64_t*>(s_dyn);
             uint2* dec = reinterpret_cast<uint2*>(K + ns * ML);
             uint8_t* R = reinterpret_cast<uint8_t*>(dec + nn);
@@ -656,15 +654,13 @@ static void dag_batch(igr_ctx* c, const DagBatch& b, const DagBatch* rip, int st
     KScope ks(c, K_DAG_DP, b.bytes_dp);
     const unsigned grid = (unsigned)std::min<int64_t>(n, c->tune.dag_grid ? c->tune.dag_grid : DEF_DAG_GRID);
     NetArgs a{c->g, D.nrec.p, D.edge.p, D.npos.p, D.lvl.p, D.node_off.p, D.ebase.p, D.sbase.p, D.lbase.p,
-              D.route_slot.p, D.cost_edges.p, D.change.p, D.nets.p, D.glist.p + b.net0, n, b.edge0,
+              D.rorder.p, D.r_node_off.p, D.cost_edges.p, D.change.p, D.nets.p, b.net0, n, b.edge0,
               D.queue.p + b.index, c->nets.dag_routes.back()->p, c->nets.rptr.p, stamp, b.lds, D.packed.p,
               D.big_range.p, D.big_dec.p, b.node0, b.slot0};
     if (c->tune.dag_waves == 2) k_dag_net<L, 2><<<grid, 128, b.lds, st>>>(a);
     else k_dag_net<L, 4><<<grid, 256, b.lds, st>>>(a);
     HIP_OK(hipGetLastError());
 }
-
-int64_t dag_net_lds(int64_t nodes, int64_t slots, int64_t levels, int L) { return net_lds(nodes, slots, levels, L + 1); }
 
 void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, const DagBatch* rip, int stamp) {
     switch (c->g.L) {

@@ -1,8 +1,8 @@
 // Device layout of one rip-up-and-reroute pass's DAGs (batched form).
 //
 // The host uploads the DAGs as the builder produced them (net list order,
-// local parent indices) and, once the scheduler has fixed the routing order,
-// the per-net bases of that order.  One 64-lane workgroup per routed net then
+// local parent indices); once the scheduler has fixed the routing order,
+// device kernels compute the per-net bases of that order.  One 64-lane workgroup per routed net then
 // writes the net's node records grouped by depth level, its parent-edge records
 // grouped by child in the same order (a child's edges keep their own order),
 // the level boundaries and the node positions (the order inside a level is

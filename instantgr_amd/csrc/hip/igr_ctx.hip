@@ -374,21 +374,21 @@ int igr_pattern_route(igr_ctx* c, const int* order, int64_t n, int form, igr_pas
         if (form != IGR_FORM_PLAIN && form != IGR_FORM_BATCHED) throw std::invalid_argument("unknown form");
         reset_pattern_ptrs(c, order, n);
         double t0 = now_s();
-        std::vector<int> batch_of(n);
+        std::vector<int> batch_of(form == IGR_FORM_PLAIN ? n : 0);
         int nb = form == IGR_FORM_PLAIN ? run_schedule(c, order, n, 0, batch_of.data())
-                                        : run_schedule_batched(c, order, n, 0, batch_of.data());
+                                        : run_schedule_batched(c, order, n, 0, nullptr);
         double t1 = now_s();
         progress("pattern pass: %d batches scheduled in %.3f s", nb, t1 - t0);
-        // Batches in routing order: the scheduler's last batch first; inside a
-        // batch, the scheduler's index order (src/Lshape_route.hpp:175-183).
-        std::vector<int64_t> cnt(nb + 1, 0);
-        for (int64_t i = 0; i < n; i++) cnt[nb - 1 - batch_of[i] + 1]++;
-        for (int b = 0; b < nb; b++) cnt[b + 1] += cnt[b];
-        std::vector<int> list(n);
-        std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
-        for (int64_t i = n - 1; i >= 0; i--) list[pos[nb - 1 - batch_of[i]]++] = order[i];
-        std::vector<int64_t> off(n);
         if (form == IGR_FORM_PLAIN) {
+            // Batches in routing order: the scheduler's last batch first; inside
+            // a batch, the scheduler's index order (src/Lshape_route.hpp:175-183).
+            std::vector<int64_t> cnt(nb + 1, 0);
+            for (int64_t i = 0; i < n; i++) cnt[nb - 1 - batch_of[i] + 1]++;
+            for (int b = 0; b < nb; b++) cnt[b + 1] += cnt[b];
+            std::vector<int> list(n);
+            std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
+            for (int64_t i = n - 1; i >= 0; i--) list[pos[nb - 1 - batch_of[i]]++] = order[i];
+            std::vector<int64_t> off(n);
             int64_t max_nodes = 0;
             for (int b = 0; b < nb; b++)
                 max_nodes = std::max(max_nodes, scratch_offsets(c, list.data() + cnt[b], cnt[b + 1] - cnt[b],
@@ -402,41 +402,33 @@ int igr_pattern_route(igr_ctx* c, const int* order, int64_t n, int form, igr_pas
             for (int b = 0; b < nb; b++)
                 plain_batch(c, c->scratch.net_list.p + cnt[b], c->scratch.scr_off.p + cnt[b], cnt[b + 1] - cnt[b],
                             lbytes[b]);
-        } else {
-            // Each batch's nets by decreasing node count, so that the nets of a
-            // wave are alike and the longest start first: the order of nets
-            // inside a batch changes no result (their footprints are disjoint
-            // and their demand updates integer adds).  Nets above
-            // LSWAVE_MAX_NODES (none under the 12-pin subnet cap) come first
-            // and take the thread-per-net kernel.
-            constexpr int NK = LSWAVE_MAX_NODES + 1;   // keys: larger nets, then LSWAVE_MAX_NODES .. 1 nodes
-            std::vector<int> wl(n);
+        } else if (n > 0) {
+            // The last batch first; each batch's nets by decreasing node count,
+            // so that the nets of a wave are alike and the longest start first.
+            // Nets above LSWAVE_MAX_NODES (none under the 12-pin subnet cap)
+            // come first and take the thread-per-net kernel.
+            constexpr int NK = PATTERN_KEYS;
             std::vector<int64_t> co((size_t)nb * NK + 1, 0);
+            c->scratch.net_list.alloc(n);
+            launch_pattern_order(c, c->sched.ids.p, n, nb, c->scratch.net_list.p, co.data());
             std::vector<double> bbytes((size_t)nb * 2, 0.0);
-            {
-                auto key = [&](int64_t i, int b) {
-                    const int64_t k = c->nets.h_node_off[list[i] + 1] - c->nets.h_node_off[list[i]];
-                    return (size_t)b * NK + (k > LSWAVE_MAX_NODES ? 0 : (size_t)(NK - k));
-                };
-                for (int b = 0; b < nb; b++)
-                    for (int64_t i = cnt[b]; i < cnt[b + 1]; i++) {
-                        const size_t k = key(i, b);
-                        co[k + 1]++;
-                        bbytes[(size_t)b * 2 + (k % NK != 0)] += c->nets.h_lbytes[list[i]];
-                    }
-                for (size_t k = 0; k + 1 < co.size(); k++) co[k + 1] += co[k];
-                std::vector<int64_t> pos(co.begin(), co.end() - 1);
-                for (int b = 0; b < nb; b++)
-                    for (int64_t i = cnt[b]; i < cnt[b + 1]; i++) wl[pos[key(i, b)]++] = list[i];
+            bool big = false;
+            for (int b = 0; b < nb; b++) big = big || co[(size_t)b * NK + 1] > co[(size_t)b * NK];
+            if (big || c->prof.on) {
+                std::vector<int> wl(n);
+                std::vector<int64_t> off(n, 0);
+                HIP_OK(hipMemcpyAsync(wl.data(), c->scratch.net_list.p, sizeof(int) * n, hipMemcpyDeviceToHost,
+                                      c->stream));
+                HIP_OK(hipStreamSynchronize(c->stream));
+                int64_t max_nodes = 0;
+                for (int b = 0; b < nb; b++) {
+                    const int64_t a = co[(size_t)b * NK], m = co[(size_t)b * NK + 1], e = co[(size_t)(b + 1) * NK];
+                    max_nodes = std::max(max_nodes, scratch_offsets(c, wl.data() + a, m - a, off.data() + a));
+                    for (int64_t i = a; i < e; i++) bbytes[(size_t)b * 2 + (i >= m)] += c->nets.h_lbytes[wl[i]];
+                }
+                if (max_nodes) ensure_scratch(c, max_nodes);
+                c->scratch.scr_off.upload(off.data(), n, c->stream);
             }
-            int64_t max_nodes = 0;
-            for (int b = 0; b < nb; b++) {
-                const int64_t a = cnt[b], e = co[(size_t)b * NK + 1];
-                max_nodes = std::max(max_nodes, scratch_offsets(c, wl.data() + a, e - a, off.data() + a));
-            }
-            if (max_nodes) ensure_scratch(c, max_nodes);
-            c->scratch.net_list.upload(wl.data(), n, c->stream);
-            c->scratch.scr_off.upload(off.data(), n, c->stream);
             // Costs of every track once, then per batch: DP (scattering wires,
             // vias and dirty flags), then the fused commit + cost pass over the
             // touched tracks.  The last pass leaves the costs as the plain
@@ -445,13 +437,16 @@ int igr_pattern_route(igr_ctx* c, const int* order, int64_t n, int form, igr_pas
             launch_track_fused(c, 0, 0, true);
             for (int b = 0; b < nb; b++) {
                 const int stamp = ++c->stamp;
-                const int64_t a = cnt[b], m = co[(size_t)b * NK + 1], e = cnt[b + 1];
-                launch_lshape_plain(c, c->scratch.net_list.p + a, c->scratch.scr_off.p + a, m - a, stamp,
-                                    bbytes[(size_t)b * 2]);
-                if (e > m)
-                    launch_lshape_wave(c, c->scratch.net_list.p + m, e - m,
-                                       (int)(c->nets.h_node_off[wl[m] + 1] - c->nets.h_node_off[wl[m]]), stamp,
+                const int64_t* k = co.data() + (size_t)b * NK;   // first entry of every key
+                if (k[1] > k[0])
+                    launch_lshape_plain(c, c->scratch.net_list.p + k[0], c->scratch.scr_off.p + k[0], k[1] - k[0],
+                                        stamp, bbytes[(size_t)b * 2]);
+                if (k[NK] > k[1]) {
+                    int largest = 1;
+                    while (k[largest + 1] == k[largest]) largest++;
+                    launch_lshape_wave(c, c->scratch.net_list.p + k[1], k[NK] - k[1], NK - largest, stamp,
                                        bbytes[(size_t)b * 2 + 1]);
+                }
                 launch_track_fused(c, stamp, 0, b + 1 < nb);
             }
             HIP_OK(hipStreamSynchronize(c->stream));
@@ -523,15 +518,52 @@ int igr_get_routes(igr_ctx* c, int64_t* off, int* data, int64_t cap) {
 
 namespace {
 
+// Threads for a loop over cnt nets: a short list is done before a second
+// thread has started.
+int loop_threads(int64_t cnt) { return (int)std::max<int64_t>(1, std::min<int64_t>(host_threads(), cnt / 2048)); }
+
 void pfor(int64_t cnt, const std::function<void(int64_t, int64_t)>& fn) {
-    const int nthreads = std::max(1, std::min(16, (int)std::thread::hardware_concurrency()));
-    std::vector<std::thread> th;
-    const int64_t chunk = (cnt + nthreads - 1) / nthreads;
-    for (int t = 0; t < nthreads; t++) {
-        const int64_t a0 = t * chunk, a1 = std::min(cnt, a0 + chunk);
-        if (a0 < a1) th.emplace_back(fn, a0, a1);
-    }
-    for (auto& x : th) x.join();
+    igr::parallel_ranges(cnt, loop_threads(cnt), [&](int64_t a, int64_t b, int) { fn(a, b); });
+}
+
+// Kernel timing only: algorithmic bytes of the DAG kernels per net, list order
+// (the models are stated in the plain path).
+void dag_bytes(igr_ctx* c, const igr_dag_desc* dg, int64_t n, std::vector<double>& l_eb, std::vector<double>& l_db) {
+    const int XY = c->g.X * c->g.Y, L = c->g.L, ML = L + 1;
+    double pairs[2] = {0, 0}, pvia[2] = {0, 0};
+    for (int fl = 0; fl < L; fl++)
+        for (int tl = fl & 1; tl < L; tl += 2) {
+            pairs[layer_dir(fl, c->g.DIR)] += 1;
+            pvia[layer_dir(fl, c->g.DIR)] += std::abs(fl - tl);
+        }
+    l_eb.resize(n);
+    l_db.resize(n);
+    pfor(n, [&](int64_t a0, int64_t a1) {
+        for (int64_t i = a0; i < a1; i++) {
+            const int64_t b0 = dg->node_off[i], b1 = dg->node_off[i + 1];
+            int64_t slots = 0;
+            double eb = 0, longp = 0;
+            for (int64_t k = b0; k < b1; k++) {
+                slots += dg->child_num[k];
+                const int v = dg->nodes[k];
+                for (int64_t q = dg->par_off[k]; q < dg->par_off[k + 1]; q++) {
+                    const int64_t pl = dg->par[q];
+                    if (pl < 0 || pl >= b1 - b0) continue;   // rejected by the layout
+                    const int u = dg->nodes[b0 + pl];
+                    const int vx = v % XY / c->g.Y, vy = v % c->g.Y, ux = u % XY / c->g.Y, uy = u % c->g.Y;
+                    const int dist = std::abs(vx - ux) + std::abs(vy - uy);
+                    if (dist <= 4 || (vx != ux && vy != uy)) continue;
+                    const int dir = vx == ux ? 1 : 0;
+                    const int dd = dist / std::min(dist, 20);
+                    eb += ((dist - 1) / dd) * (16 * pairs[dir] + 4 * pvia[dir]) + 12 * pairs[dir];
+                    longp += pairs[dir];
+                }
+            }
+            const int64_t nn = b1 - b0, ne = dg->par_off[b1] - dg->par_off[b0];
+            l_eb[i] = eb;
+            l_db[i] = nn * (4.0 + 4 * L + 16 * ML + 32) + ne * (8.0 + 8 * L + 8 * ML) + longp * 8 + slots * 16.0 * ML;
+        }
+    });
 }
 
 // Batched form of one rip-up-and-reroute pass.  While the scheduler runs on
@@ -539,8 +571,8 @@ void pfor(int64_t cnt, const std::function<void(int64_t, int64_t)>& fn) {
 // and measures every net (nodes, edges, slots, levels, algorithmic bytes).
 // With 'complete' set, dg holds only the points on entry and the helper first
 // has the rest of it built, so that building overlaps the scheduler too.
-// Once the routing order is known the host only computes per-net bases and
-// batch bounds; the device lays the DAGs out (k_dag_layout) and checks them.
+// The device sorts the nets into routing order, computes their bases and the
+// batch bounds (order_kernels.hip), and lays the DAGs out (k_dag_layout).
 void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const igr_dag_desc* dg_in,
                       const std::function<void(igr_dag_desc&)>& complete, igr_pass_stats* st) {
     const int XY = c->g.X * c->g.Y, L = c->g.L, ML = L + 1;
@@ -564,22 +596,14 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     D.pt_off.upload(dg->pt_off, n + 1, s);
     D.pt.upload(dg->pts, dg->pt_off[n], s);
 
-    double pairs[2] = {0, 0}, pvia[2] = {0, 0};
-    for (int fl = 0; fl < L; fl++)
-        for (int tl = fl & 1; tl < L; tl += 2) {
-            pairs[layer_dir(fl, c->g.DIR)] += 1;
-            pvia[layer_dir(fl, c->g.DIR)] += std::abs(fl - tl);
-        }
     int64_t NN = 0, NE = 0;
-    std::vector<int64_t> l_ns(n);
-    std::vector<int> l_nl(n);
-    std::vector<double> l_eb(n), l_db(n);
-    std::atomic<int> bad_dag{0};
+    std::vector<double> l_eb, l_db;   // kernel timing only: algorithmic bytes of the DAG kernels, list order
     std::exception_ptr herr;
     double t_helper = 0;
     std::thread helper([&]() {
         try {
             const double h0 = now_s();
+            HIP_OK(hipSetDevice(c->device));   // per thread
             if (complete) complete(dgv);
             if (dg->node_off[0] != 0 || dg->par_off[0] != 0) throw std::invalid_argument("DAG offsets must start at 0");
             std::atomic<int> empty{0};
@@ -590,131 +614,70 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
             if (empty.load()) throw std::invalid_argument("empty DAG");
             NN = dg->node_off[n];
             NE = dg->par_off[NN];
+            if (NE < 0) throw std::invalid_argument("malformed DAG (edge offsets, depths or slot counts)");
             hipStream_t cs = c->copy_stream;
             D.r_node_off.upload(dg->node_off, n + 1, cs);
-            D.r_nodes.upload(dg->nodes, NN, cs);
             D.r_par_off.upload(dg->par_off, NN + 1, cs);
-            D.r_par.upload(dg->par, NE, cs);
-            D.r_slot.upload(dg->slot, NE, cs);
             D.r_child_num.upload(dg->child_num, NN, cs);
             D.r_depth.upload(dg->depth, NN, cs);
-            // Per net (list order): slots, levels and the algorithmic bytes
-            // of the DAG kernels (the models are stated in the plain path).
-            pfor(n, [&](int64_t a0, int64_t a1) {
-                for (int64_t i = a0; i < a1; i++) {
-                    const int64_t b0 = dg->node_off[i], b1 = dg->node_off[i + 1];
-                    int64_t slots = 0;
-                    int maxd = 0;
-                    double eb = 0, longp = 0;
-                    for (int64_t k = b0; k < b1; k++) {
-                        // the layout kernel trusts the edge offsets and depths
-                        if (dg->par_off[k + 1] < dg->par_off[k] || dg->par_off[k + 1] > NE || dg->depth[k] < 0 ||
-                            dg->depth[k] >= b1 - b0 || dg->child_num[k] < 0 || dg->child_num[k] > 10) {
-                            bad_dag.store(1);
-                            break;
-                        }
-                        slots += dg->child_num[k];
-                        maxd = std::max(maxd, dg->depth[k]);
-                        const int v = dg->nodes[k];
-                        for (int64_t q = dg->par_off[k]; q < dg->par_off[k + 1]; q++) {
-                            const int64_t pl = dg->par[q];
-                            if (pl < 0 || pl >= b1 - b0) continue;   // rejected by the layout
-                            const int u = dg->nodes[b0 + pl];
-                            const int vx = v % XY / c->g.Y, vy = v % c->g.Y, ux = u % XY / c->g.Y, uy = u % c->g.Y;
-                            const int dist = std::abs(vx - ux) + std::abs(vy - uy);
-                            if (dist <= 4 || (vx != ux && vy != uy)) continue;
-                            const int dir = vx == ux ? 1 : 0;
-                            const int dd = dist / std::min(dist, 20);
-                            eb += ((dist - 1) / dd) * (16 * pairs[dir] + 4 * pvia[dir]) + 12 * pairs[dir];
-                            longp += pairs[dir];
-                        }
-                    }
-                    const int64_t nn = b1 - b0, ne = dg->par_off[b1] - dg->par_off[b0];
-                    l_ns[i] = slots;
-                    l_nl[i] = maxd + 1;
-                    l_eb[i] = eb;
-                    l_db[i] = nn * (4.0 + 4 * L + 16 * ML + 32) + ne * (8.0 + 8 * L + 8 * ML) + longp * 8 +
-                              slots * 16.0 * ML;
-                }
-            });
+            launch_dag_measure(c, n, NE, cs);
+            D.r_nodes.upload(dg->nodes, NN, cs);
+            D.r_par.upload(dg->par, NE, cs);
+            D.r_slot.upload(dg->slot, NE, cs);
+            int err = 0;
+            HIP_OK(hipMemcpyAsync(&err, D.err.p, sizeof(int), hipMemcpyDeviceToHost, cs));
             HIP_OK(hipStreamSynchronize(cs));
+            if (err) throw std::invalid_argument("malformed DAG (edge offsets, depths or slot counts)");
+            if (c->prof.on) dag_bytes(c, dg, n, l_eb, l_db);
             t_helper = now_s() - h0;
         } catch (...) {
             herr = std::current_exception();
         }
     });
-    std::vector<int> batch_of(n);
     int nb = 0;
     try {
-        nb = run_schedule_batched(c, nets, n, mode, batch_of.data(), D.pt_off.p, D.pt.p);
+        nb = run_schedule_batched(c, nets, n, mode, nullptr, D.pt_off.p, D.pt.p);
     } catch (...) {
         helper.join();
         throw;
     }
     helper.join();
     if (herr) std::rethrow_exception(herr);
-    if (bad_dag.load()) throw std::invalid_argument("malformed DAG (edge offsets, depths or slot counts)");
     progress("DAG pass: %d batches scheduled in %.3f s", nb, now_s() - t0);
     const double t1 = now_s();
 
-    // Routing order: batch nb-1 first, inside a batch decreasing list
-    // position (the scheduler's index order).
-    std::vector<int64_t> cntb(nb + 1, 0);
-    for (int64_t i = 0; i < n; i++) cntb[nb - 1 - batch_of[i] + 1]++;
-    for (int b = 0; b < nb; b++) cntb[b + 1] += cntb[b];
-    std::vector<int> rorder(n), rnets(n);
-    {
-        std::vector<int64_t> pos(cntb.begin(), cntb.end() - 1);
-        for (int64_t i = n - 1; i >= 0; i--) rorder[pos[nb - 1 - batch_of[i]]++] = (int)i;
+    // Routing order: batch nb-1 first, inside a batch the deepest DAG first
+    // (dag_order 1) or as they come (2).
+    const bool deep_first = (c->tune.dag_order ? c->tune.dag_order : DEF_DAG_ORDER) == 1;
+    std::vector<DagBound> bound(nb + 1);
+    int any_big = 0;
+    launch_dag_order(c, c->sched.ids.p, n, nb, deep_first, bound.data(), &any_big);
+    std::vector<int> rorder;   // kernel timing and traces only
+    if (c->prof.on || std::getenv("IGR_DAG_TRACE")) {
+        rorder.resize(n);
+        HIP_OK(hipMemcpyAsync(rorder.data(), D.rorder.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+        HIP_OK(hipStreamSynchronize(s));
     }
-    std::vector<int64_t> nbase(n + 1, 0), ebase(n + 1, 0), sbase(n + 1, 0), lbase(n + 1, 0), route_slot(n + 1, 0);
-    for (int64_t r = 0; r < n; r++) {
-        const int64_t i = rorder[r];
-        const int64_t nn = dg->node_off[i + 1] - dg->node_off[i];
-        rnets[r] = nets[i];
-        nbase[r + 1] = nbase[r] + nn;
-        ebase[r + 1] = ebase[r] + (dg->par_off[dg->node_off[i + 1]] - dg->par_off[dg->node_off[i]]);
-        sbase[r + 1] = sbase[r] + l_ns[i];
-        lbase[r + 1] = lbase[r] + l_nl[i];
-        route_slot[r + 1] = route_slot[r] + 8 * nn + 1;
-    }
-    const int64_t NL = lbase[n];
     std::vector<DagBatch> batches(nb);
     int64_t mx_nodes = 0, mx_edges = 0, mx_slots = 0;
-    bool any_big = false;
-    // Per batch, the routed nets in launch order of the workgroup-per-net
-    // kernel: deepest DAG first, then most nodes (dag_order 1), or routing
-    // order (2).
-    const bool deep_first = (c->tune.dag_order ? c->tune.dag_order : DEF_DAG_ORDER) == 1;
-    std::vector<int> glist(n);
-    std::vector<std::pair<int64_t, int64_t>> gl;   // (sort key, routed net)
     for (int b = 0; b < nb; b++) {
         DagBatch& B = batches[b];
-        gl.clear();
-        for (int64_t r = cntb[b]; r < cntb[b + 1]; r++)
-            gl.emplace_back(deep_first ? -((lbase[r + 1] - lbase[r]) << 32 | (nbase[r + 1] - nbase[r])) : 0, r);
-        if (deep_first) std::sort(gl.begin(), gl.end());
-        for (size_t k = 0; k < gl.size(); k++) glist[cntb[b] + k] = (int)gl[k].second;
-        B.net0 = cntb[b];
-        B.net1 = cntb[b + 1];
-        B.node0 = nbase[B.net0];
-        B.node1 = nbase[B.net1];
-        B.edge0 = ebase[B.net0];
-        B.edge1 = ebase[B.net1];
-        B.slot0 = sbase[B.net0];
-        B.slot1 = sbase[B.net1];
-        int maxl = 1;
-        int64_t lds = 0;
-        for (int64_t r = B.net0; r < B.net1; r++) {
-            maxl = std::max(maxl, l_nl[rorder[r]]);
-            const int64_t need = dag_net_lds(nbase[r + 1] - nbase[r], sbase[r + 1] - sbase[r], lbase[r + 1] - lbase[r], L);
-            if (need <= DAG_LDS_MAX) lds = std::max(lds, need);
-            else any_big = true;
-            B.bytes_edges += l_eb[rorder[r]];
-            B.bytes_dp += l_db[rorder[r]];
-        }
-        B.levels = maxl;
-        B.lds = (int)lds;
+        const DagBound &lo = bound[b], &hi = bound[b + 1];
+        B.net0 = lo.net0;
+        B.net1 = hi.net0;
+        B.node0 = lo.node0;
+        B.node1 = hi.node0;
+        B.edge0 = lo.edge0;
+        B.edge1 = hi.edge0;
+        B.slot0 = lo.slot0;
+        B.slot1 = hi.slot0;
+        B.lds = (int)lo.lds;
+        if (c->prof.on)
+            for (int64_t r = B.net0; r < B.net1; r++) {
+                B.bytes_edges += l_eb[rorder[r]];
+                B.bytes_dp += l_db[rorder[r]];
+            }
+        B.levels = 0;
         B.index = b;
         B.lvl0 = 0;
         mx_nodes = std::max(mx_nodes, B.node1 - B.node0);
@@ -730,22 +693,22 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
             for (int b = 0; b < nb; b++) {
                 const DagBatch& B = batches[b];
                 int64_t mxn = 0;
-                for (int64_t r = B.net0; r < B.net1; r++) mxn = std::max(mxn, nbase[r + 1] - nbase[r]);
+                int mxl = 0;
+                for (int64_t r = B.net0; r < B.net1; r++) {
+                    const int64_t i = rorder[r];
+                    mxn = std::max(mxn, dg->node_off[i + 1] - dg->node_off[i]);
+                    for (int64_t k = dg->node_off[i]; k < dg->node_off[i + 1]; k++) mxl = std::max(mxl, dg->depth[k] + 1);
+                }
                 std::fprintf(f, "%d %lld %lld %lld %lld %d %lld\n", b, (long long)(B.net1 - B.net0),
                              (long long)(B.node1 - B.node0), (long long)(B.edge1 - B.edge0),
-                             (long long)(B.slot1 - B.slot0), B.levels, (long long)mxn);
+                             (long long)(B.slot1 - B.slot0), mxl, (long long)mxn);
             }
             std::fclose(f);
         }
     }
-    D.glist.upload(glist.data(), n, s);
-    D.nets.upload(rnets.data(), n, s);
-    D.rorder.upload(rorder.data(), n, s);
-    D.node_off.upload(nbase.data(), n + 1, s);
-    D.ebase.upload(ebase.data(), n + 1, s);
-    D.sbase.upload(sbase.data(), n + 1, s);
-    D.lbase.upload(lbase.data(), n + 1, s);
-    D.route_slot.upload(route_slot.data(), n + 1, s);
+    int64_t NL = 0;
+    HIP_OK(hipMemcpyAsync(&NL, D.lbase.p + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    HIP_OK(hipStreamSynchronize(s));
     D.nrec.alloc(NN);
     D.npos.alloc(NN);
     D.edge.alloc(NE);
@@ -753,7 +716,6 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     D.lcur.alloc(NL + n);
     D.lpos.alloc(NN);
     D.lslot.alloc(NN);
-    D.err.zero(1, s);
     const double t_meta = now_s();
     DagLayoutArgs la{D.r_node_off.p, D.r_nodes.p, D.r_par_off.p, D.r_par.p, D.r_slot.p, D.r_child_num.p, D.r_depth.p,
                      D.rorder.p, D.node_off.p, D.ebase.p, D.sbase.p, D.lbase.p, c->g.X, c->g.Y, (L + 1) * XY,
@@ -774,7 +736,7 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     D.change.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
     NetsDev& N = c->nets;
     N.dag_routes.push_back(new DevBuf<int>());
-    N.dag_routes.back()->alloc(route_slot[n]);
+    N.dag_routes.back()->alloc(dag_route_slot(NN, n));
     int* rbase = N.dag_routes.back()->p;
     const double tp = now_s();
 
@@ -812,7 +774,7 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
         bs.check();
     }
     HIP_OK(hipStreamSynchronize(s));
-    N.adopt(rnets.data(), route_slot.data(), n, rbase);
+    N.adopt(nets, n, rbase, loop_threads(n), [&](int64_t i) { return dag_route_slot(dg->node_off[i], i); });
     const double t2 = now_s();
     c->last_dag_prep_s = tp - t1;
     c->last_dag_prep_parts[0] = t_meta - t1;     // routing-order bases, batch bounds, small uploads
@@ -1065,7 +1027,7 @@ int igr_dag_pass(igr_ctx* c, const int* nets, int64_t n, int mode, int form, con
             HIP_OK(hipStreamSynchronize(s));
         }
         HIP_OK(hipStreamSynchronize(s));
-        N.adopt(rnets.data(), route_slot.data(), n, rbase);
+        N.adopt(rnets.data(), n, rbase, 1, [&](int64_t r) { return route_slot[r]; });
         double t2 = now_s();
         c->last_dag_prep_s = tp - t1;
         c->last_dag_prep_parts[0] = t_fill - t1;

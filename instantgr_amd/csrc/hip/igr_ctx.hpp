@@ -3,6 +3,7 @@
 #pragma once
 #include "igr_dev.h"
 #include "igr.h"
+#include "par.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -85,22 +86,31 @@ struct NetsDev {
             dag_routes[k] = nullptr;
         }
     }
-    // The listed nets' routes now live in the newest buffer at rbase + slot[r].
-    void adopt(const int* rnets, const int64_t* slot, int64_t n, int* rbase) {
+    // The listed nets' routes now live in the newest buffer, net rnets[r] at
+    // rbase + slot(r), on 'threads' host threads.
+    template <class Slot>
+    void adopt(const int* rnets, int64_t n, int* rbase, int threads, Slot slot) {
         const int k = (int)dag_routes.size() - 1;
         dag_live.resize(dag_routes.size(), 0);
-        for (int64_t r = 0; r < n; r++) {
-            const int net = rnets[r];
-            release(net);
-            h_rptr[net] = rbase + slot[r];
-            h_rcap[net] = slot[r + 1] - slot[r];
-            h_rbuf[net] = k;
-            dag_live[k]++;
-        }
-        if (dag_live[k] == 0) {
-            delete dag_routes[k];
-            dag_routes[k] = nullptr;
-        }
+        std::vector<std::vector<int64_t>> left(threads);   // nets that leave each buffer
+        igr::parallel_ranges(n, threads, [&](int64_t a, int64_t b, int t) {
+            left[t].assign(dag_routes.size(), 0);
+            for (int64_t r = a; r < b; r++) {
+                const int net = rnets[r];
+                if (h_rbuf[net] >= 0) left[t][h_rbuf[net]]++;
+                h_rptr[net] = rbase + slot(r);
+                h_rcap[net] = slot(r + 1) - slot(r);
+                h_rbuf[net] = k;
+            }
+        });
+        dag_live[k] += n;
+        for (const auto& v : left)
+            for (size_t j = 0; j < v.size(); j++) dag_live[j] -= v[j];
+        for (size_t j = 0; j < dag_routes.size(); j++)
+            if (dag_routes[j] && dag_live[j] == 0) {
+                delete dag_routes[j];
+                dag_routes[j] = nullptr;
+            }
     }
 };
 
@@ -131,6 +141,10 @@ struct alignas(16) DagEdge {
     uint32_t child;               // record of the child in the net
 };
 
+struct alignas(16) DagSize {
+    int nodes, edges, slots, levels;
+};
+
 // One rip-up-and-reroute pass on the device: DAGs of the rerouted nets in
 // routing order (batch by batch), with global node/edge/slot numbering.
 struct DagDev {
@@ -157,10 +171,30 @@ struct DagDev {
     // positions and slot bases.
     DevBuf<int64_t> r_node_off, r_par_off, ebase, sbase, lbase;
     DevBuf<int> r_nodes, r_par, r_slot, r_child_num, r_depth, rorder, err, lcur, lpos, lslot;
-    // Batched form: the routed nets of each batch in launch order, and the
-    // per-batch work-queue counters.
-    DevBuf<int> glist, queue;
+    // Batched form: the per-batch work-queue counters and the DAGs' sizes.
+    DevBuf<int> queue;
+    DevBuf<DagSize> size;         // per list entry
 };
+
+// Workspaces of the device routing order (order_kernels.hip).
+constexpr int PATTERN_KEYS = 25;  // nets above LSWAVE_MAX_NODES, then LSWAVE_MAX_NODES .. 1 nodes
+constexpr int DAG_KEYS = 64;      // 64 or more depth levels, then 63 .. 1
+struct DagBound {
+    int64_t net0, node0, edge0, slot0;
+    int64_t lds;                  // LDS of the batch's net kernel
+};
+struct OrderDev {
+    DevBuf<int> cnt, rank, lds;
+    DevBuf<int64_t> off, tot;
+    DevBuf<int4> rsize;
+    DevBuf<DagBound> bound;
+};
+// A DAG pass's route slots, in list order: 8 ints a node and one a net.
+__host__ __device__ inline int64_t dag_route_slot(int64_t nodes_before, int64_t entry) { return 8 * nodes_before + entry; }
+// LDS bytes of one net's DAG tables: keys, layer ranges, decisions, levels.
+__host__ __device__ inline int64_t dag_net_lds_bytes(int64_t nodes, int64_t slots, int64_t levels, int ML) {
+    return 8 * slots * ML + 24 * nodes + 4 * (levels + 2);
+}
 
 // Arguments of the device DAG layout (one workgroup per routed net).
 struct DagLayoutArgs {
@@ -252,6 +286,7 @@ struct igr_ctx {
     igr_dev::Sched sched;
     igr_dev::Scratch scratch;
     igr_dev::DagDev dag;
+    igr_dev::OrderDev order;
     int stamp = 0;
     igr_tuning tune{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // launch-shape overrides (0 = built-in)
     double last_dag_prep_s = 0;   // host preparation time of the last DAG pass
@@ -358,7 +393,8 @@ void noalloc_init(int device);
 int run_schedule(igr_ctx* c, const int* h_order, int64_t n, int mode, int* h_batch_of,
                  const int64_t* d_pt_off = nullptr, const int* d_pt = nullptr);
 // The same schedule computed incrementally with device-side round control
-// (batched form).
+// (batched form).  The batches also stay on the device (sched.batch, by
+// scheduler index); h_batch_of may be null.
 int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, int* h_batch_of,
                          const int64_t* d_pt_off = nullptr, const int* d_pt = nullptr);
 void launch_rip_wire(igr_ctx* c, const int* d_nets, int64_t n, int stamp);
@@ -379,11 +415,21 @@ void launch_dag_compact(igr_ctx* c, const DagBatch& b);
 // queue counters are zeroed first.  The batch to rip up next (or null) is
 // scattered by the same launches.
 void launch_dag_batch_wave(igr_ctx* c, const DagBatch& b, const DagBatch* rip, int stamp);
-// LDS bytes of a net's tables in that form, and the most a launch takes (a
-// larger net's tables live in global memory).
-int64_t dag_net_lds(int64_t nodes, int64_t slots, int64_t levels, int L);
+// The most LDS a launch of that form takes for a net's tables (a larger net's
+// live in global memory).
 constexpr int64_t DAG_LDS_MAX = 60 * 1024;
 void launch_dag_queue_reset(igr_ctx* c, int64_t batches);
+// Routing order of the last schedule's n nets (nb batches) by device kernels.
+// Pattern: the net list by (batch, decreasing node count), h_off[nb *
+// PATTERN_KEYS + 1] the first entry of every (batch, key).  DAG pass, after
+// launch_dag_measure (sizes and checks of the uploaded DAGs; D.err): the routed
+// order, nets and bases, h_bound[nb + 1] every batch's bounds, *h_big whether a
+// net's tables exceed LDS.  Both wait for the stream.
+void launch_pattern_order(igr_ctx* c, const int* d_order, int64_t n, int nb, int* d_list, int64_t* h_off);
+void launch_dag_measure(igr_ctx* c, int64_t n, int64_t edges, hipStream_t s);
+void launch_dag_order(igr_ctx* c, const int* d_nets, int64_t n, int nb, bool deep_first, DagBound* h_bound, int* h_big);
+// off[i] = cnt[0] + .. + cnt[i - 1], off[n] the total (n > 0).
+void launch_exclusive_scan(igr_ctx* c, const int* cnt, int64_t n, int64_t* off);
 // Batched form: the device layout of a pass's DAGs.
 void launch_dag_layout(igr_ctx* c, const DagLayoutArgs& a, int64_t n);
 void launch_expf(const float* in, float* out, int64_t n, hipStream_t s);

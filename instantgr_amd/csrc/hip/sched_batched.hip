@@ -1163,6 +1163,15 @@ inline unsigned blocks(int64_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
 } // namespace
 
+void launch_exclusive_scan(igr_ctx* c, const int* cnt, int64_t n, int64_t* off) {
+    const int64_t nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
+    c->sched.bsum.alloc(nb);
+    k_scan_reduce<<<(unsigned)nb, TPB, 0, c->stream>>>(cnt, n, c->sched.bsum.p);
+    k_scan_bsums<<<1, TPB, 0, c->stream>>>(c->sched.bsum.p, nb);
+    k_scan_apply<<<(unsigned)nb, TPB, 0, c->stream>>>(cnt, n, c->sched.bsum.p, off);
+    HIP_OK(hipGetLastError());
+}
+
 int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, int* h_batch_of,
                          const int64_t* d_pt_off, const int* d_pt) {
     if (n == 0) return 0;
@@ -1194,12 +1203,7 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     S.bits.zero(nwords, st);
     // Per-cell lists of the nets' point cells, highest priority first.
     k_cell_count<<<blocks(n), TPB, 0, st>>>(n, sn, d_pt_off ? d_pt : N.pt.p, S.cnt.p);
-    const int64_t nb = (XYc + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    S.bsum.alloc(nb);
-    k_scan_reduce<<<(unsigned)nb, TPB, 0, st>>>(S.cnt.p, XYc, S.bsum.p);
-    k_scan_bsums<<<1, TPB, 0, st>>>(S.bsum.p, nb);
-    k_scan_apply<<<(unsigned)nb, TPB, 0, st>>>(S.cnt.p, XYc, S.bsum.p, S.c_off.p);
-    HIP_OK(hipGetLastError());
+    launch_exclusive_scan(c, S.cnt.p, XYc, S.c_off.p);
     int64_t entries = 0;
     HIP_OK(hipMemcpyAsync(&entries, S.c_off.p + XYc, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
@@ -1301,6 +1305,7 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         throw;
     }
     const int nbatch = h_ctrl[(g & 1) * C_WORDS + C_CUR];
+    const int64_t placed = h_ctrl[2 * C_WORDS];
     HIP_OK(hipHostFree(h_ctrl));
     if (a.bytes) {
         std::vector<unsigned long long> slots(BYTE_SLOTS);
@@ -1339,13 +1344,12 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
                  "batch", release ? "release-driven" : "active-list", nbatch, sv[0],
                  sv[0] ? (double)sv[1] / (double)sv[0] : 0.0, nbatch ? (double)sv[2] / nbatch : 0.0);
     }
+    if (placed != n) throw std::runtime_error("scheduler left a net without a batch");
+    if (!h_batch_of) return nbatch;
     std::vector<int> b(n);
     HIP_OK(hipMemcpyAsync(b.data(), S.batch.p, sizeof(int) * n, hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
-    for (int64_t i = 0; i < n; i++) {
-        if (b[i] < 0) throw std::runtime_error("scheduler left a net without a batch");
-        h_batch_of[n - 1 - i] = b[i];
-    }
+    for (int64_t i = 0; i < n; i++) h_batch_of[n - 1 - i] = b[i];
     return nbatch;
 }
 
