@@ -7,6 +7,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstdarg>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -462,16 +463,71 @@ int igr_pattern_route(igr_ctx* c, const int* order, int64_t n, int form, igr_pas
     });
 }
 
+namespace igr_dev {
+// One workgroup: a route is a few hundred words, and the read is bound by the
+// launch and the trip over the link.  Every thread's words are made visible
+// to the host before the barrier, the read's number after it.
+static __global__ void __launch_bounds__(256) k_read_route(const int* src, int room, int* mail, int number) {
+    const int first = (int)threadIdx.x < room ? src[threadIdx.x] : 0;   // beside the length, not after it
+    const int used = min(max(src[0], 0), room);
+    for (int i = threadIdx.x; i < used; i += 256) mail[MAIL_HEAD + i] = i == 0 ? used : i < 256 ? first : src[i];
+    if (used == 0 && threadIdx.x == 0) mail[MAIL_HEAD] = 0;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(mail, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+const int* read_route(igr_ctx* c, const int* src, int64_t rc) {
+    Mailbox& m = c->mail;
+    if (!m.word) {
+        int* w = nullptr;
+        void* d = nullptr;
+        HIP_OK(hipHostMalloc(&w, sizeof(int) * (MAIL_HEAD + MAIL_WORDS), hipHostMallocMapped | hipHostMallocCoherent));
+        if (hipHostGetDevicePointer(&d, w, 0) != hipSuccess) {
+            (void)hipHostFree(w);
+            throw std::runtime_error("route mailbox is not visible to the device");
+        }
+        std::memset(w, 0, sizeof(int) * (MAIL_HEAD + MAIL_WORDS));
+        m.word = w;
+        m.dev = static_cast<int*>(d);
+    }
+    const int number = m.reads = m.reads == INT_MAX ? 1 : m.reads + 1;
+    k_read_route<<<1, 256, 0, c->stream>>>(src, (int)rc, m.dev, number);
+    HIP_OK(hipGetLastError());
+    // Behind other work of the stream, or after a failure, the wait is the runtime's.
+    const auto arrived = [&] { return __atomic_load_n(m.word, __ATOMIC_ACQUIRE) == number; };
+    for (int spin = 0; spin < 20000 && !arrived(); spin++) __builtin_ia32_pause();
+    if (!arrived()) {
+        HIP_OK(hipStreamSynchronize(c->stream));
+        if (!arrived()) throw std::runtime_error("a route read did not finish");
+    }
+    return m.word + MAIL_HEAD;
+}
+} // namespace igr_dev
+
 int igr_get_route(igr_ctx* c, int net, int* buf, int cap, int* len) {
     return guard([&]() {
         if (net < 0 || net >= c->nets.n) throw std::invalid_argument("net id out of range");
         const int64_t rc = c->nets.h_rcap[net];
+        const auto give = [&](const int* r) {
+            const int used = r[0];
+            if (len) *len = used;
+            for (int i = 0; i < used && i < cap; i++) buf[i] = r[i];
+        };
+        // A kernel writes the route into host memory in 9 us; a copy of the
+        // slot to pageable memory and a wait took 23.  It stays for a route
+        // larger than the mailbox and for callers on another device (a launch
+        // needs the context's, a copy does not).
+        int cur = -1;
+        if (rc <= MAIL_WORDS && hipGetDevice(&cur) == hipSuccess && cur == c->device) {
+            std::lock_guard<std::mutex> lk(c->mail.mu);
+            give(read_route(c, c->nets.h_rptr[net], rc));
+            return;
+        }
         std::vector<int> tmp(rc);
         HIP_OK(hipMemcpyAsync(tmp.data(), c->nets.h_rptr[net], sizeof(int) * rc, hipMemcpyDeviceToHost, c->stream));
         HIP_OK(hipStreamSynchronize(c->stream));
-        int used = tmp[0];
-        if (len) *len = used;
-        for (int i = 0; i < used && i < cap; i++) buf[i] = tmp[i];
+        give(tmp.data());
     });
 }
 

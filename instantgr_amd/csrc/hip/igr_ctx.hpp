@@ -9,6 +9,7 @@
 
 #include <stdexcept>
 #include <string>
+#include <mutex>
 #include <vector>
 
 #define HIP_OK(expr)                                                                               \
@@ -47,6 +48,21 @@ struct DevBuf {
     void zero(size_t count, hipStream_t s) {
         alloc(count);
         HIP_OK(hipMemsetAsync(p, 0, count * sizeof(T), s));
+    }
+};
+
+// Host memory that kernels write straight into (mapped, coherent): the route
+// reads of igr_get_route.  word[0] holds the number of the last read that
+// finished, the route follows from word[MAIL_HEAD].  'mu' makes one read at a
+// time use it.
+constexpr int MAIL_HEAD = 16, MAIL_WORDS = 16384;
+struct Mailbox {
+    std::mutex mu;
+    int* word = nullptr;    // host address
+    int* dev = nullptr;     // the same memory to the device
+    int reads = 0;
+    ~Mailbox() {
+        if (word) (void)hipHostFree(word);
     }
 };
 
@@ -287,6 +303,7 @@ struct igr_ctx {
     igr_dev::Scratch scratch;
     igr_dev::DagDev dag;
     igr_dev::OrderDev order;
+    igr_dev::Mailbox mail;
     int stamp = 0;
     igr_tuning tune{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // launch-shape overrides (0 = built-in)
     double last_dag_prep_s = 0;   // host preparation time of the last DAG pass
@@ -428,6 +445,10 @@ void launch_dag_queue_reset(igr_ctx* c, int64_t batches);
 void launch_pattern_order(igr_ctx* c, const int* d_order, int64_t n, int nb, int* d_list, int64_t* h_off);
 void launch_dag_measure(igr_ctx* c, int64_t n, int64_t edges, hipStream_t s);
 void launch_dag_order(igr_ctx* c, const int* d_nets, int64_t n, int nb, bool deep_first, DagBound* h_bound, int* h_big);
+// Net's route (rc words of room, at most MAIL_WORDS) from device memory into
+// the context's mailbox, after all work on the stream; returns its host address.
+// Needs c->mail.mu.
+const int* read_route(igr_ctx* c, const int* src, int64_t rc);
 // off[i] = cnt[0] + .. + cnt[i - 1], off[n] the total (n > 0).
 void launch_exclusive_scan(igr_ctx* c, const int* cnt, int64_t n, int64_t* off);
 // Batched form: the device layout of a pass's DAGs.
