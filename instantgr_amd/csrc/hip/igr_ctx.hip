@@ -125,26 +125,18 @@ void igr_destroy(igr_ctx* c) {
 
 static void to_host_ref(igr_ctx* c, const void* dev, void* host, int eb) {
     const int64_t n = c->cells();
-    if (eb == 4) {
-        DevBuf<int> t;
-        t.alloc(n);
-        launch_to_ref(c, dev, t.p, 4);
-        HIP_OK(hipMemcpyAsync(host, t.p, 4 * n, hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipStreamSynchronize(c->stream));
-    } else {
-        DevBuf<double> t;
-        t.alloc(n);
-        launch_to_ref(c, dev, t.p, 8);
-        HIP_OK(hipMemcpyAsync(host, t.p, 8 * n, hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipStreamSynchronize(c->stream));
-    }
+    std::lock_guard<std::mutex> lk(c->ref_mu);
+    c->ref.alloc(n);
+    launch_to_ref(c, dev, c->ref.p, eb);
+    copy_to_host(c, host, c->ref.p, n * eb, c->stream);
 }
 
 int igr_set_demand(igr_ctx* c, const float* demand) {
     return guard([&]() {
-        DevBuf<float> t;
-        t.upload(demand, c->cells(), c->stream);
-        launch_from_ref(c, t.p, c->demand.p, 4);
+        std::lock_guard<std::mutex> lk(c->ref_mu);
+        c->ref.alloc(c->cells());
+        copy_to_device(c, c->ref.p, demand, 4 * c->cells(), c->stream);
+        launch_from_ref(c, c->ref.p, c->demand.p, 4);
         HIP_OK(hipStreamSynchronize(c->stream));
     });
 }
@@ -186,7 +178,6 @@ __global__ void k_route_starts(const int64_t* route_off, int64_t n, int* routes)
     if (i < n) routes[route_off[i]] = 1;
 }
 
-int host_threads() { return std::max(1, std::min(16, (int)std::thread::hardware_concurrency())); }
 } // namespace
 
 int igr_set_nets(igr_ctx* c, const igr_net_desc* d) {
@@ -566,8 +557,7 @@ int igr_get_routes(igr_ctx* c, int64_t* off, int* data, int64_t cap) {
         doff.upload(o.data(), n + 1, c->stream);
         out.alloc(o[n]);
         gather_routes(c, doff.p, out.p);
-        HIP_OK(hipMemcpyAsync(data, out.p, sizeof(int) * o[n], hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipStreamSynchronize(c->stream));
+        copy_to_host(c, data, out.p, sizeof(int) * o[n], c->stream);
         std::memcpy(off, o.data(), sizeof(int64_t) * (n + 1));
     });
 }
@@ -650,7 +640,7 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     hipStream_t s = c->stream;
     const double t0 = now_s();
     D.pt_off.upload(dg->pt_off, n + 1, s);
-    D.pt.upload(dg->pts, dg->pt_off[n], s);
+    upload(c, D.pt, dg->pts, dg->pt_off[n], s);
 
     int64_t NN = 0, NE = 0;
     std::vector<double> l_eb, l_db;   // kernel timing only: algorithmic bytes of the DAG kernels, list order
@@ -672,14 +662,14 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
             NE = dg->par_off[NN];
             if (NE < 0) throw std::invalid_argument("malformed DAG (edge offsets, depths or slot counts)");
             hipStream_t cs = c->copy_stream;
-            D.r_node_off.upload(dg->node_off, n + 1, cs);
-            D.r_par_off.upload(dg->par_off, NN + 1, cs);
-            D.r_child_num.upload(dg->child_num, NN, cs);
-            D.r_depth.upload(dg->depth, NN, cs);
+            upload(c, D.r_node_off, dg->node_off, n + 1, cs);
+            upload(c, D.r_par_off, dg->par_off, NN + 1, cs);
+            upload(c, D.r_child_num, dg->child_num, NN, cs);
+            upload(c, D.r_depth, dg->depth, NN, cs);
             launch_dag_measure(c, n, NE, cs);
-            D.r_nodes.upload(dg->nodes, NN, cs);
-            D.r_par.upload(dg->par, NE, cs);
-            D.r_slot.upload(dg->slot, NE, cs);
+            upload(c, D.r_nodes, dg->nodes, NN, cs);
+            upload(c, D.r_par, dg->par, NE, cs);
+            upload(c, D.r_slot, dg->slot, NE, cs);
             int err = 0;
             HIP_OK(hipMemcpyAsync(&err, D.err.p, sizeof(int), hipMemcpyDeviceToHost, cs));
             HIP_OK(hipStreamSynchronize(cs));
@@ -791,9 +781,7 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     D.cost_edges.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
     D.change.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
     NetsDev& N = c->nets;
-    N.dag_routes.push_back(new DevBuf<int>());
-    N.dag_routes.back()->alloc(dag_route_slot(NN, n));
-    int* rbase = N.dag_routes.back()->p;
+    int* rbase = N.new_dag_routes(dag_route_slot(NN, n));
     const double tp = now_s();
 
     // Batch b: DAG routing (scattering its wires, vias and dirty flags), the
@@ -1057,9 +1045,7 @@ int igr_dag_pass(igr_ctx* c, const int* nets, int64_t n, int mode, int form, con
         D.cost_edges.alloc(std::max<int64_t>(1, mx_edges) * LL);
         D.best_change.alloc(std::max<int64_t>(1, mx_edges) * LL);
         NetsDev& N = c->nets;
-        N.dag_routes.push_back(new DevBuf<int>());
-        N.dag_routes.back()->alloc(route_slot[n]);
-        int* rbase = N.dag_routes.back()->p;
+        int* rbase = N.new_dag_routes(route_slot[n]);
         double tp = now_s();
 
         double t_note = tp;
@@ -1134,9 +1120,8 @@ int igr_congestion_view(igr_ctx* c, float* xsum, float* ysum) {
         c->scratch.xsum.alloc(q);
         c->scratch.ysum.alloc(q);
         launch_congestion(c, c->scratch.xsum.p, c->scratch.ysum.p);
-        HIP_OK(hipMemcpyAsync(xsum, c->scratch.xsum.p, 4 * q, hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipMemcpyAsync(ysum, c->scratch.ysum.p, 4 * q, hipMemcpyDeviceToHost, c->stream));
-        HIP_OK(hipStreamSynchronize(c->stream));
+        copy_to_host(c, xsum, c->scratch.xsum.p, 4 * q, c->stream);
+        copy_to_host(c, ysum, c->scratch.ysum.p, 4 * q, c->stream);
     });
 }
 

@@ -66,11 +66,26 @@ struct Mailbox {
     }
 };
 
+// Pinned slots for large copies to and from pageable memory (staging.hip): 16
+// MiB a context, allocated by its first large copy.  'mu' lets one copy at a
+// time use them; done[k] is the last copy through slot k.
+struct Staging {
+    static constexpr int SLOTS = 8, THREADS = 4;
+    static constexpr int64_t SLOT_BYTES = 2 << 20, MIN_BYTES = 1 << 20;
+    std::mutex mu;
+    char* mem = nullptr;
+    hipEvent_t done[SLOTS] = {};
+    ~Staging();
+    void open();
+    char* slot(int k) { return mem + k * SLOT_BYTES; }
+};
+
 // Net trees and footprints on the device (pattern pass).  Every net's current
 // route is reached through rptr[net]: pattern routes live in 'routes' at
 // route_off[net]; a rip-up-and-reroute pass moves the nets it reroutes to a
 // buffer of its own (dag_routes).
 struct NetsDev {
+    static constexpr size_t SPARE_WORDS = 16 << 20;   // 64 MiB: what a context may hold back
     int64_t n = 0;
     DevBuf<int64_t> node_off, route_off, pt_off, hs_off, vs_off;
     DevBuf<int> node, parent, routes, pt, hs, vs;
@@ -84,8 +99,23 @@ struct NetsDev {
     std::vector<int64_t> dag_live;          // nets whose route lives in dag_routes[k]
     std::vector<int> h_rbuf;                // per net: its dag_routes buffer, -1 = pattern slot
     int max_nodes = 0;
+    DevBuf<int>* spare = nullptr;           // one retired buffer, for a next pass of about its size
     ~NetsDev() { clear_dag_routes(); }
+    // The routes buffer of a new pass.
+    int* new_dag_routes(int64_t words) {
+        const bool fits = spare && (int64_t)spare->n >= words && (int64_t)spare->n / 4 <= words;
+        dag_routes.push_back(fits ? spare : new DevBuf<int>());
+        if (fits) spare = nullptr;
+        dag_routes.back()->alloc(words);
+        return dag_routes.back()->p;
+    }
+    void retire(DevBuf<int>* b) {
+        if (!spare && b->n <= SPARE_WORDS) spare = b;
+        else delete b;
+    }
     void clear_dag_routes() {
+        delete spare;
+        spare = nullptr;
         for (auto* b : dag_routes) delete b;
         dag_routes.clear();
         dag_live.clear();
@@ -98,7 +128,7 @@ struct NetsDev {
         if (k < 0) return;
         h_rbuf[net] = -1;
         if (--dag_live[k] == 0) {
-            delete dag_routes[k];
+            retire(dag_routes[k]);
             dag_routes[k] = nullptr;
         }
     }
@@ -124,7 +154,7 @@ struct NetsDev {
             for (size_t j = 0; j < v.size(); j++) dag_live[j] -= v[j];
         for (size_t j = 0; j < dag_routes.size(); j++)
             if (dag_routes[j] && dag_live[j] == 0) {
-                delete dag_routes[j];
+                retire(dag_routes[j]);
                 dag_routes[j] = nullptr;
             }
     }
@@ -140,6 +170,10 @@ struct Sched {
     DevBuf<unsigned long long> stat;
     DevBuf<uint8_t> sn;           // the nets' records
     DevBuf<int> bits;             // per-net state bits (assigned, blocked in this batch)
+    int* h_ctrl = nullptr;        // pinned copy of 'ctrl'
+    ~Sched() {
+        if (h_ctrl) (void)hipHostFree(h_ctrl);
+    }
 };
 
 // Batched form: the records of a DAG's nodes and parent edges, by depth level
@@ -304,6 +338,9 @@ struct igr_ctx {
     igr_dev::DagDev dag;
     igr_dev::OrderDev order;
     igr_dev::Mailbox mail;
+    igr_dev::Staging staging;
+    std::mutex ref_mu;
+    igr_dev::DevBuf<double> ref;   // a grid array in the callers' order, on its way in or out (ref_mu)
     int stamp = 0;
     igr_tuning tune{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // launch-shape overrides (0 = built-in)
     double last_dag_prep_s = 0;   // host preparation time of the last DAG pass
@@ -449,6 +486,16 @@ void launch_dag_order(igr_ctx* c, const int* d_nets, int64_t n, int nb, bool dee
 // the context's mailbox, after all work on the stream; returns its host address.
 // Needs c->mail.mu.
 const int* read_route(igr_ctx* c, const int* src, int64_t rc);
+inline int host_threads() { return std::max(1, std::min(16, (int)std::thread::hardware_concurrency())); }
+// Copies between the device and pageable memory, after all work on the stream.
+// To the host: done on return.  To the device: 'src' is free on return.
+void copy_to_host(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipStream_t s);
+void copy_to_device(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipStream_t s);
+template <class T>
+void upload(igr_ctx* c, DevBuf<T>& b, const T* h, int64_t count, hipStream_t s) {
+    b.alloc(count);
+    copy_to_device(c, b.p, h, count * (int64_t)sizeof(T), s);
+}
 // off[i] = cnt[0] + .. + cnt[i - 1], off[n] the total (n > 0).
 void launch_exclusive_scan(igr_ctx* c, const int* cnt, int64_t n, int64_t* off);
 // Batched form: the device layout of a pass's DAGs.

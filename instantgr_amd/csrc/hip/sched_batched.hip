@@ -1257,56 +1257,50 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     const unsigned wgrid = (unsigned)std::min<int64_t>(1024, std::max<int64_t>(16, n / 64));
     const unsigned cgrid = (wgrid + 3) / 4;
     const unsigned gm = (unsigned)std::min<int64_t>(512, (std::max(XYc, n) + LTPB - 1) / LTPB);   // grid-stride
-    int* h_ctrl = nullptr;
-    HIP_OK(hipHostMalloc(&h_ctrl, sizeof(int) * (2 * C_WORDS + 1)));
+    if (!S.h_ctrl) HIP_OK(hipHostMalloc(&S.h_ctrl, sizeof(int) * (2 * C_WORDS + 1)));
+    int* h_ctrl = S.h_ctrl;
     const int64_t max_rounds = (int64_t)ROUNDS * (n + 1) + CHUNK;
     int64_t g = 0;
     const auto t_start = std::chrono::steady_clock::now();
     auto t_note = t_start;
-    try {
-        for (;;) {
-            if (g > max_rounds) throw std::runtime_error("scheduler did not finish");
-            const auto t_now = std::chrono::steady_clock::now();
-            if (std::chrono::duration<double>(t_now - t_note).count() > 20) {
-                t_note = t_now;
-                progress("scheduler: %d batches after %.1f s", h_ctrl[(g & 1) * C_WORDS + C_CUR],
-                         std::chrono::duration<double>(t_now - t_start).count());
-            }
-            auto round = [&](auto gv) {
-                constexpr int GV = decltype(gv)::value;
-                if (release) {
-                    k_r_claim<GV><<<vgrid, LTPB, 0, st>>>(a, g);
-                    k_r_viable<GV><<<vgrid, LTPB, 0, st>>>(a, g, S.viable.p);
-                    k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
-                    k_r_commit<<<cgrid, LTPB, 0, st>>>(a, g, S.viable.p);
-                    k_r_block<64><<<ggrid, TPB, 0, st>>>(a, g);
-                    k_r_clear_end<<<gm, LTPB, 0, st>>>(a, g, XYc);
-                    return;
-                }
-                k_a_claim<GV><<<ggrid, TPB, 0, st>>>(a, g);
-                k_a_viable<GV><<<vgrid, LTPB, 0, st>>>(a, g, S.viable.p);
-                k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
-                k_a_commit<<<cgrid, LTPB, 0, st>>>(a, g, S.viable.p);
-                k_a_revert<GV><<<ggrid, TPB, 0, st>>>(a, g);
-                k_a_clear_end<<<gm, LTPB, 0, st>>>(a, g, XYc);
-            };
-            for (int r = 0; r < CHUNK; r++, g++) {
-                if (G == 4) round(std::integral_constant<int, 4>{});
-                else if (G == 8) round(std::integral_constant<int, 8>{});
-                else round(std::integral_constant<int, 16>{});
-            }
-            HIP_OK(hipGetLastError());
-            HIP_OK(hipMemcpyAsync(h_ctrl, S.ctrl.p, sizeof(int) * (2 * C_WORDS + 1), hipMemcpyDeviceToHost, st));
-            HIP_OK(hipStreamSynchronize(st));
-            if (h_ctrl[(g & 1) * C_WORDS + C_DONE]) break;
+    for (;;) {
+        if (g > max_rounds) throw std::runtime_error("scheduler did not finish");
+        const auto t_now = std::chrono::steady_clock::now();
+        if (std::chrono::duration<double>(t_now - t_note).count() > 20) {
+            t_note = t_now;
+            progress("scheduler: %d batches after %.1f s", h_ctrl[(g & 1) * C_WORDS + C_CUR],
+                     std::chrono::duration<double>(t_now - t_start).count());
         }
-    } catch (...) {
-        (void)hipHostFree(h_ctrl);
-        throw;
+        auto round = [&](auto gv) {
+            constexpr int GV = decltype(gv)::value;
+            if (release) {
+                k_r_claim<GV><<<vgrid, LTPB, 0, st>>>(a, g);
+                k_r_viable<GV><<<vgrid, LTPB, 0, st>>>(a, g, S.viable.p);
+                k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
+                k_r_commit<<<cgrid, LTPB, 0, st>>>(a, g, S.viable.p);
+                k_r_block<64><<<ggrid, TPB, 0, st>>>(a, g);
+                k_r_clear_end<<<gm, LTPB, 0, st>>>(a, g, XYc);
+                return;
+            }
+            k_a_claim<GV><<<ggrid, TPB, 0, st>>>(a, g);
+            k_a_viable<GV><<<vgrid, LTPB, 0, st>>>(a, g, S.viable.p);
+            k_b_claim_rest<<<wgrid, TPB, 0, st>>>(a, g, S.viable.p);
+            k_a_commit<<<cgrid, LTPB, 0, st>>>(a, g, S.viable.p);
+            k_a_revert<GV><<<ggrid, TPB, 0, st>>>(a, g);
+            k_a_clear_end<<<gm, LTPB, 0, st>>>(a, g, XYc);
+        };
+        for (int r = 0; r < CHUNK; r++, g++) {
+            if (G == 4) round(std::integral_constant<int, 4>{});
+            else if (G == 8) round(std::integral_constant<int, 8>{});
+            else round(std::integral_constant<int, 16>{});
+        }
+        HIP_OK(hipGetLastError());
+        HIP_OK(hipMemcpyAsync(h_ctrl, S.ctrl.p, sizeof(int) * (2 * C_WORDS + 1), hipMemcpyDeviceToHost, st));
+        HIP_OK(hipStreamSynchronize(st));
+        if (h_ctrl[(g & 1) * C_WORDS + C_DONE]) break;
     }
     const int nbatch = h_ctrl[(g & 1) * C_WORDS + C_CUR];
     const int64_t placed = h_ctrl[2 * C_WORDS];
-    HIP_OK(hipHostFree(h_ctrl));
     if (a.bytes) {
         std::vector<unsigned long long> slots(BYTE_SLOTS);
         HIP_OK(hipMemcpyAsync(slots.data(), a.bytes, sizeof(unsigned long long) * BYTE_SLOTS, hipMemcpyDeviceToHost,

@@ -100,6 +100,9 @@ struct igr_server {
     std::string fail_msg;
     igr_server_stats st{};
     std::thread worker;
+    // the worker's buffers, kept from tick to tick
+    std::vector<float> xs, ys;
+    DevBuf<int> d_nets, d_box;
 
     void run();
     void tick(std::vector<std::shared_ptr<Request>>& cand);
@@ -112,7 +115,8 @@ void igr_server::tick(std::vector<std::shared_ptr<Request>>& cand) {
     const int TX = (X + TILE - 1) / TILE, TY = (Y + TILE - 1) / TILE;
     const double t0 = now_s();
     // 1-2. view and DAGs of every candidate's nets, in candidate order
-    std::vector<float> xs((size_t)XY), ys((size_t)XY);
+    xs.resize((size_t)XY);
+    ys.resize((size_t)XY);
     int rc = igr_congestion_view(c, xs.data(), ys.data());
     if (rc) throw std::runtime_error(std::string("congestion view: ") + igr_last_error());
     std::vector<int> all;
@@ -127,7 +131,6 @@ void igr_server::tick(std::vector<std::shared_ptr<Request>>& cand) {
     // current route boxes
     std::vector<int> box((size_t)(4 * std::max<int64_t>(1, na)));
     {
-        DevBuf<int> d_nets, d_box;
         d_nets.upload(all.data(), na, c->stream);
         d_box.alloc(4 * std::max<int64_t>(1, na));
         k_route_bbox<<<(unsigned)((na + TPB - 1) / TPB), TPB, 0, c->stream>>>(d_nets.p, na, c->nets.rptr.p, XY, Y,
