@@ -73,9 +73,10 @@ constexpr int64_t SCHED_RELEASE_NETS = 150000, SCHED_RELEASE_LIST = 25;
 // v0); C_NR, cells the previous round released (list rel); C_NK, new owners
 // of those cells (list cand); C_NC, nets committed in this round;
 // C_NH, cells those nets own (list hits).
-// C_LASTC, nets placed when the lists were last compacted.
+// C_LASTC, nets placed when the lists were last compacted.  C_LEFT (active-list
+// rounds): some net of the active list is still active after the round.
 enum { C_DONE = 0, C_CUR, C_ROUND, C_COMMIT, C_HAVE, C_NVIABLE, C_NU, C_UL, C_NA, C_AL, C_NR, C_NK, C_NC, C_NH,
-       C_NV0, C_LASTC, C_WORDS };
+       C_NV0, C_LASTC, C_LEFT, C_WORDS };
 constexpr int NLISTS = 3;         // net list buffers of n entries each
 constexpr int COMPACT_DIV = 64;   // release-driven rounds: compact the cell lists every n/64 placed nets
 
@@ -84,6 +85,12 @@ constexpr int COMPACT_DIV = 64;   // release-driven rounds: compact the cell lis
 struct alignas(16) SNet {
     int64_t pt0;
     int npt, pad;
+};
+// An entry of the active-list rounds' net lists: the net with its points, so
+// that a round's kernels read a list and then points, not a record between.
+struct alignas(16) ANet {
+    int i, npt;
+    int64_t pt0;
 };
 // Its segments, read beside it by the kernels that walk a net's rest cells.
 struct alignas(8) SSeg {
@@ -106,7 +113,8 @@ struct BArgs {
     int64_t* head;                // X*Y first unassigned entry of each list
     int* batch;
     int* ctrl;
-    int* lists;                   // NLISTS buffers of n net indices
+    int* lists;                   // release-driven rounds: NLISTS buffers of n net indices
+    ANet* alists;                 // active-list rounds: NLISTS buffers of n nets
     // release-driven rounds only
     int* rel;                     // X*Y cells released by the previous round
     int* cand;                    // nets that took a released cell this round
@@ -160,9 +168,9 @@ __device__ __forceinline__ void set_blocked(const BArgs& a, int64_t i) {
 constexpr uint32_t NST_ASSIGNED = 0x55555555u;
 
 // Active-list rounds: the batch's active list of the round whose state is st.
-__device__ __forceinline__ const int* a_list(const BArgs& a, const int* st, int64_t& na) {
+__device__ __forceinline__ const ANet* a_list(const BArgs& a, const int* st, int64_t& na) {
     na = st[C_NA] < 0 ? st[C_NU] : st[C_NA];
-    return a.lists + (int64_t)st[C_AL] * a.n;
+    return a.alists + (int64_t)st[C_AL] * a.n;
 }
 
 // Release-driven rounds: the nets whose viability the round whose state is st
@@ -313,7 +321,8 @@ __device__ __forceinline__ uint64_t group_bits(uint64_t m, int G) {
 // Appends v to list for every thread with want, one counter atomic per
 // workgroup (a returning atomic per wave on one counter serialises thousands
 // of waves).  Every thread of the workgroup calls it; s holds LTPB/64+1 ints.
-__device__ __forceinline__ void block_append(bool want, int v, int* counter, int* list, int* s) {
+template <class T>
+__device__ __forceinline__ void block_append(bool want, const T& v, int* counter, T* list, int* s) {
     constexpr int NW = LTPB / 64;
     const uint64_t m = __ballot(want);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -509,15 +518,14 @@ __global__ void __launch_bounds__(TPB) k_a_claim(BArgs a, int64_t g) {
     const int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE] || st[C_ROUND] == 0) return;
     int64_t na;
-    const int* al = a_list(a, st, na);
+    const ANet* al = a_list(a, st, na);
     const int64_t nth = (int64_t)gridDim.x * TPB / G;
     const int lg = threadIdx.x & (G - 1);
     for (int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G; t < na; t += nth) {
-        const int64_t i = al[t];
-        const SNet s = a.sn[i];   // every listed net is active
+        const ANet s = al[t];   // every listed net is active
         for (int k = lg; k < s.npt; k += G) {
             int* m = &a.map[a.pt[s.pt0 + k]];
-            if (*m < (int)i) atomicMax(m, (int)i);
+            if (*m < s.i) atomicMax(m, s.i);
         }
     }
 }
@@ -537,22 +545,21 @@ __global__ void __launch_bounds__(LTPB) k_a_viable(BArgs a, int64_t g, int* vlis
         nx[C_NU] = 0;
     }
     int64_t na;
-    const int* al = a_list(a, st, na);
+    const ANet* al = a_list(a, st, na);
     const int64_t nth = (int64_t)gridDim.x * LTPB / G;
     const int lg = threadIdx.x & (G - 1);
     const int64_t rounds = (na + nth - 1) / nth;   // the same for every lane of the wave
     for (int64_t r = 0; r < rounds; r++) {
         const int64_t t = ((int64_t)blockIdx.x * LTPB + threadIdx.x) / G + r * nth;
-        const int64_t i = t < na ? al[t] : 0;
         const bool live = t < na;   // every listed net is active
-        const SNet s = live ? a.sn[i] : SNet{0, 0, 0};
+        const ANet s = live ? al[t] : ANet{0, 0, 0};
         bool fail = !live;
         for (int k = lg;; k += G) {
-            const bool f = !fail && k < s.npt && a.map[a.pt[s.pt0 + k]] != (int)i;
+            const bool f = !fail && k < s.npt && a.map[a.pt[s.pt0 + k]] != s.i;
             fail = fail || group_bits(__ballot(f), G) != 0;
             if (__ballot(!fail && k + G < s.npt) == 0) break;
         }
-        gl.add(lg == 0 && !fail, (int)i);
+        gl.add(lg == 0 && !fail, s.i);
     }
     gl.flush();
 }
@@ -585,18 +592,18 @@ __global__ void __launch_bounds__(LTPB) k_a_commit(BArgs a, int64_t g, const int
 //    sit out the batch
 template <int G>
 __global__ void __launch_bounds__(TPB) k_a_revert(BArgs a, int64_t g) {
-    const int* st = a.ctrl + (g & 1) * C_WORDS;
+    int* st = a.ctrl + (g & 1) * C_WORDS;
     if (st[C_DONE] || !st[C_COMMIT]) return;
     int64_t na;
-    const int* al = a_list(a, st, na);
+    const ANet* al = a_list(a, st, na);
     const int64_t nth = (int64_t)gridDim.x * TPB / G;
     const int lg = threadIdx.x & (G - 1);
     const int64_t rounds = (na + nth - 1) / nth;
+    bool left = false;
     for (int64_t r = 0; r < rounds; r++) {
         const int64_t t = ((int64_t)blockIdx.x * TPB + threadIdx.x) / G + r * nth;
-        const int64_t i = t < na ? al[t] : 0;
-        SNet s = t < na ? a.sn[i] : SNet{0, 0, 0};
-        const bool live = t < na && !assigned(a, i);
+        ANet s = t < na ? al[t] : ANet{0, 0, 0};
+        const bool live = t < na && !assigned(a, s.i);
         if (!live) s.npt = 0;
         bool hit = false;
         for (int k = lg;; k += G) {
@@ -608,14 +615,16 @@ __global__ void __launch_bounds__(TPB) k_a_revert(BArgs a, int64_t g) {
             hit = hit || group_bits(__ballot(h), G) != 0;
             if (__ballot(!hit && k + G < s.npt) == 0) break;
         }
-        if (lg == 0 && live && hit) {
-            set_blocked(a, i);
-        }
+        if (lg == 0 && live && hit) set_blocked(a, s.i);
+        left = left || (live && !hit);
     }
+    if (__ballot(left) != 0 && (threadIdx.x & 63) == 0) st[C_LEFT] = 1;
 }
 
-// 6. end of the round.  The batch goes on after a commit below the round
-//    limit: cells of blocked nets are released.  Otherwise the batch ends:
+// 6. end of the round.  The batch goes on after a commit that left active
+//    nets, below the round limit: cells of blocked nets are released.
+//    Otherwise the batch ends (without active nets the next round would commit
+//    nothing and end it; that round's six kernels took 17 us):
 //    each cell's list moves past assigned nets, the next batch starts from
 //    the kept map with every unassigned net active.  The successor lists go
 //    to a buffer neither current list uses.  Thread 0 writes the successor
@@ -629,10 +638,10 @@ __global__ void __launch_bounds__(LTPB) k_a_clear_end(BArgs a, int64_t g, int64_
     const bool done = st[C_DONE] != 0;
     const bool commit = st[C_COMMIT] != 0;
     const int round = st[C_ROUND];
-    const bool end = !commit || round + 1 >= ROUNDS;
+    const bool end = !commit || !st[C_LEFT] || round + 1 >= ROUNDS;
     int fresh = 0;   // the first list buffer neither current list uses
     while (fresh == st[C_AL] || fresh == st[C_UL]) fresh++;
-    int* nl = a.lists + (int64_t)fresh * a.n;
+    ANet* nl = a.alists + (int64_t)fresh * a.n;
     if (!done) {
         if (end) {
             for (int64_t q = t; q < cells; q += stride) {
@@ -644,13 +653,12 @@ __global__ void __launch_bounds__(LTPB) k_a_clear_end(BArgs a, int64_t g, int64_
                 a.base[q] = b;
                 a.map[q] = b;
             }
-            const int* ul = a.lists + (int64_t)st[C_UL] * a.n;
+            const ANet* ul = a.alists + (int64_t)st[C_UL] * a.n;
             const int64_t nu = st[C_NU], passes = (nu + stride - 1) / stride;   // the same for every thread
             for (int64_t ps = 0; ps < passes; ps++) {
                 const int64_t u = ps * stride + t;
-                const int i = u < nu ? ul[u] : 0;
-                const bool left = u < nu && !assigned(a, i);
-                block_append(left, i, &nx[C_NU], nl, s_app);
+                const ANet s = u < nu ? ul[u] : ANet{0, 0, 0};
+                block_append(u < nu && !assigned(a, s.i), s, &nx[C_NU], nl, s_app);
             }
             // every unassigned net is active again in the next batch
             for (int64_t w = t; w < a.nwords; w += stride) a.nst[w] &= NST_ASSIGNED;
@@ -660,12 +668,12 @@ __global__ void __launch_bounds__(LTPB) k_a_clear_end(BArgs a, int64_t g, int64_
                 if (m >= 0 && blocked(a, m)) a.map[q] = -1;
             }
             int64_t na;
-            const int* al = a_list(a, st, na);
+            const ANet* al = a_list(a, st, na);
             const int64_t passes = (na + stride - 1) / stride;   // the same for every thread
             for (int64_t ps = 0; ps < passes; ps++) {
                 const int64_t u = ps * stride + t;
-                const int i = u < na ? al[u] : 0;
-                block_append(u < na && active(a, i), i, &nx[C_NA], nl, s_app);
+                const ANet s = u < na ? al[u] : ANet{0, 0, 0};
+                block_append(u < na && active(a, s.i), s, &nx[C_NA], nl, s_app);
             }
         }
     }
@@ -707,6 +715,8 @@ __global__ void __launch_bounds__(LTPB) k_a_clear_end(BArgs a, int64_t g, int64_
         nx[C_ROUND] = r;
         nx[C_HAVE] = have;
         nx[C_COMMIT] = 0;
+        nx[C_LEFT] = 0;
+        nx[C_NC] = 0;
         nx[C_NVIABLE] = 0;
         if (done) {
             nx[C_NA] = st[C_NA];
@@ -1148,7 +1158,8 @@ __global__ void k_nets(int64_t n, const int* order, const int64_t* pt_off, bool 
 __global__ void k_start(BArgs a) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i < a.n) {
-        a.lists[i] = (int)i;
+        if (a.alists) a.alists[i] = ANet{(int)i, a.sn[i].npt, a.sn[i].pt0};
+        else a.lists[i] = (int)i;
         a.batch[i] = -1;
     }
     if (i == 0) {
@@ -1196,7 +1207,6 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     S.cnt.zero(XYc, st);
     S.batch.alloc(n);
     S.viable.alloc(n);
-    S.lists.alloc(NLISTS * n);
     S.stat.zero(3, st);
     S.ctrl.zero(2 * C_WORDS + 1, st);
     const int64_t nwords = (n + 15) / 16;
@@ -1210,7 +1220,9 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     S.c_net.alloc(std::max<int64_t>(1, entries));
     const bool release = c->tune.sched_kind ? c->tune.sched_kind == 2
                                             : n >= SCHED_RELEASE_NETS && entries >= SCHED_RELEASE_LIST * XYc;
+    if (!release) S.alists.alloc(sizeof(ANet) * NLISTS * (size_t)n);
     if (release) {
+        S.lists.alloc(NLISTS * n);
         S.rel.alloc(XYc);
         S.cand.alloc(n);
         S.cstamp.zero(n, st);
@@ -1219,7 +1231,7 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         S.cur.alloc(XYc);
     }
     BArgs a{n, sn, sg, d_pt_off ? d_pt : N.pt.p, N.hs.p, N.vs.p, S.map.p, S.base.p, S.c_off.p, S.c_end.p, S.c_net.p, S.head.p,
-            S.batch.p, S.ctrl.p, S.lists.p,
+            S.batch.p, S.ctrl.p, S.lists.p, release ? nullptr : reinterpret_cast<ANet*>(S.alists.p),
             release ? S.rel.p : nullptr, release ? S.cand.p : nullptr, release ? S.cstamp.p : nullptr,
             release ? S.lists.p + 2 * n : nullptr,
             release ? S.hits.p : nullptr, release ? S.hstamp.p : nullptr,
