@@ -168,6 +168,8 @@ struct Sched {
     DevBuf<int> base, cnt, c_net, ctrl, lists, rel, cand, cstamp, hits, hstamp;
     DevBuf<int64_t> head, c_off, c_end, bsum, cur;
     DevBuf<unsigned long long> stat;
+    DevBuf<uint8_t> small;        // one-workgroup rounds: the nets left and their points' slots
+    DevBuf<int> slot;             // X*Y slot of a cell in their map, or -1
     DevBuf<uint8_t> sn, alists;   // the nets' records; active-list rounds: their lists
     DevBuf<int> bits;             // per-net state bits (assigned, blocked in this batch)
     int* h_ctrl = nullptr;        // pinned copy of 'ctrl'

@@ -31,6 +31,8 @@
 //      per round follows the released cells and committed nets.
 //    On a 640k-cell grid with 0.5M nets the active-list rounds cost less; on a
 //    2.25M-cell grid with 3M-10M nets the release-driven ones do.
+//  * Short lists, and the last batches of long ones, run in one workgroup
+//    (k_small_rounds) unless the tuning asks for a kind of rounds.
 //  * List orders are free: every decision is an atomic maximum or a test
 //    against the map.
 //  * The round and batch control lives in a device word block; the host
@@ -115,6 +117,7 @@ struct BArgs {
     int* ctrl;
     int* lists;                   // release-driven rounds: NLISTS buffers of n net indices
     ANet* alists;                 // active-list rounds: NLISTS buffers of n nets
+    int small_at;                 // a batch that leaves this many nets or fewer stops the rounds (C_DONE 2)
     // release-driven rounds only
     int* rel;                     // X*Y cells released by the previous round
     int* cand;                    // nets that took a released cell this round
@@ -411,16 +414,16 @@ struct GroupList {
 
 // Calls f(valid, q) with U cells per lane at a time, over the sampled cells of
 // a net's segments (every sparsity-th cell from each segment's start,
-// src/database_cuda.hpp:320-352), the cells of up to 64 segments at a time
-// spread evenly over the wave's lanes (a lane per segment would walk a long
-// segment alone).  Every lane of the wave calls it together; valid is false on
-// the lanes past the last cell, and f may use ballots.
-template <int U, class F>
-__device__ __forceinline__ void wave_segment_cells(const BArgs& a, const SSeg& g, F f) {
-    const int lane = threadIdx.x & 63;
+// src/database_cuda.hpp:320-352), the cells of up to W segments at a time
+// spread evenly over the W lanes of the net's group (a lane per segment would
+// walk a long segment alone).  Every lane of the wave calls it together; valid
+// is false on the lanes past the last cell, and f may use ballots.
+template <int W, int U, class F>
+__device__ __forceinline__ void group_segment_cells(const BArgs& a, const SSeg& g, F f) {
+    const int lane = threadIdx.x & (W - 1);
     const int Y = a.Y, sp = a.sparsity;
     const int ns = g.nh + g.nv;
-    for (int sb = 0; sb < ns; sb += 64) {
+    for (int sb = 0; __ballot(sb < ns); sb += W) {
         const int k = sb + lane;
         int cnt = 0, first = 0, step = 0;
         if (k < ns) {
@@ -434,28 +437,32 @@ __device__ __forceinline__ void wave_segment_cells(const BArgs& a, const SSeg& g
             step = hor ? sp * Y : sp;
         }
         int incl = cnt;                  // inclusive scan of the cell counts
-        for (int d = 1; d < 64; d <<= 1) {
-            const int v = __shfl_up(incl, d);
+        for (int d = 1; d < W; d <<= 1) {
+            const int v = __shfl_up(incl, d, W);
             if (lane >= d) incl += v;
         }
-        const int total = __shfl(incl, 63);
+        const int total = __shfl(incl, W - 1, W);
         const int excl = incl - cnt;
-        for (int cb = 0; cb < total; cb += 64 * U) {
+        for (int cb = 0; __ballot(cb < total); cb += W * U) {
             bool valid[U];
             int q[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const int c = cb + 64 * u + lane;
+                const int c = cb + W * u + lane;
                 int sg = 0;              // the first lane whose inclusive count exceeds c
-                for (int b2 = 32; b2 > 0; b2 >>= 1)
-                    if (__shfl(incl, sg + b2 - 1) <= c) sg += b2;
-                const int f0 = __shfl(first, sg), st0 = __shfl(step, sg), ex = __shfl(excl, sg);
+                for (int b2 = W / 2; b2 > 0; b2 >>= 1)
+                    if (__shfl(incl, sg + b2 - 1, W) <= c) sg += b2;
+                const int f0 = __shfl(first, sg, W), st0 = __shfl(step, sg, W), ex = __shfl(excl, sg, W);
                 valid[u] = c < total;
                 q[u] = valid[u] ? f0 + (c - ex) * st0 : 0;
             }
             f(valid, q);
         }
     }
+}
+template <int U, class F>
+__device__ __forceinline__ void wave_segment_cells(const BArgs& a, const SSeg& g, F f) {
+    group_segment_cells<64, U>(a, g, f);
 }
 
 // The neighbour cells (0,-1), (-1,0), (1,0) of a point.
@@ -707,7 +714,8 @@ __global__ void __launch_bounds__(LTPB) k_a_clear_end(BArgs a, int64_t g, int64_
                 cur += 1;
                 r = 0;
                 have = 0;
-                if ((int64_t)a.ctrl[2 * C_WORDS] == a.n) d = 1;
+                const int64_t rest = a.n - a.ctrl[2 * C_WORDS];
+                d = rest == 0 ? 1 : rest <= a.small_at ? 2 : 0;
             }
         }
         nx[C_DONE] = d;
@@ -1110,7 +1118,8 @@ __global__ void __launch_bounds__(LTPB) k_r_clear_end(BArgs a, int64_t g, int64_
                 cur += 1;
                 r = 0;
                 have = 0;
-                if ((int64_t)a.ctrl[2 * C_WORDS] == a.n) d = 1;
+                const int64_t rest = a.n - a.ctrl[2 * C_WORDS];
+                d = rest == 0 ? 1 : rest <= a.small_at ? 2 : 0;
             }
         }
         nx[C_DONE] = d;
@@ -1138,6 +1147,339 @@ __global__ void __launch_bounds__(LTPB) k_r_clear_end(BArgs a, int64_t g, int64_
         }
     }
     flush_bytes(a, nb);
+}
+
+// ---- few nets: all rounds in one workgroup ----------------------------------
+// With few nets left a round's six kernels are launches and load chains (26 us
+// whatever they do).  Here one workgroup runs the remaining batches with the
+// owner map in LDS.  Only the point cells of the nets left can decide
+// anything, so the map has a slot per such cell: k_small_mark leaves at each
+// one of its points' positions in the list of all of them (any one serves),
+// and the points that find their own number there take the slots.  The points'
+// slots follow the map in LDS.  Owners are
+// ranks in the nets' order, which keeps the priorities.  The rounds are the active-list rounds: point
+// claims, viability, the viable nets' neighbour and segment claims, commits,
+// block, release.  Bound by one CU's instruction issue: a pass over a batch's
+// first 1000 nets of 33 points takes some 3 us, a late round 3 us in all, so
+// beyond 2000 nets the kernels win (pattern pass of 20k nets with its last 512,
+// 1024, 2048, 4096 nets here: 8.3, 8.2, 8.1, 8.7 ms, without 8.95).  Schedules
+// of 1000 nets (81 batches) 10.5 -> 3.4 ms, of 40 nets 0.46 -> 0.15 ms.
+constexpr int SMALL_NETS = 2048, SMALL_PTS = 65535;
+constexpr int SMALL_LDS = 144 << 10;   // of the 160 KB: the map (4 bytes a cell), then the points' slots (2 each)
+constexpr int SLOT_BASE = 1 << 17;   // a cell's slot in the map is its entry less this
+struct SmallNet {
+    ANet net;
+    SSeg seg;
+};
+
+// The unassigned nets in index order with their points' offsets; *res is how
+// many they are, -1 if they or their points exceed the limits.
+__global__ void __launch_bounds__(LTPB) k_small_list(BArgs a, SmallNet* sl, int* soff, int* res) {
+    __shared__ int s_w[LTPB / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // exclusive scan over the workgroup; *total: its sum (the same everywhere)
+    const auto scan = [&](int v, int* total) {
+        int incl = v;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int u = __shfl_up(incl, d);
+            if (lane >= d) incl += u;
+        }
+        if (lane == 63) s_w[wv] = incl;
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < LTPB / 64; w++) {
+            if (w < wv) before += s_w[w];
+            all += s_w[w];
+        }
+        __syncthreads();
+        *total = all;
+        return before + incl - v;
+    };
+    int n = 0;
+    for (int64_t w0 = 0; w0 < a.nwords; w0 += LTPB) {
+        const int64_t w = w0 + tid;
+        uint32_t m = w < a.nwords ? ~a.nst[w] & NST_ASSIGNED : 0;
+        if (w == a.nwords - 1 && (a.n & 15)) m &= (1u << (2 * (a.n & 15))) - 1;
+        int total;
+        int pos = n + scan(__popc(m), &total);
+        for (; m; m &= m - 1, pos++)
+            if (pos < SMALL_NETS) sl[pos].net.i = (int)(w * 16 + (__builtin_ctz(m) >> 1));
+        n += total;
+    }
+    __syncthreads();   // sl is read by other threads below
+    int64_t pts = 0;
+    if (n <= SMALL_NETS)
+        for (int r0 = 0; r0 < n; r0 += LTPB) {
+            const int r = r0 + tid;
+            SNet s{0, 0, 0};
+            if (r < n) s = a.sn[sl[r].net.i];
+            // a net of more points than the limit counts as the limit and one
+            int total;
+            const int off = (int)pts + scan(s.npt <= SMALL_PTS ? s.npt : SMALL_PTS + 1, &total);
+            if (r < n) {
+                sl[r].net.npt = s.npt;
+                sl[r].net.pt0 = s.pt0;
+                sl[r].seg = a.sg[sl[r].net.i];
+                soff[r] = off;
+            }
+            pts += total;
+            if (pts > SMALL_PTS) break;
+        }
+    if (tid == 0) {
+        const bool fits = n <= SMALL_NETS && pts <= SMALL_PTS;
+        if (fits) soff[n] = (int)pts;
+        *res = fits ? n : -1;
+    }
+}
+
+__global__ void k_small_fill(int* slot, int64_t cells) {
+    const int64_t q = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    if (q < cells) slot[q] = -1;
+}
+
+// Sixteen lanes a net: the cells' slots.
+__global__ void __launch_bounds__(TPB) k_small_mark(BArgs a, const SmallNet* sl, const int* soff, int* slot, const int* res) {
+    const int r = (int)(((int64_t)blockIdx.x * TPB + threadIdx.x) >> 4);
+    if (r >= *res) return;
+    const ANet s = sl[r].net;
+    const int off = soff[r];
+    for (int k = threadIdx.x & 15; k < s.npt; k += 16) slot[a.pt[s.pt0 + k]] = off + k;
+}
+
+__global__ void __launch_bounds__(LTPB) k_small_rounds(BArgs a, int64_t g, const SmallNet* sl,
+                                                       const int* soff, int* slot, int* res) {
+    __shared__ __align__(16) int s_map[SMALL_LDS / 4];
+    __shared__ uint16_t s_off[SMALL_NETS + 2], s_act[SMALL_NETS], s_via[SMALL_NETS];
+    __shared__ uint8_t s_st[SMALL_NETS];   // 0 active, 1 assigned, 2 blocked in this batch
+    __shared__ int s_na, s_nv, s_won, s_cells;
+    constexpr int PER = SMALL_NETS / LTPB;
+    const int nu = *res;
+    if (nu < 0) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int grp = tid >> 4, lg = tid & 15;
+    constexpr int GROUPS = LTPB / 16, U = 4, CHUNK_NETS = GROUPS * U, KEEP = 1;
+    if (tid == 0) s_cells = 0;
+    for (int r = tid; r <= nu; r += LTPB) s_off[r] = (uint16_t)soff[r];
+    for (int r = tid; r < nu; r += LTPB) s_st[r] = 0;
+    __syncthreads();
+    // slots: f(point's position, cell) over all points, sixteen lanes a net
+    const auto points = [&](auto f) {
+        for (int r0 = 0; r0 < nu; r0 += GROUPS) {
+            const int r = r0 + grp;
+            const ANet s = r < nu ? sl[r].net : ANet{0, 0, 0};
+            const int off = r < nu ? s_off[r] : 0;
+            for (int k = lg; __ballot(k < s.npt); k += 16) f(k < s.npt, off + k, k < s.npt ? a.pt[s.pt0 + k] : 0);
+        }
+    };
+    points([&](bool in, int e, int q) {
+        const bool mine = in && slot[q] == e;
+        const uint64_t m = __ballot(mine);
+        if (m == 0) return;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&s_cells, __popcll(m));
+        base = __shfl(base, 0);
+        if (mine) slot[q] = SLOT_BASE + base + __popcll(m & ((1ull << lane) - 1));
+    });
+    __threadfence();
+    __syncthreads();
+    const int ne = s_cells, ne4 = (ne + 3) / 4 * 4;
+    if (4 * ne4 + 2 * s_off[nu] > SMALL_LDS) {
+        if (tid == 0) *res = -1;
+        return;
+    }
+    uint16_t* const pid = reinterpret_cast<uint16_t*>(s_map + ne4);
+    points([&](bool in, int e, int q) {
+        if (in) pid[e] = (uint16_t)(slot[q] - SLOT_BASE);
+    });
+    __syncthreads();
+    // A chunk: 256 listed nets, sixteen lanes a net, U nets a group, with the
+    // lanes' first two points' slots.  A round's first KEEP chunks stay in
+    // registers from pass to pass: the loads of a pass, not its work, are its
+    // time.
+    struct Chunk {
+        int net[U];      // rank, -1: none
+        int cnt[U];      // points
+        int slot[U];     // two slots, 0xffff: none
+        int live;        // steps of GROUPS nets that hold any
+    };
+    const auto load = [&](const uint16_t* list, int n, int t0) {
+        Chunk c;
+        c.live = (n - t0 + GROUPS - 1) / GROUPS;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u >= c.live) break;
+            const int t = t0 + u * GROUPS + grp;
+            const int r = t < n ? list[t] : -1;
+            const int beg = r >= 0 ? s_off[r] : 0;
+            c.cnt[u] = r >= 0 ? s_off[r + 1] - beg : 0;
+            c.net[u] = r;
+            const int p0 = lg < c.cnt[u] ? pid[beg + lg] : 0xffff;
+            const int p1 = lg + 16 < c.cnt[u] ? pid[beg + lg + 16] : 0xffff;
+            c.slot[u] = p0 | p1 << 16;
+        }
+        return c;
+    };
+    // test(rank, slot) over the points of a chunk's nets for which begin(rank)
+    // holds; end(rank, whether any of the lane's points gave true).
+    const auto apply = [&](const Chunk& c, auto begin, auto test, auto end) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u >= c.live) break;   // the same for every thread
+            const int r = c.net[u];
+            const bool on = r >= 0 && begin(r);
+            const int p0 = c.slot[u] & 0xffff, p1 = c.slot[u] >> 16 & 0xffff;
+            bool f = on && p0 != 0xffff && test(r, p0);
+            if (on && p1 != 0xffff) f |= test(r, p1);
+            if (on && c.cnt[u] > 32) {
+                const int beg = s_off[r];
+                for (int k = lg + 32; k < c.cnt[u]; k += 16) f |= test(r, (int)pid[beg + k]);
+            }
+            end(r, f);
+        }
+    };
+    Chunk kept[KEEP];
+    const auto over = [&](int n, auto begin, auto point, auto end) {
+#pragma unroll
+        for (int k = 0; k < KEEP; k++)
+            if (k * CHUNK_NETS < n) apply(kept[k], begin, point, end);
+        for (int t0 = KEEP * CHUNK_NETS; t0 < n; t0 += CHUNK_NETS) apply(load(s_act, n, t0), begin, point, end);
+    };
+    const auto all = [](int) { return true; };
+    // appends rank v for every lane with want (all lanes of the wave call)
+    const auto append = [&](bool want, int v, uint16_t* list, int* counter) {
+        const uint64_t m = __ballot(want);
+        if (m == 0) return;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(counter, __popcll(m));
+        base = __shfl(base, 0);
+        if (want) list[base + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)v;
+    };
+    int cur = a.ctrl[(g & 1) * C_WORDS + C_CUR];
+    int placed = 0;
+    unsigned long long rounds = 0, tested = 0, starts = 0;
+    while (placed < nu) {
+        // every unassigned net is active again, the map empty
+        __syncthreads();
+        if (tid == 0) s_na = s_nv = s_won = 0;
+        for (int e = 4 * tid; e < ne; e += 4 * LTPB) *reinterpret_cast<int4*>(s_map + e) = make_int4(-1, -1, -1, -1);
+        __syncthreads();
+        for (int r0 = 0; r0 < nu; r0 += LTPB) {
+            const int r = nu - 1 - r0 - tid;   // the highest priority claims first: most others then only look
+            const bool live = r >= 0 && s_st[r] != 1;
+            if (live) s_st[r] = 0;
+            append(live, r, s_act, &s_na);
+        }
+        __syncthreads();
+        int na = s_na;
+        starts += na;
+        bool have = false;
+        for (int round = 0; round < ROUNDS; round++) {
+            rounds++;
+            tested += na;
+#pragma unroll
+            for (int k = 0; k < KEEP; k++)
+                if (k * CHUNK_NETS < na) kept[k] = load(s_act, na, k * CHUNK_NETS);
+            // point claims
+            over(na, all,
+                 [&](int r, int p) {
+                     if (s_map[p] < r) atomicMax(&s_map[p], r);
+                     return false;
+                 },
+                 [](int, bool) {});
+            __syncthreads();
+            // the nets that own every point cell
+            over(na, all, [&](int r, int p) { return s_map[p] != r; },
+                 [&](int r, bool lost) {
+                     const bool any = group_bits(__ballot(lost), 16) != 0;
+                     append(lg == 0 && r >= 0 && !any, r, s_via, &s_nv);
+                 });
+            __syncthreads();
+            const int nv = s_nv;
+            // their neighbour and segment claims
+            for (int w0 = 0; w0 < nv; w0 += GROUPS) {
+                const int r = w0 + grp < nv ? s_via[w0 + grp] : -1;
+                const SmallNet s = r >= 0 ? sl[r] : SmallNet{};
+                const auto claim = [&](bool in, int q) {
+                    const int p = in ? slot[q] - SLOT_BASE : -1;
+                    if (p >= 0) atomicMax(&s_map[p], r);
+                };
+                for (int k = lg; k < s.net.npt; k += 16) {
+                    bool valid[3];
+                    int q[3], p[3];
+                    point_neighbours(a, true, a.pt[s.net.pt0 + k], valid, q);
+                    for (int u = 0; u < 3; u++) p[u] = slot[valid[u] ? q[u] : 0];
+                    for (int u = 0; u < 3; u++)
+                        if (valid[u] && p[u] >= 0) atomicMax(&s_map[p[u] - SLOT_BASE], r);
+                }
+                group_segment_cells<16, 1>(a, s.seg, [&](bool(&valid)[1], int(&q)[1]) { claim(valid[0], q[0]); });
+            }
+            __syncthreads();
+            // commits
+            for (int t0 = 0; t0 < nv; t0 += CHUNK_NETS)
+                apply(load(s_via, nv, t0), all, [&](int r, int p) { return s_map[p] != r; },
+                      [&](int r, bool lost) {
+                          const bool any = group_bits(__ballot(lost), 16) != 0;
+                          if (lg == 0 && r >= 0 && !any) {
+                              s_st[r] = 1;
+                              a.batch[sl[r].net.i] = cur;
+                              atomicAdd(&s_won, 1);
+                          }
+                      });
+            __syncthreads();
+            const int won = s_won;
+            if (won == 0) break;
+            have = true;
+            placed += won;
+            // active nets with a point cell of a committed net sit out the batch
+            over(na, [&](int r) { return s_st[r] == 0; },
+                 [&](int, int p) {
+                     const int o = s_map[p];
+                     return o >= 0 && s_st[o] == 1;
+                 },
+                 [&](int r, bool hit) {
+                     const bool any = group_bits(__ballot(hit), 16) != 0;
+                     if (lg == 0 && r >= 0 && any) s_st[r] = 2;
+                 });
+            int keep[PER];
+            for (int j = 0; j < PER; j++) keep[j] = j * LTPB + tid < na ? s_act[j * LTPB + tid] : -1;
+            __syncthreads();
+            if (tid == 0) s_na = s_nv = s_won = 0;
+            // their cells are free again; the nets still active
+            for (int e = 4 * tid; e < ne; e += 4 * LTPB) {   // past ne: -1 since the batch start
+                const int4 m = *reinterpret_cast<const int4*>(s_map + e);
+                const int bx = s_st[max(m.x, 0)], by = s_st[max(m.y, 0)], bz = s_st[max(m.z, 0)], bw = s_st[max(m.w, 0)];
+                const bool fx = (m.x >= 0) & (bx == 2), fy = (m.y >= 0) & (by == 2);
+                const bool fz = (m.z >= 0) & (bz == 2), fw = (m.w >= 0) & (bw == 2);
+                if (fx | fy | fz | fw)
+                    *reinterpret_cast<int4*>(s_map + e) =
+                        make_int4(fx ? -1 : m.x, fy ? -1 : m.y, fz ? -1 : m.z, fw ? -1 : m.w);
+            }
+            __syncthreads();
+            for (int j = 0; j < PER; j++)
+                if (j * LTPB < na) append(keep[j] >= 0 && s_st[keep[j]] == 0, keep[j], s_act, &s_na);
+            __syncthreads();
+            na = s_na;
+            if (na == 0) break;
+        }
+        if (!have) break;   // cannot happen while nets are left: the host reports it
+        cur++;
+    }
+    if (tid == 0) {
+        for (int k = 0; k < 2; k++) {
+            a.ctrl[k * C_WORDS + C_DONE] = 1;
+            a.ctrl[k * C_WORDS + C_CUR] = cur;
+        }
+        a.ctrl[2 * C_WORDS] += placed;
+        a.stat[0] += rounds;
+        a.stat[1] += tested;
+        a.stat[2] += starts;
+    }
+}
+
+// The nets left do not fit: the rounds go on from the batch start they stopped at.
+__global__ void k_small_resume(BArgs a) {
+    a.ctrl[C_DONE] = 0;
+    a.ctrl[C_WORDS + C_DONE] = 0;
 }
 
 // Net records.  Scheduler index i is entry n - 1 - i of the order (its net
@@ -1208,9 +1550,66 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     S.batch.alloc(n);
     S.viable.alloc(n);
     S.stat.zero(3, st);
-    S.ctrl.zero(2 * C_WORDS + 1, st);
+    S.ctrl.zero(2 * C_WORDS + 2, st);   // the last word: k_small_list's result
     const int64_t nwords = (n + 15) / 16;
     S.bits.zero(nwords, st);
+    const char* trace_path = std::getenv("IGR_SCHED_TRACE");
+    const bool tracing = trace_path && *trace_path;
+    if (!S.h_ctrl) HIP_OK(hipHostMalloc(&S.h_ctrl, sizeof(int) * (2 * C_WORDS + 2)));
+    int* h_ctrl = S.h_ctrl;
+    const auto read_ctrl = [&] {
+        HIP_OK(hipMemcpyAsync(h_ctrl, S.ctrl.p, sizeof(int) * (2 * C_WORDS + 2), hipMemcpyDeviceToHost, st));
+        HIP_OK(hipStreamSynchronize(st));
+    };
+    // The one-workgroup rounds for the nets that are left, where they fit.
+    const bool small_ok = c->tune.sched_kind == 0 && !tracing;
+    const auto small_rounds = [&](const BArgs& b, int64_t g) {
+        S.small.alloc(sizeof(SmallNet) * SMALL_NETS + sizeof(int) * (SMALL_NETS + 4));
+        S.slot.alloc(XYc);
+        SmallNet* sl = reinterpret_cast<SmallNet*>(S.small.p);
+        int* soff = reinterpret_cast<int*>(sl + SMALL_NETS);
+        int* res = S.ctrl.p + 2 * C_WORDS + 1;
+        k_small_list<<<1, LTPB, 0, st>>>(b, sl, soff, res);
+        k_small_fill<<<blocks(XYc), TPB, 0, st>>>(S.slot.p, XYc);
+        k_small_mark<<<blocks((int64_t)SMALL_NETS * 16), TPB, 0, st>>>(b, sl, soff, S.slot.p, res);
+        k_small_rounds<<<1, LTPB, 0, st>>>(b, g, sl, soff, S.slot.p, res);
+        HIP_OK(hipGetLastError());
+        read_ctrl();
+        return h_ctrl[2 * C_WORDS + 1] >= 0;
+    };
+    BArgs a{};
+    a.n = n;
+    a.sn = sn;
+    a.sg = sg;
+    a.pt = d_pt_off ? d_pt : N.pt.p;
+    a.hs = N.hs.p;
+    a.vs = N.vs.p;
+    a.batch = S.batch.p;
+    a.ctrl = S.ctrl.p;
+    a.stat = S.stat.p;
+    a.nst = (uint32_t*)S.bits.p;
+    a.nwords = nwords;
+    a.X = c->g.X;
+    a.Y = c->g.Y;
+    a.sparsity = (mode == 1 || mode == 2) ? 2 : 15;
+    const auto finish = [&](const char* kind) {
+        const int nbatch = h_ctrl[C_CUR];
+        const int64_t placed = h_ctrl[2 * C_WORDS];
+        unsigned long long sv[3] = {0, 0, 0};
+        HIP_OK(hipMemcpyAsync(sv, S.stat.p, sizeof(sv), hipMemcpyDeviceToHost, st));
+        HIP_OK(hipStreamSynchronize(st));
+        progress("scheduler (%s rounds): %d batches, %llu rounds, %.0f nets tested per round, %.0f unassigned per "
+                 "batch", kind, nbatch, sv[0], sv[0] ? (double)sv[1] / (double)sv[0] : 0.0,
+                 nbatch ? (double)sv[2] / nbatch : 0.0);
+        if (placed != n) throw std::runtime_error("scheduler left a net without a batch");
+        if (!h_batch_of) return nbatch;
+        std::vector<int> b(n);
+        HIP_OK(hipMemcpyAsync(b.data(), S.batch.p, sizeof(int) * n, hipMemcpyDeviceToHost, st));
+        HIP_OK(hipStreamSynchronize(st));
+        for (int64_t i = 0; i < n; i++) h_batch_of[n - 1 - i] = b[i];
+        return nbatch;
+    };
+    if (small_ok && n <= SMALL_NETS && small_rounds(a, 0)) return finish("one-workgroup");
     // Per-cell lists of the nets' point cells, highest priority first.
     k_cell_count<<<blocks(n), TPB, 0, st>>>(n, sn, d_pt_off ? d_pt : N.pt.p, S.cnt.p);
     launch_exclusive_scan(c, S.cnt.p, XYc, S.c_off.p);
@@ -1230,15 +1629,27 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         S.hstamp.zero(XYc, st);
         S.cur.alloc(XYc);
     }
-    BArgs a{n, sn, sg, d_pt_off ? d_pt : N.pt.p, N.hs.p, N.vs.p, S.map.p, S.base.p, S.c_off.p, S.c_end.p, S.c_net.p, S.head.p,
-            S.batch.p, S.ctrl.p, S.lists.p, release ? nullptr : reinterpret_cast<ANet*>(S.alists.p),
-            release ? S.rel.p : nullptr, release ? S.cand.p : nullptr, release ? S.cstamp.p : nullptr,
-            release ? S.lists.p + 2 * n : nullptr,
-            release ? S.hits.p : nullptr, release ? S.hstamp.p : nullptr,
-            release ? S.cur.p : nullptr, S.stat.p,
-            (uint32_t*)S.bits.p, nwords,
-            c->g.X, c->g.Y,
-            (mode == 1 || mode == 2) ? 2 : 15, nullptr, 0, nullptr};
+    a.map = S.map.p;
+    a.base = S.base.p;
+    a.c_off = S.c_off.p;
+    a.c_end = S.c_end.p;
+    a.c_net = S.c_net.p;
+    a.head = S.head.p;
+    if (release) {
+        a.lists = S.lists.p;
+        a.rel = S.rel.p;
+        a.cand = S.cand.p;
+        a.cstamp = S.cstamp.p;
+        a.v0 = S.lists.p + 2 * n;
+        a.hits = S.hits.p;
+        a.hstamp = S.hstamp.p;
+        a.cur = S.cur.p;
+    } else {
+        a.alists = reinterpret_cast<ANet*>(S.alists.p);
+    }
+    // Nets that fit the one-workgroup rounds if they are like the others, with
+    // two points a cell (4 bytes a point).
+    if (small_ok) a.small_at = (int)std::min<int64_t>(SMALL_NETS, SMALL_LDS / 4 * n / std::max<int64_t>(1, entries));
     // kernel timing on: the round kernels count the bytes they move
     DevBuf<unsigned long long> byte_slots;
     if (c->prof.on && release) {
@@ -1246,9 +1657,8 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
         a.bytes = byte_slots.p;
     }
     // IGR_SCHED_TRACE=<file>: append one line per round (the TR_* record)
-    const char* trace_path = std::getenv("IGR_SCHED_TRACE");
     DevBuf<long long> trace;
-    if (trace_path && *trace_path) {
+    if (tracing) {
         a.trace_cap = 1 << 20;
         trace.zero(a.trace_cap * TR_WORDS, st);
         a.trace = trace.p;
@@ -1269,8 +1679,6 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
     const unsigned wgrid = (unsigned)std::min<int64_t>(1024, std::max<int64_t>(16, n / 64));
     const unsigned cgrid = (wgrid + 3) / 4;
     const unsigned gm = (unsigned)std::min<int64_t>(512, (std::max(XYc, n) + LTPB - 1) / LTPB);   // grid-stride
-    if (!S.h_ctrl) HIP_OK(hipHostMalloc(&S.h_ctrl, sizeof(int) * (2 * C_WORDS + 1)));
-    int* h_ctrl = S.h_ctrl;
     const int64_t max_rounds = (int64_t)ROUNDS * (n + 1) + CHUNK;
     int64_t g = 0;
     const auto t_start = std::chrono::steady_clock::now();
@@ -1307,12 +1715,17 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
             else round(std::integral_constant<int, 16>{});
         }
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(h_ctrl, S.ctrl.p, sizeof(int) * (2 * C_WORDS + 1), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipStreamSynchronize(st));
-        if (h_ctrl[(g & 1) * C_WORDS + C_DONE]) break;
+        read_ctrl();
+        const int done = h_ctrl[(g & 1) * C_WORDS + C_DONE];
+        if (done == 1) break;
+        if (done == 2) {
+            const int64_t rest = n - h_ctrl[2 * C_WORDS];
+            if (small_rounds(a, g)) break;
+            a.small_at = (int)(rest / 2);
+            k_small_resume<<<1, 1, 0, st>>>(a);
+        }
     }
-    const int nbatch = h_ctrl[(g & 1) * C_WORDS + C_CUR];
-    const int64_t placed = h_ctrl[2 * C_WORDS];
+    h_ctrl[C_CUR] = h_ctrl[(g & 1) * C_WORDS + C_CUR];
     if (a.bytes) {
         std::vector<unsigned long long> slots(BYTE_SLOTS);
         HIP_OK(hipMemcpyAsync(slots.data(), a.bytes, sizeof(unsigned long long) * BYTE_SLOTS, hipMemcpyDeviceToHost,
@@ -1342,21 +1755,7 @@ int run_schedule_batched(igr_ctx* c, const int* h_order, int64_t n, int mode, in
             std::fclose(f);
         }
     }
-    {
-        unsigned long long sv[3] = {0, 0, 0};
-        HIP_OK(hipMemcpyAsync(sv, S.stat.p, sizeof(sv), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipStreamSynchronize(st));
-        progress("scheduler (%s rounds): %d batches, %llu rounds, %.0f nets tested per round, %.0f unassigned per "
-                 "batch", release ? "release-driven" : "active-list", nbatch, sv[0],
-                 sv[0] ? (double)sv[1] / (double)sv[0] : 0.0, nbatch ? (double)sv[2] / nbatch : 0.0);
-    }
-    if (placed != n) throw std::runtime_error("scheduler left a net without a batch");
-    if (!h_batch_of) return nbatch;
-    std::vector<int> b(n);
-    HIP_OK(hipMemcpyAsync(b.data(), S.batch.p, sizeof(int) * n, hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
-    for (int64_t i = 0; i < n; i++) h_batch_of[n - 1 - i] = b[i];
-    return nbatch;
+    return finish(release ? "release-driven" : "active-list");
 }
 
 } // namespace igr_dev
