@@ -59,139 +59,157 @@ __global__ void k_fill_i32(int* p, int64_t n, int v) {
     if (i < n) p[i] = v;
 }
 
-// precompute_cost_edge: one thread per (edge, from layer).
+// precompute_cost_edge: one thread per (edge, from layer, to layer).  A thread
+// walks up to 39 samples of some ten loads each, so a launch is a latency
+// chain: 34 us a batch of 600 nets (175 with one thread per (edge, from layer),
+// over every to layer).
 __global__ void __launch_bounds__(TPB) k_dag_edges(DagArgs a, int64_t edges) {
     int64_t t = (int64_t)blockIdx.x * TPB + threadIdx.x;
     const GridDev& g = a.g;
     const int L = g.L, LL = L * L;
-    if (t >= edges * L) return;
-    const int64_t e = a.edge0 + t / L;
-    const int fl = (int)(t % L);
+    if (t >= edges * LL) return;
+    const int64_t e = a.edge0 + t / LL;
+    const int fl = (int)(t % LL) / L, tl = (int)(t % LL) % L;
     const int64_t er = e - a.edge0;
     const int to = a.par[e], from = a.enode[e];
     const int tox = a.node[to] / g.Y % g.X, toy = a.node[to] % g.Y;
     const int fromx = a.node[from] / g.Y % g.X, fromy = a.node[from] % g.Y;
     if ((layer_dir(fl, g.DIR) == 0 && fromy != toy) || (layer_dir(fl, g.DIR) == 1 && fromx != tox)) {
-        for (int tl = 0; tl < L; tl++) a.cost_edges[er * LL + fl * L + tl] = INF;
+        a.cost_edges[er * LL + fl * L + tl] = INF;
         return;
     }
     const int distance = abs(tox - fromx) + abs(toy - fromy);
-    if (distance == 0) return;
+    if (distance == 0 || (tl % 2) != (fl % 2)) return;
     const int dd = distance / min(distance, 20);
     const bool vert = fromx == tox;
     const int s0 = vert ? min(fromy, toy) : min(fromx, tox);
     const int s1 = vert ? max(fromy, toy) : max(fromx, tox);
-    for (int tl = 0; tl < L; tl++) {
-        if ((tl % 2) != (fl % 2)) continue;
-        double mn = INF;
-        int decide = -1;
-        for (int sp = s0 + dd; sp < s1; sp += dd) {
-            const int sx = vert ? fromx : sp, sy = vert ? sp : fromy;
-            double via = 0;
-            for (int ll = min(fl, tl); ll < max(fl, tl); ll++) via += (double)g.vcost[gidx(g, ll, sx, sy)];
-            double cost = via;
-            if (vert)
-                cost += (wseg(g, fl, fromx, fromx, min(fromy, sy), max(fromy, sy)) +
-                         wseg(g, tl, tox, tox, min(toy, sy), max(toy, sy)));
-            else
-                cost += (wseg(g, fl, min(fromx, sx), max(fromx, sx), fromy, fromy) +
-                         wseg(g, tl, min(tox, sx), max(tox, sx), toy, toy));
-            if (cost < mn) { mn = cost; decide = sp; }
-        }
-        a.cost_edges[er * LL + fl * L + tl] = mn;
-        a.best_change[er * LL + fl * L + tl] = decide;
-    }
-}
-
-// Bottom-up DP of one node by one thread (Lshape_route_node_layer_change_cuda,
-// src/Lshape_route_detour.hpp:281-353): for each lowest layer, the running
-// minimum of every child slot over the layers above it, the via costs in
-// layer order, then the downward sweep.
-__device__ void dp_node_seq(const DagArgs& a, int node) {
-    const GridDev& g = a.g;
-    const int L = g.L, ML = L + 1, XY = g.X * g.Y;
-    const int nr = (int)(node - a.node0);
-    const int x = a.node[node] / g.Y % g.X, y = a.node[node] % g.Y;
-    const int fixed_low = 1 + a.node[node] / XY;
-    const int fixed_high = fixed_low == ML ? 0 : fixed_low;
-    const int nc = a.child_num[node];
-    const int64_t cs = a.csum[node] - a.slot0;
-    uint64_t* cur_best = a.best + cs * ML;
-    const uint64_t* cur_packed = a.packed + cs * ML;
-    double* cst = a.costs + (int64_t)nr * ML;
-    double mcc[10];
-    uint64_t bp[10];
-    // low above L visits no layer (the reference's loop runs it empty)
-    const int lowtop = min(fixed_low, L);
-    for (int low = 1; low <= lowtop; low++) {
-        for (int k = 0; k < nc; k++) mcc[k] = INF;
+    double mn = INF;
+    int decide = -1;
+    for (int sp = s0 + dd; sp < s1; sp += dd) {
+        const int sx = vert ? fromx : sp, sy = vert ? sp : fromy;
         double via = 0;
-        for (int li = low; li < L + 1; li++) {
-            if (li > low) via += (double)g.vcost[gidx(g, li - 2, x, y)];
-            for (int k = 0; k < nc; k++) {
-                const uint64_t key = cur_packed[k * ML + li];
-                double cc = unpack_cost(key);
-                if (cc < mcc[k]) {
-                    mcc[k] = cc;
-                    bp[k] = (uint64_t)(uint32_t)key * ML + li;
-                }
-            }
-            if (li >= fixed_high) {
-                double cost = via;
-                for (int k = 0; k < nc; k++) cost += mcc[k];
-                if (cost < INF && cost < cst[li]) {
-                    cst[li] = cost;
-                    for (int k = 0; k < nc; k++) cur_best[k * ML + li] = bp[k];
-                }
-            }
-        }
-        for (int li = L + 1 - 2; li >= low; li--)
-            if (cst[li + 1] < cst[li]) {
-                cst[li] = cst[li + 1];
-                for (int k = 0; k < nc; k++) cur_best[k * ML + li] = cur_best[k * ML + li + 1];
-            }
+        for (int ll = min(fl, tl); ll < max(fl, tl); ll++) via += (double)g.vcost[gidx(g, ll, sx, sy)];
+        double cost = via;
+        if (vert)
+            cost += (wseg(g, fl, fromx, fromx, min(fromy, sy), max(fromy, sy)) +
+                     wseg(g, tl, tox, tox, min(toy, sy), max(toy, sy)));
+        else
+            cost += (wseg(g, fl, min(fromx, sx), max(fromx, sx), fromy, fromy) +
+                     wseg(g, tl, min(tox, sx), max(tox, sx), toy, toy));
+        if (cost < mn) { mn = cost; decide = sp; }
     }
+    a.cost_edges[er * LL + fl * L + tl] = mn;
+    a.best_change[er * LL + fl * L + tl] = decide;
 }
 
-// Bottom-up DP of one node (thread) of the current depth level.
-__global__ void __launch_bounds__(TPB) k_dag_dp(DagArgs a, const int* lvl_nodes, int64_t lo_i, int64_t hi_i) {
-    int64_t t = lo_i + (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (t >= hi_i) return;
+// Bottom-up DP of the nodes of one depth level
+// (Lshape_route_node_layer_change_cuda, src/Lshape_route_detour.hpp:281-406),
+// sixteen lanes a node.  Lane s first takes lowest layer s: the running
+// minimum of every child slot over the layers above it, the via costs in layer
+// order, which gives the cost of every range [s, hi].  The downward sweeps
+// leave on each layer the smallest range that holds it, ties to the smaller
+// low, then the smaller hi: lane s picks layer s's, and its children's
+// layers.  Then lane s forms the keys of parent layer s for every parent edge.
+// A level is a few hundred nodes, so a launch is the latency of one node: 26 us
+// (119 with a thread per node).
+constexpr int DP_NODES = 4, DP_SLOTS = 10;   // nodes a workgroup, child slots a node
+__global__ void __launch_bounds__(16 * DP_NODES) k_dag_dp(DagArgs a, const int* lvl_nodes, int64_t lo_i, int64_t hi_i) {
+    __shared__ uint64_t s_key[DP_NODES][DP_SLOTS * (MAXL + 1)];
+    __shared__ double s_cost[DP_NODES][MAXL * MAXL], s_cst[DP_NODES][MAXL + 1];
+    __shared__ float s_via[DP_NODES][16];
+    const int gi = threadIdx.x >> 4, s = threadIdx.x & 15;
+    const int64_t t = lo_i + (int64_t)blockIdx.x * DP_NODES + gi;
+    const bool live = t < hi_i;
     const GridDev& g = a.g;
     const int L = g.L, ML = L + 1, LL = L * L, SENT = LL + 1, XY = g.X * g.Y;
-    const int node = lvl_nodes[t];
-    const int nr = (int)(node - a.node0);
-    const int x = a.node[node] / g.Y % g.X, y = a.node[node] % g.Y;
-    const double* cst = a.costs + (int64_t)nr * ML;
-    dp_node_seq(a, node);
-    const uint32_t myid = (uint32_t)a.loc[node] * ID_MUL;
-    for (int64_t e = a.par_off[node]; e < a.par_off[node + 1]; e++) {
-        const int p = a.par[e], ci = a.slot[e];
-        uint64_t* ppk = a.packed + (a.csum[p] - a.slot0 + ci) * ML;
-        const int px = a.node[p] / g.Y % g.X, py = a.node[p] % g.Y;
-        const int minx = min(x, px), maxx = max(x, px), miny = min(y, py), maxy = max(y, py);
-        const int64_t er = e - a.edge0;
-        uint64_t cache[MAXL + 1];
-        for (int tt = 1; tt < ML; tt++) cache[tt] = ppk[tt];
-        for (int layer = 1; layer < ML; layer++) {
-            if (((layer & 1) ^ g.DIR) == 1 && y != py) continue;
-            if (((layer & 1) ^ g.DIR) == 0 && x != px) continue;
-            const double base = cst[layer];
-            for (int tt = 1 + (1 - layer % 2); tt < ML; tt += 2) {
-                double cost2;
-                int choice = SENT;
-                if (tt == layer) cost2 = base + wseg(g, layer - 1, minx, maxx, miny, maxy);
-                else if (abs(x - px) + abs(y - py) > 4) {
-                    const int q = (layer - 1) * L + (tt - 1);
-                    const double ce = a.cost_edges[er * LL + q];
-                    if (ce < INF) { cost2 = base + ce; choice = q; }
-                    else continue;
-                } else continue;
-                const uint64_t key = pack_key((float)cost2, myid + (uint32_t)choice);
-                if (key < cache[tt]) cache[tt] = key;
+    const int node = live ? lvl_nodes[t] : 0;
+    const int v = live ? a.node[node] : 0;
+    const int x = v / g.Y % g.X, y = v % g.Y;
+    const int fixed_low = 1 + v / XY;
+    const int fixed_high = fixed_low == ML ? 0 : fixed_low;
+    const int nc = live ? a.child_num[node] : 0;
+    const int64_t cs = live ? a.csum[node] - a.slot0 : 0;
+    for (int i = s; i < nc * ML; i += 16) s_key[gi][i] = a.packed[cs * ML + i];
+    s_via[gi][s] = live && s < L - 1 ? g.vcost[gidx(g, s, x, y)] : 0.f;
+    __syncthreads();
+    // low above L visits no layer (the reference's loop runs it empty)
+    const int lowtop = min(fixed_low, L);
+    if (live && s >= 1 && s <= lowtop) {
+        double mcc[DP_SLOTS];
+#pragma unroll
+        for (int k = 0; k < DP_SLOTS; k++) mcc[k] = INF;
+        double via = 0;
+        for (int li = s; li < ML; li++) {
+            if (li > s) via += (double)s_via[gi][li - 2];
+            double cost = via;
+#pragma unroll
+            for (int k = 0; k < DP_SLOTS; k++) {
+                if (k >= nc) break;
+                const double cc = unpack_cost(s_key[gi][k * ML + li]);
+                mcc[k] = cc < mcc[k] ? cc : mcc[k];
+                cost += mcc[k];
+            }
+            s_cost[gi][(s - 1) * MAXL + li - 1] = li >= fixed_high ? cost : INF;
+        }
+    }
+    __syncthreads();
+    if (s <= L) {
+        double best = INF;
+        int blo = 0, bhi = 0;
+        if (live && s >= 1)
+            for (int low = 1; low <= min(s, lowtop); low++)
+                for (int hi = s; hi < ML; hi++) {
+                    const double cost = s_cost[gi][(low - 1) * MAXL + hi - 1];
+                    if (cost < best) {
+                        best = cost;
+                        blo = low;
+                        bhi = hi;
+                    }
+                }
+        s_cst[gi][s] = best;
+        if (blo) {
+            a.costs[(int64_t)(node - a.node0) * ML + s] = best;
+            for (int k = 0; k < nc; k++) {
+                double m = INF;
+                uint64_t bp = 0;
+                for (int li = blo; li <= bhi; li++) {
+                    const uint64_t key = s_key[gi][k * ML + li];
+                    const double cc = unpack_cost(key);
+                    if (cc < m) {
+                        m = cc;
+                        bp = (uint64_t)(uint32_t)key * ML + li;
+                    }
+                }
+                a.best[(cs + k) * ML + s] = bp;
             }
         }
-        for (int tt = 1; tt < ML; tt++) atomicMin((unsigned long long*)&ppk[tt], (unsigned long long)cache[tt]);
+    }
+    __syncthreads();
+    if (!live || s < 1 || s > L) return;
+    const uint32_t myid = (uint32_t)a.loc[node] * ID_MUL;
+    for (int64_t e = a.par_off[node]; e < a.par_off[node + 1]; e++) {
+        const int p = a.par[e];
+        const int px = a.node[p] / g.Y % g.X, py = a.node[p] % g.Y;
+        if (((s & 1) ^ g.DIR) == 1 ? y != py : x != px) continue;
+        const bool far = abs(x - px) + abs(y - py) > 4;
+        uint64_t key = ~0ull;
+        for (int layer = 2 - (s & 1); layer < ML; layer += 2) {
+            double cost2 = s_cst[gi][layer];
+            int choice = SENT;
+            if (s == layer) {
+                cost2 += wseg(g, layer - 1, min(x, px), max(x, px), min(y, py), max(y, py));
+            } else if (far) {
+                choice = (layer - 1) * L + (s - 1);
+                const double ce = a.cost_edges[(e - a.edge0) * LL + choice];
+                if (!(ce < INF)) continue;
+                cost2 += ce;
+            } else {
+                continue;
+            }
+            key = min(key, pack_key((float)cost2, myid + (uint32_t)choice));
+        }
+        atomicMin((unsigned long long*)&a.packed[(a.csum[p] - a.slot0 + a.slot[e]) * ML + s], (unsigned long long)key);
     }
 }
 
@@ -353,14 +371,15 @@ void launch_dag_batch_plain(igr_ctx* c, const DagBatch& b, int stamp, const std:
     DagArgs a = make_args(c, b, stamp);
     if (ne > 0) {
         KScope ks(c, K_DAG_EDGES, b.bytes_edges);
-        k_dag_edges<<<blocks(ne * c->g.L), TPB, 0, s>>>(a, ne);
+        k_dag_edges<<<blocks(ne * c->g.L * c->g.L), TPB, 0, s>>>(a, ne);
         HIP_OK(hipGetLastError());
     }
     {
         KScope ks(c, K_DAG_DP, b.bytes_dp);
         for (int d = b.levels - 1; d >= 0; d--) {
             int64_t lo = h_lvl_off[b.lvl0 + d], hi = h_lvl_off[b.lvl0 + d + 1];
-            if (hi > lo) k_dag_dp<<<blocks(hi - lo), TPB, 0, s>>>(a, D.lvl_nodes.p, lo, hi);
+            if (hi > lo)
+                k_dag_dp<<<(unsigned)((hi - lo + DP_NODES - 1) / DP_NODES), 16 * DP_NODES, 0, s>>>(a, D.lvl_nodes.p, lo, hi);
         }
     }
     {

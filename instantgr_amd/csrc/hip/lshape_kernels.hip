@@ -448,7 +448,7 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
             };
             if (minl < maxl) {
                 push(minl * XY + x * Y + y, maxl * XY + x * Y + y);
-                emit_via(g, minl, maxl, x, y);
+                if (g.vc) emit_via(g, minl, maxl, x, y);
             }
             if (i > 0) {
                 const int minx = min(x, px), maxx = max(x, px), miny = min(y, py), maxy = max(y, py);
@@ -462,7 +462,7 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
                     push(curl * XY + x * Y + y, curl * XY + hx * Y + hy);
                     add_segment(g, curl, min(x, hx), max(x, hx), min(y, hy), max(y, hy), stamp);
                     push(curl * XY + hx * Y + hy, parl * XY + hx * Y + hy);
-                    emit_via(g, curl, parl, hx, hy);
+                    if (g.vc) emit_via(g, curl, parl, hx, hy);
                     push(parl * XY + hx * Y + hy, parl * XY + px * Y + py);
                     add_segment(g, parl, min(px, hx), max(px, hx), min(py, hy), max(py, hy), stamp);
                 }

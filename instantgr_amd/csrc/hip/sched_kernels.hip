@@ -45,31 +45,53 @@ struct SchedArgs {
 
 __device__ __forceinline__ bool active(const SchedArgs& a, int64_t i) { return a.status[i] != 2 && a.batch[i] == -1; }
 
+// The kernels over nets take LPN lanes a net, a point each: a round of a few
+// thousand nets is the latency of its longest net (claims of points and of the
+// rest 22 and 24 us a round with a thread a net, 4 and 9 so).
+constexpr int LPN = 8;
+struct NetLanes {
+    int64_t i;                   // scheduler index
+    int lane;
+    uint64_t mask;               // the net's lanes in the wave
+    __device__ NetLanes()
+        : i(((int64_t)blockIdx.x * TPB + threadIdx.x) / LPN), lane(threadIdx.x % LPN),
+          mask(((1ull << LPN) - 1) << (threadIdx.x & 63 & ~(LPN - 1))) {}
+    __device__ bool any(bool v) const { return (__ballot(v) & mask) != 0; }   // over the net's lanes
+};
+
 __global__ void __launch_bounds__(TPB) k_claim_points(SchedArgs a) {
-    int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    const NetLanes t;
+    const int64_t i = t.i;
     if (i >= a.n || !active(a, i)) return;
-    a.status[i] = 1;
-    for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++) atomicMax(&a.map[a.pt[k]], (int)i);
+    if (t.lane == 0) a.status[i] = 1;
+    const int64_t e = a.pt_off[a.pids[i] + 1];
+    for (int64_t k = a.pt_off[a.pids[i]] + t.lane; k < e; k += LPN) atomicMax(&a.map[a.pt[k]], (int)i);
+}
+
+// Whether net i has a point cell that 'bad' rejects (its lanes call together).
+template <class F>
+__device__ __forceinline__ bool any_point(const SchedArgs& a, const NetLanes& t, F bad) {
+    const int64_t e = a.pt_off[a.pids[t.i] + 1];
+    bool b = false;
+    for (int64_t k = a.pt_off[a.pids[t.i]] + t.lane; k < e && !b; k += LPN) b = bad(a.map[a.pt[k]]);
+    return t.any(b);
 }
 
 __global__ void __launch_bounds__(TPB) k_viable(SchedArgs a) {
-    int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i >= a.n) return;
-    int ok = 0;
-    if (active(a, i)) {
-        ok = 1;
-        for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++)
-            if (a.map[a.pt[k]] != (int)i) { ok = 0; break; }
-    }
-    a.viable[i] = ok;
+    const NetLanes t;
+    if (t.i >= a.n) return;
+    const int ok = active(a, t.i) && !any_point(a, t, [&](int m) { return m != (int)t.i; });
+    if (t.lane == 0) a.viable[t.i] = ok;
 }
 
 __global__ void __launch_bounds__(TPB) k_claim_rest(SchedArgs a) {
-    int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    const NetLanes t;
+    const int64_t i = t.i;
     if (i >= a.n || !a.viable[i]) return;
     const int net = a.ids[i];
     const int X = a.X, Y = a.Y;
-    for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++) {
+    const int64_t pe = a.pt_off[a.pids[i] + 1];
+    for (int64_t k = a.pt_off[a.pids[i]] + t.lane; k < pe; k += LPN) {
         int p = a.pt[k], x = p / Y, y = p % Y;
         if (y - 1 >= 0) atomicMax(&a.map[x * Y + y - 1], (int)i);
         if (x - 1 >= 0) atomicMax(&a.map[(x - 1) * Y + y], (int)i);
@@ -77,30 +99,26 @@ __global__ void __launch_bounds__(TPB) k_claim_rest(SchedArgs a) {
     }
     for (int64_t k = a.hs_off[net]; k < a.hs_off[net + 1]; k++) {
         int s = a.hs[2 * k], e = a.hs[2 * k + 1], y = s % Y;
-        for (int x = s / Y; x <= e / Y; x += a.sparsity) atomicMax(&a.map[x * Y + y], (int)i);
+        for (int x = s / Y + t.lane * a.sparsity; x <= e / Y; x += LPN * a.sparsity) atomicMax(&a.map[x * Y + y], (int)i);
     }
     for (int64_t k = a.vs_off[net]; k < a.vs_off[net + 1]; k++) {
         int s = a.vs[2 * k], e = a.vs[2 * k + 1], x = s / Y;
-        for (int y = s % Y; y <= e % Y; y += a.sparsity) atomicMax(&a.map[x * Y + y], (int)i);
+        for (int y = s % Y + t.lane * a.sparsity; y <= e % Y; y += LPN * a.sparsity) atomicMax(&a.map[x * Y + y], (int)i);
     }
 }
 
 __global__ void __launch_bounds__(TPB) k_commit(SchedArgs a, int cur) {
-    int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i >= a.n || !active(a, i)) return;
-    for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++)
-        if (a.map[a.pt[k]] != (int)i) return;
-    a.batch[i] = cur;
+    const NetLanes t;
+    if (t.i >= a.n || !active(a, t.i)) return;
+    if (any_point(a, t, [&](int m) { return m != (int)t.i; }) || t.lane != 0) return;
+    a.batch[t.i] = cur;
     a.flags[0] = 1;
 }
 
 __global__ void __launch_bounds__(TPB) k_revert(SchedArgs a) {
-    int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i >= a.n || a.status[i] != 1 || a.batch[i] != -1) return;
-    for (int64_t k = a.pt_off[a.pids[i]]; k < a.pt_off[a.pids[i] + 1]; k++) {
-        int pre = a.map[a.pt[k]];
-        if (pre != -1 && a.batch[pre] != -1) { a.status[i] = 2; return; }
-    }
+    const NetLanes t;
+    if (t.i >= a.n || a.status[t.i] != 1 || a.batch[t.i] != -1) return;
+    if (any_point(a, t, [&](int m) { return m != -1 && a.batch[m] != -1; }) && t.lane == 0) a.status[t.i] = 2;
 }
 
 __global__ void __launch_bounds__(TPB) k_clear(SchedArgs a) {
@@ -162,16 +180,16 @@ int run_schedule(igr_ctx* c, const int* h_order, int64_t n, int mode, int* h_bat
             bool have_commit = false;
             for (int round = 0; round < 30; round++) {
                 k_fill<<<1, TPB, 0, st>>>(S.flags.p, 1, 0);
-                k_claim_points<<<blocks(n), TPB, 0, st>>>(a);
-                k_viable<<<blocks(n), TPB, 0, st>>>(a);
-                k_claim_rest<<<blocks(n), TPB, 0, st>>>(a);
-                k_commit<<<blocks(n), TPB, 0, st>>>(a, cur);
+                k_claim_points<<<blocks(n * LPN), TPB, 0, st>>>(a);
+                k_viable<<<blocks(n * LPN), TPB, 0, st>>>(a);
+                k_claim_rest<<<blocks(n * LPN), TPB, 0, st>>>(a);
+                k_commit<<<blocks(n * LPN), TPB, 0, st>>>(a, cur);
                 HIP_OK(hipGetLastError());
                 HIP_OK(hipMemcpyAsync(h_flag, S.flags.p, sizeof(int), hipMemcpyDeviceToHost, st));
                 HIP_OK(hipStreamSynchronize(st));
                 if (!*h_flag) break;
                 have_commit = true;
-                k_revert<<<blocks(n), TPB, 0, st>>>(a);
+                k_revert<<<blocks(n * LPN), TPB, 0, st>>>(a);
                 k_clear<<<blocks(XYc), TPB, 0, st>>>(a);
             }
             if (!have_commit) break;
