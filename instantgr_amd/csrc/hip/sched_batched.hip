@@ -417,19 +417,29 @@ struct GroupList {
 // src/database_cuda.hpp:320-352), the cells of up to W segments at a time
 // spread evenly over the W lanes of the net's group (a lane per segment would
 // walk a long segment alone).  Every lane of the wave calls it together; valid
-// is false on the lanes past the last cell, and f may use ballots.
+// is false on the lanes past the last cell, and f may use ballots.  The ends of
+// the first W segments come from segment_ends, called ahead of other work: its
+// loads then wait beside that work's.
+struct SegEnds {
+    int b, e;
+};
+__device__ __forceinline__ SegEnds segment_ends(const BArgs& a, const SSeg& g, int k) {
+    if (k >= g.nh + g.nv) return SegEnds{0, 0};
+    const int* seg = k < g.nh ? a.hs + 2 * (g.h0 + k) : a.vs + 2 * (g.v0 + k - g.nh);
+    return SegEnds{seg[0], seg[1]};
+}
 template <int W, int U, class F>
-__device__ __forceinline__ void group_segment_cells(const BArgs& a, const SSeg& g, F f) {
+__device__ __forceinline__ void group_segment_cells(const BArgs& a, const SSeg& g, SegEnds se, F f) {
     const int lane = threadIdx.x & (W - 1);
     const int Y = a.Y, sp = a.sparsity;
     const int ns = g.nh + g.nv;
     for (int sb = 0; __ballot(sb < ns); sb += W) {
         const int k = sb + lane;
         int cnt = 0, first = 0, step = 0;
+        if (sb > 0) se = segment_ends(a, g, k);
         if (k < ns) {
             const bool hor = k < g.nh;
-            const int* seg = hor ? a.hs + 2 * (g.h0 + k) : a.vs + 2 * (g.v0 + k - g.nh);
-            const int b = seg[0], e = seg[1];
+            const int b = se.b, e = se.e;
             const int bx = b / Y, by = b - bx * Y, ex = e / Y, ey = e - ex * Y;
             const int span = hor ? ex - bx : ey - by;   // along x at y = by, or along y at x = bx
             cnt = span >= 0 ? span / sp + 1 : 0;
@@ -461,8 +471,8 @@ __device__ __forceinline__ void group_segment_cells(const BArgs& a, const SSeg& 
     }
 }
 template <int U, class F>
-__device__ __forceinline__ void wave_segment_cells(const BArgs& a, const SSeg& g, F f) {
-    group_segment_cells<64, U>(a, g, f);
+__device__ __forceinline__ void wave_segment_cells(const BArgs& a, const SSeg& g, SegEnds se, F f) {
+    group_segment_cells<64, U>(a, g, se, f);
 }
 
 // The neighbour cells (0,-1), (-1,0), (1,0) of a point.
@@ -488,6 +498,7 @@ __global__ void __launch_bounds__(TPB) k_b_claim_rest(BArgs a, int64_t g, const 
         const SNet s = a.sn[i];
         const SSeg sg = a.sg[i];
         const int lane = threadIdx.x & 63;
+        const SegEnds se = segment_ends(a, sg, lane);
         if (lane == 0) nb += 4 + 16 + 24;   // list entry, net and segment records
         for (int k = lane; k < s.npt; k += 64) {
             bool valid[3];
@@ -499,7 +510,7 @@ __global__ void __launch_bounds__(TPB) k_b_claim_rest(BArgs a, int64_t g, const 
                     nb += 4;
                 }
         }
-        wave_segment_cells<1>(a, sg, [&](bool(&valid)[1], int(&q)[1]) {
+        wave_segment_cells<1>(a, sg, se, [&](bool(&valid)[1], int(&q)[1]) {
             if (valid[0]) {
                 atomicMax(&a.map[q[0]], i);
                 nb += 4;
@@ -875,10 +886,26 @@ __global__ void __launch_bounds__(LTPB) k_r_commit(BArgs a, int64_t g, const int
         // round 0's viable nets: the batch end lists those still unassigned
         if (lane == 0 && st[C_ROUND] == 0) a.v0[w] = i;
         if (lane == 0) nb += 4 + 16 + 24;   // list entry, net and segment records
-        bool lost = false;
-        for (int k = lane; k < s.npt; k += 64) {
+        // the first 64 points' neighbours and the segments are read beside the
+        // points, whatever comes of the net
+        const SegEnds se = segment_ends(a, sg, lane);
+        const bool in0 = lane < s.npt;
+        const int p0 = in0 ? a.pt[s.pt0 + lane] : 0;
+        bool valid0[3];
+        int q0[4], m0[3];
+        {
+            int nq[3];
+            point_neighbours(a, in0, p0, valid0, nq);
+            for (int u = 0; u < 3; u++) q0[u] = nq[u];
+            q0[3] = p0;
+        }
+#pragma unroll
+        for (int u = 0; u < 3; u++) m0[u] = valid0[u] ? a.map[q0[u]] : -1;
+        bool lost = in0 && a.map[p0] != i;
+        if (in0) nb += 8;   // point, map cell
+        for (int k = lane + 64; k < s.npt; k += 64) {
             lost = lost || a.map[a.pt[s.pt0 + k]] != i;
-            nb += 8;   // point, map cell
+            nb += 8;
         }
         if (__ballot(lost) != 0) continue;
         if (lane == 0) {
@@ -889,7 +916,11 @@ __global__ void __launch_bounds__(LTPB) k_r_commit(BArgs a, int64_t g, const int
         }
         // several cells a lane at a time: their map loads, then their stamp
         // exchanges, overlap
-        for (int k = lane; k - lane < s.npt; k += 64) {
+        {
+            const bool own[4] = {m0[0] == i, m0[1] == i, m0[2] == i, in0};
+            hit<4>(a, gl, stamp, own, q0, nb);
+        }
+        for (int k = lane + 64; k - lane < s.npt; k += 64) {
             const bool in = k < s.npt;
             const int p = in ? a.pt[s.pt0 + k] : 0;
             bool valid[3], own[4];
@@ -904,7 +935,7 @@ __global__ void __launch_bounds__(LTPB) k_r_commit(BArgs a, int64_t g, const int
             }
             hit<4>(a, gl, stamp, own, q, nb);
         }
-        wave_segment_cells<2>(a, sg, [&](bool(&valid)[2], int(&q)[2]) {
+        wave_segment_cells<2>(a, sg, se, [&](bool(&valid)[2], int(&q)[2]) {
             bool own[2];
 #pragma unroll
             for (int u = 0; u < 2; u++) own[u] = valid[u] && a.map[q[u]] == i;
@@ -1403,6 +1434,7 @@ __global__ void __launch_bounds__(LTPB) k_small_rounds(BArgs a, int64_t g, const
                     const int p = in ? slot[q] - SLOT_BASE : -1;
                     if (p >= 0) atomicMax(&s_map[p], r);
                 };
+                const SegEnds se = segment_ends(a, s.seg, lg);
                 for (int k = lg; k < s.net.npt; k += 16) {
                     bool valid[3];
                     int q[3], p[3];
@@ -1411,7 +1443,7 @@ __global__ void __launch_bounds__(LTPB) k_small_rounds(BArgs a, int64_t g, const
                     for (int u = 0; u < 3; u++)
                         if (valid[u] && p[u] >= 0) atomicMax(&s_map[p[u] - SLOT_BASE], r);
                 }
-                group_segment_cells<16, 1>(a, s.seg, [&](bool(&valid)[1], int(&q)[1]) { claim(valid[0], q[0]); });
+                group_segment_cells<16, 1>(a, s.seg, se, [&](bool(&valid)[1], int(&q)[1]) { claim(valid[0], q[0]); });
             }
             __syncthreads();
             // commits
