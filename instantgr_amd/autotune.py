@@ -10,7 +10,8 @@ results (include/igr.h, igr_tuning):
   dag_waves    waves per net of the DAG kernel (2 or 4)
   track_k      cells per thread of the fused track kernel (4, 8, 16)
   sched_kind   scheduler rounds: active-list (work follows the active nets) or release-driven
-               (work follows the released cells)
+               (work follows the released cells); 0 leaves the choice to the schedule's sizes and
+               runs short lists and last batches in one workgroup
   dag_grid     persistent workgroups of the DAG kernel pulling nets from the batch's work queue
 
 In the terms of a tile shape: nets per workgroup (dag_grid) and waves per net
@@ -41,7 +42,7 @@ CANDIDATES = {
     "track_k": [4, 8, 16],
     "dag_edges": [1],
     "dag_seq": [16],
-    "sched_kind": [1, 2],
+    "sched_kind": [0, 1, 2],
     "dag_grid": [1024, 2048, 4096],
     "lshape_groups": [4],
 }

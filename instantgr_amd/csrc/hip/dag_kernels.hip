@@ -61,8 +61,8 @@ __global__ void k_fill_i32(int* p, int64_t n, int v) {
 
 // precompute_cost_edge: one thread per (edge, from layer, to layer).  A thread
 // walks up to 39 samples of some ten loads each, so a launch is a latency
-// chain: 34 us a batch of 600 nets (175 with one thread per (edge, from layer),
-// over every to layer).
+// chain: 34 us a batch on a 600-net design (175 with one thread per (edge, from
+// layer), over every to layer).
 __global__ void __launch_bounds__(TPB) k_dag_edges(DagArgs a, int64_t edges) {
     int64_t t = (int64_t)blockIdx.x * TPB + threadIdx.x;
     const GridDev& g = a.g;
