@@ -179,15 +179,15 @@ __global__ void __launch_bounds__(TPB) k_lshape_plain(GridDev g, const int* nets
 // bit-identical.  Which child layers a range used is found again on the way
 // down, for the ranges chosen.
 //
-// Nets are short chains of nodes, so a net's time is the latency of a node:
-// the prefix sums and via costs of the next node and its parent edge are
-// loaded while the current one is worked on.  One launch takes a batch: nets
-// of one wave have similar node counts (the host sorts them), and under 3 KB
-// of LDS a net leaves the waves to the registers.  With the layer-range tables
-// in LDS (450 bytes a node), the grid read inside the chain and a launch per
-// node-count class, a batch took 295 us on 200x200 (20k nets, 40 batches), 252
-// us on 800x800 (500k nets, 58 batches) and 315 us on 1237x989 with 11 layers;
-// this kernel takes 56, 68 and 79 us.
+// Nets are short chains of nodes, so a net's time is the latency of a node
+// (some 1350 instructions): the prefix sums and via costs of the next node and
+// its parent edge are loaded while the current one is worked on.  One launch
+// takes a batch: nets of one wave have similar node counts (the device sorts
+// them), and under 3 KB of LDS a net leaves the waves to the registers.  With
+// the layer-range tables in LDS (450 bytes a node), the grid read inside the
+// chain and a launch per node-count class, a batch took 295 us on 200x200 (20k
+// nets, 40 batches), 252 us on 800x800 (500k nets, 58 batches) and 315 us on
+// 1237x989 with 11 layers; this kernel takes 41, 68 and 79 us.
 // ---------------------------------------------------------------------------
 // What a node's step reads from the grid, by lane.
 struct NodeIn {
@@ -196,9 +196,15 @@ struct NodeIn {
     float va, vb;                 // via cut of the lane's layer at the L corners (x, py) and (px, y)
 };
 
+// Batches of at most this many nets leave most of the chip's 1024 SIMDs idle
+// with four nets a wave, and a batch then takes as long as its longest net: a
+// wave takes one net, its four rows up to four nodes of a depth level. Batches
+// of 500 nets 56 -> 41 us; with thousands of nets both are bound by the
+// instructions issued, which one net a wave does not reduce.
+constexpr int64_t LSWAVE_WIDE_NETS = 2048;
 __host__ __device__ constexpr int lswave_net_lds(int L, int cap) { return (cap * (8 * L + 12 + 34) + 15) / 16 * 16; }
 
-template <int L>
+template <int L, bool WIDE>
 __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __restrict__ nets, int64_t n, int cap,
                                                     const int64_t* __restrict__ node_off,
                                                     const int* __restrict__ node, const int* __restrict__ parent,
@@ -209,7 +215,7 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
     // choice made on the way down; by layer, the edge's child layer and the
     // best range's ends; last child and next lower sibling (0: none)
     const int gi = threadIdx.x >> 4, lane = threadIdx.x & 15, s = lane;
-    unsigned char* base = reinterpret_cast<unsigned char*>(s_dyn) + gi * lswave_net_lds(L, cap);
+    unsigned char* base = reinterpret_cast<unsigned char*>(s_dyn) + (WIDE ? 0 : gi * lswave_net_lds(L, cap));
     double* mcp = reinterpret_cast<double*>(base);
     int* pos = reinterpret_cast<int*>(mcp + cap * L);
     int* par = pos + cap;
@@ -218,7 +224,11 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
     uint8_t* range_of = curl_of + 16 * cap;
     uint8_t* child_of = range_of + 16 * cap;
     uint8_t* sib_of = child_of + cap;
-    const int64_t t = (int64_t)blockIdx.x * 4 + gi;
+    // WIDE: the nodes by falling depth, and the ends of each one's level there
+    uint8_t* ord = reinterpret_cast<uint8_t*>(s_dyn) + lswave_net_lds(L, cap);
+    uint8_t* lvl_beg = ord + cap;
+    uint8_t* lvl_end = lvl_beg + cap;
+    const int64_t t = WIDE ? blockIdx.x : (int64_t)blockIdx.x * 4 + gi;
     int nn = 0, net = 0;
     int64_t nb = 0;
     if (t < n) {
@@ -245,14 +255,41 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
         }
         child_of[k] = (uint8_t)c;
         sib_of[k] = (uint8_t)b;
+        if (WIDE) {
+            int d = 0;
+            for (int q = k; q > 0; q = par[q]) d++;
+            pick[k] = d;
+        }
     }
     __syncthreads();
+    if (WIDE) {
+        for (int k = lane; k < nn; k += 16) {
+            const int d = pick[k];
+            int deeper = 0, same = 0, before = 0;
+            for (int q = 0; q < nn; q++) {
+                const int dq = pick[q];
+                deeper += dq > d;
+                same += dq == d;
+                before += dq == d && q > k;
+            }
+            ord[deeper + before] = (uint8_t)k;
+            lvl_beg[deeper + before] = (uint8_t)deeper;
+            lvl_end[deeper + before] = (uint8_t)(deeper + same);
+        }
+        __syncthreads();
+    }
+    // The row's node in the step that starts at 'at' (WIDE: up to four nodes of
+    // a level from there; else node 'at' of the row's own net), -1 for none.
+    auto node_at = [&](int at) {
+        if (!WIDE) return at < nn ? at : -1;
+        return at >= 0 && at < nn && at + gi < lvl_end[at] ? (int)ord[at + gi] : -1;
+    };
     const int l = s - 1;                               // the lane's layer
     const bool on = s >= 1 && s <= L;
     const int dl = layer_dir(l & 15, g.DIR);
     auto fetch = [&](int i) {
         NodeIn in{0, 0, 0, 0, 0};
-        if (i >= nn) return in;
+        if (i < 0) return in;
         const int v = pos[i] % XY, x = v / Y, y = v - x * Y;
         if (lane < L - 1) in.vl = g.vcost[gidx(g, lane, x, y)];
         if (i > 0 && on) {
@@ -270,10 +307,14 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
         return in;
     };
     const double PINF = __longlong_as_double(0x7ff0000000000000LL);
-    NodeIn in = fetch(nmax - 1);
-    for (int i = nmax - 1; i >= 0; i--) {
-        const NodeIn next = i > 0 ? fetch(i - 1) : NodeIn{0, 0, 0, 0, 0};
-        const bool act = i < nn;
+    int step = WIDE ? 0 : nmax - 1;
+    NodeIn in = fetch(node_at(step));
+    while (WIDE ? step < nn : step >= 0) {
+        const int after = WIDE ? min(step + 4, (int)lvl_end[step]) : step - 1;
+        const NodeIn next = (WIDE ? after < nn : after >= 0) ? fetch(node_at(after)) : NodeIn{0, 0, 0, 0, 0};
+        const int own_node = node_at(step), i = max(own_node, 0);
+        const bool act = own_node >= 0;
+        const bool root = WIDE ? step == nn - 1 : step == 0;
         const int v = act ? pos[i] : 0;
         const int pl = v / XY;                         // the pin's layer, L for none
         // cost[low - 1] of the range [low, s]
@@ -322,7 +363,7 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
         });
         if (code) code |= (s + __builtin_ctzll(at >> (threadIdx.x & 63))) << 4;
         if (act && on) range_of[i * 16 + l] = (uint8_t)code;
-        if (i == 0) {
+        if (root) {
             // the root's range: the smallest cost, ties to the smaller low,
             // then the smaller hi (every range through the best layer is one
             // of the candidates, so the row's smallest (cost, range) is it)
@@ -334,7 +375,7 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
                 const int oc = __shfl_xor(cd, o, 16);
                 if (om < m || (om == m && oc < cd)) { m = om; cd = oc; }
             }
-            if (lane == 0 && nn > 0) pick[0] = (cd >> 4) | (cd & 15) << 4;
+            if (lane == 0 && act) pick[0] = (cd >> 4) | (cd & 15) << 4;
             break;
         }
         // edge to the parent: cost by parent layer and the child layer it uses
@@ -384,12 +425,17 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
         }
         __syncthreads();
         in = next;
+        step = after;
     }
     __syncthreads();
     // Top-down (parents first): within the parent's range the lowest of the
     // cheapest layers, the child layer its edge uses, and that layer's range.
-    for (int i = 1; i < nmax; i++) {
-        const bool act = i < nn;
+    for (int at2 = WIDE ? nn - 2 : 1; WIDE ? at2 >= 0 : at2 < nmax;) {
+        const int first = WIDE ? max((int)lvl_beg[at2], at2 - 3) : at2;
+        const int node2 = WIDE ? (first + gi <= at2 ? (int)ord[first + gi] : -1) : at2 < nn ? at2 : -1;
+        const int i = max(node2, 0);
+        const bool act = node2 >= 0;
+        at2 = WIDE ? first - 1 : at2 + 1;
         const int up = act ? pick[par[i]] : 0;
         const int low = up & 15, hi = up >> 4 & 15;
         double c = act && s >= low && s <= hi ? mcp[i * L + l] : PINF;
@@ -408,7 +454,7 @@ __global__ void __launch_bounds__(64) k_lshape_wave(GridDev g, const int* __rest
         }
         __syncthreads();
     }
-    if (t >= n) return;
+    if (t >= n || (WIDE && gi != 0)) return;
     // Route pairs in node order: the node's via stack, then the edge to its
     // parent (one piece, or wire-via-wire for an L).
     int* r = routes + route_off[net];
@@ -480,17 +526,20 @@ void launch_lshape_wave(igr_ctx* c, const int* d_nets, int64_t n, int nodes, int
     if (nodes < 1 || nodes > LSWAVE_MAX_NODES) throw std::runtime_error("L-shape node count out of range");
     KScope ks(c, K_LSHAPE, bytes);
     NetsDev& N = c->nets;
-    const unsigned grid = (unsigned)((n + 3) / 4);
+    const bool wide = n <= LSWAVE_WIDE_NETS;
+    const unsigned grid = (unsigned)(wide ? n : (n + 3) / 4);
+#define ARGS c->g, d_nets, n, nodes, N.node_off.p, N.node.p, N.parent.p, N.route_off.p, N.routes.p, stamp
 #define CASE(LV)                                                                                                    \
     case LV:                                                                                                        \
-        k_lshape_wave<LV><<<grid, 64, 4 * lswave_net_lds(LV, nodes), c->stream>>>(                                  \
-            c->g, d_nets, n, nodes, N.node_off.p, N.node.p, N.parent.p, N.route_off.p, N.routes.p, stamp);          \
+        if (wide) k_lshape_wave<LV, true><<<grid, 64, lswave_net_lds(LV, nodes) + 3 * nodes, c->stream>>>(ARGS);     \
+        else k_lshape_wave<LV, false><<<grid, 64, 4 * lswave_net_lds(LV, nodes), c->stream>>>(ARGS);                \
         break;
     switch (c->g.L) {
         CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12)
     default: throw std::runtime_error("unsupported routing layer count");
     }
 #undef CASE
+#undef ARGS
     HIP_OK(hipGetLastError());
 }
 
