@@ -76,7 +76,7 @@ struct Staging {
     char* mem = nullptr;
     hipEvent_t done[SLOTS] = {};
     ~Staging();
-    void open();
+    void open(int device);
     char* slot(int k) { return mem + k * SLOT_BYTES; }
 };
 

@@ -17,15 +17,20 @@ Staging::~Staging() {
     if (mem) (void)hipHostFree(mem);
 }
 
-void Staging::open() {
+// The events belong to the context's device, whichever the caller has current.
+void Staging::open(int device) {
     if (mem) return;
+    int cur = -1;
+    HIP_OK(hipGetDevice(&cur));
+    if (cur != device) HIP_OK(hipSetDevice(device));
     char* m = nullptr;
-    HIP_OK(hipHostMalloc(&m, (size_t)SLOTS * SLOT_BYTES));
-    for (hipEvent_t& e : done)
-        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-            (void)hipHostFree(m);
-            throw std::runtime_error("hipEventCreate failed");
-        }
+    bool ok = hipHostMalloc(&m, (size_t)SLOTS * SLOT_BYTES) == hipSuccess;
+    for (hipEvent_t& e : done) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+    if (cur != device) (void)hipSetDevice(cur);
+    if (!ok) {
+        if (m) (void)hipHostFree(m);
+        throw std::runtime_error("no pinned memory or events for large copies");
+    }
     mem = m;
 }
 
@@ -37,7 +42,7 @@ static void over_chunks(int device, int64_t bytes, F&& chunk) {
     int T = std::max(1, std::min(std::min(host_threads(), Staging::THREADS), (int)std::min<int64_t>(Staging::SLOTS, chunks)));
     while (Staging::SLOTS % T) T--;
     igr::parallel_ranges(T, T, [&](int64_t a, int64_t b, int) {
-        HIP_OK(hipSetDevice(device));
+        if (T > 1) HIP_OK(hipSetDevice(device));   // a thread of its own; one chunk is copied by the caller
         for (int64_t t = a; t < b; t++)
             for (int64_t k = t; k < chunks; k += T) {
                 const int64_t at = k * Staging::SLOT_BYTES;
@@ -54,7 +59,7 @@ void copy_to_host(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipStre
         return;
     }
     std::lock_guard<std::mutex> lk(g.mu);
-    g.open();
+    g.open(c->device);
     const auto start = [&](int slot, int64_t at) {
         HIP_OK(hipMemcpyAsync(g.slot(slot), static_cast<const char*>(src) + at,
                               std::min<int64_t>(Staging::SLOT_BYTES, bytes - at), hipMemcpyDeviceToHost, s));
@@ -79,7 +84,7 @@ void copy_to_device(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipSt
         return;
     }
     std::lock_guard<std::mutex> lk(g.mu);
-    g.open();
+    g.open(c->device);
     over_chunks(c->device, bytes, [&](int slot, int64_t at, int64_t len) {
         HIP_OK(hipEventSynchronize(g.done[slot]));
         std::memcpy(g.slot(slot), static_cast<const char*>(src) + at, len);
