@@ -260,7 +260,8 @@ typedef struct igr_tuning {
     int sched_kind;     /* scheduler rounds after the first of a batch: 1 active-list (work follows the
                            active nets), 2 release-driven (work follows the released cells); built-in
                            choice 2 from 150k scheduled nets where 25 of them or more list a cell on
-                           average */
+                           average, and one workgroup for lists (and last batches) of at most 2048
+                           nets that fit its LDS, which 1 and 2 leave out */
     int presum_k;       /* plain form's prefix-sum kernel: cells per thread, 4, 8 or 16 */
     int dag_grid;       /* DAG kernel: persistent workgroups pulling a batch's nets from its work queue */
     int lshape_groups;  /* 1, 2 or 4; the pattern DP always takes four nets a wave, the field has no effect */
