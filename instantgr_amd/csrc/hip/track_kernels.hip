@@ -15,9 +15,11 @@
 //   3. rip-up of the next batch: demand -= covering wire count, timestamp =
 //      rip stamp on covered cells, then the gated via cuts subtract;
 //   4. wcost / vcost from the new demand, FP64 prefix sums of wcost.
-// Demand changes by integers and halves, so the result equals the sequential
-// one.  A track no scatter touched keeps its demand and so its costs: the
-// routing kernels and the rip-up scatter flag every track they write into.
+// Demand changes by integers and halves, so from demand on the half grid, which
+// every pass leaves, the result equals the sequential one; from any other float
+// demand the FP32 sums round in the order above, a batch's count at a time.  A
+// track no scatter touched keeps its demand and so its costs: the routing
+// kernels and the rip-up scatter flag every track they write into.
 #include "dag_dev.h"
 #include "igr_ctx.hpp"
 #include "scan.h"
@@ -281,9 +283,9 @@ __global__ void __launch_bounds__(1024) k_track_fused(GridDev g, int s_c, int s_
     for (int j = 0; j < K; j++)
         if (inc[j] | gv[j] | dec[j] | cov[j] | gr[j]) clr |= 1u << j;
     block_sums<K>(inc, dec, cov, sh_tot, nw);
-    // commit of the wires, gate of the vias (s_c), then the rip-up's (s_r):
-    // the demand changes are integers and halves, so their order is free, but
-    // the timestamps gate in sequence
+    // commit of the wires, gate of the vias (s_c), then the rip-up's (s_r).
+    // Demand that a caller set may be any float, so its sums keep the passes'
+    // order too: wires and vias of the commit, then those of the rip-up.
 #pragma unroll
     for (int j = 0; j < K; j++) {
         const int p = p0 + j;
@@ -293,7 +295,8 @@ __global__ void __launch_bounds__(1024) k_track_fused(GridDev g, int s_c, int s_
             if (ts[j] != s_c) { ts[j] = s_c; wr_ts |= 1u << j; }
         }
         if (ts[j] >= s_c) gv[j] = 0;
-        if (p <= len - 2 && dec[j] > 0) { dem[j] -= (float)dec[j]; wr_dem |= 1u << j; }
+        if (p <= len - 2 && dec[j] > 0) wr_dem |= 1u << j;
+        else dec[j] = 0;
         if (p < len && cov[j] > 0 && ts[j] != s_r) { ts[j] = s_r; wr_ts |= 1u << j; }
         if (ts[j] >= s_r) gr[j] = 0;
         if (gv[j] | gr[j]) wr_dem |= (3u << j) >> 1;   // edges j-1 and j of this thread
@@ -309,6 +312,8 @@ __global__ void __launch_bounds__(1024) k_track_fused(GridDev g, int s_c, int s_
     }
     if (gvn | grn) wr_dem |= 1u << (K - 1);
     apply_vias<K>(dem, gv, gvn, len, 1.0f);
+#pragma unroll
+    for (int j = 0; j < K; j++) dem[j] -= (float)dec[j];
     apply_vias<K>(dem, gr, grn, len, -1.0f);
 #pragma unroll
     for (int j = 0; j < K; j++) {
