@@ -396,14 +396,14 @@ def run_form(design, form, name, a, tuning, budget_s, t_origin):
     for k in range(a.steps):
         if k > 0 and est is not None and time.perf_counter() - t_origin + est > budget_s:
             break
+        if last is not None:
+            last[0].close()   # two contexts of configuration 2 do not fit the device
         r, st = one_step(design, form, a.rrr, a.threads, tuning=tun)
         times.append(st["step_s"])
         est = st["step_s"]
         free, total = r.device_memory()
         _progress("%s step %d: %.3f s (device memory in use %.1f of %.1f GB)"
                   % (name, k, st["step_s"], (total - free) / 1e9, total / 1e9))
-        if last is not None:
-            last[0].close()
         last = (r, st)
     r, st = last
     routes = r.routes_flat()
