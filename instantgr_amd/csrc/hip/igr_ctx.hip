@@ -790,7 +790,7 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     D.cost_edges.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
     D.change.alloc(std::max<int64_t>(1, mx_edges) * ND * ND);
     NetsDev& N = c->nets;
-    int* rbase = N.new_dag_routes(dag_route_slot(NN, n));
+    PassRoutes routes(N, s, dag_route_slot(NN, n));
     const double tp = now_s();
 
     // Batch b: DAG routing (scattering its wires, vias and dirty flags), the
@@ -824,10 +824,10 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
             }
         }
         sg.launch();
+        HIP_OK(hipStreamSynchronize(s));
+        routes.adopt(nets, n, loop_threads(n), [&](int64_t i) { return dag_route_slot(dg->node_off[i], i); });
         bs.check();
     }
-    HIP_OK(hipStreamSynchronize(s));
-    N.adopt(nets, n, rbase, loop_threads(n), [&](int64_t i) { return dag_route_slot(dg->node_off[i], i); });
     const double t2 = now_s();
     c->last_dag_prep_s = tp - t1;
     c->last_dag_prep_parts[0] = t_meta - t1;     // routing-order bases, batch bounds, small uploads
@@ -1054,7 +1054,7 @@ int igr_dag_pass(igr_ctx* c, const int* nets, int64_t n, int mode, int form, con
         D.cost_edges.alloc(std::max<int64_t>(1, mx_edges) * LL);
         D.best_change.alloc(std::max<int64_t>(1, mx_edges) * LL);
         NetsDev& N = c->nets;
-        int* rbase = N.new_dag_routes(route_slot[n]);
+        PassRoutes routes(N, s, route_slot[n]);
         double tp = now_s();
 
         double t_note = tp;
@@ -1078,7 +1078,7 @@ int igr_dag_pass(igr_ctx* c, const int* nets, int64_t n, int mode, int form, con
             HIP_OK(hipStreamSynchronize(s));
         }
         HIP_OK(hipStreamSynchronize(s));
-        N.adopt(rnets.data(), n, rbase, 1, [&](int64_t r) { return route_slot[r]; });
+        routes.adopt(rnets.data(), n, 1, [&](int64_t r) { return route_slot[r]; });
         double t2 = now_s();
         c->last_dag_prep_s = tp - t1;
         c->last_dag_prep_parts[0] = t_fill - t1;

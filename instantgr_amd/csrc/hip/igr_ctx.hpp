@@ -7,9 +7,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
-#include <mutex>
+#include <utility>
 #include <vector>
 
 #define HIP_OK(expr)                                                                               \
@@ -101,17 +103,33 @@ struct NetsDev {
     int max_nodes = 0;
     DevBuf<int>* spare = nullptr;           // one retired buffer, for a next pass of about its size
     ~NetsDev() { clear_dag_routes(); }
-    // The routes buffer of a new pass.
+    // The routes buffer of a new pass, which ends with adopt() or abandon().
     int* new_dag_routes(int64_t words) {
         const bool fits = spare && (int64_t)spare->n >= words && (int64_t)spare->n / 4 <= words;
-        dag_routes.push_back(fits ? spare : new DevBuf<int>());
+        std::unique_ptr<DevBuf<int>> b(fits ? spare : new DevBuf<int>());
         if (fits) spare = nullptr;
-        dag_routes.back()->alloc(words);
-        return dag_routes.back()->p;
+        b->alloc(words);
+        dag_routes.push_back(b.get());
+        return b.release()->p;
     }
+    // The newest retired buffer is the spare: the next pass is most likely of its size.
     void retire(DevBuf<int>* b) {
-        if (!spare && b->n <= SPARE_WORDS) spare = b;
-        else delete b;
+        if (b->n <= SPARE_WORDS) std::swap(spare, b);
+        delete b;
+    }
+    // The pass of the newest buffer failed: its nets keep the routes they had.
+    // Its kernels may have moved their pointers, so the device gets them back
+    // before the buffer goes; a device that cannot take them keeps the buffer.
+    void abandon(hipStream_t s) {
+        if (dag_live.size() == dag_routes.size() && dag_live.back() > 0) return;   // adopt() failed half way
+        if (hipStreamSynchronize(s) == hipSuccess &&
+            hipMemcpy(rptr.p, h_rptr.data(), sizeof(int*) * h_rptr.size(), hipMemcpyHostToDevice) == hipSuccess) {
+            retire(dag_routes.back());
+            dag_routes.pop_back();
+        } else {
+            dag_live.resize(dag_routes.size(), 0);
+            dag_live.back() = 1;   // of no net
+        }
     }
     void clear_dag_routes() {
         delete spare;
@@ -138,9 +156,10 @@ struct NetsDev {
     void adopt(const int* rnets, int64_t n, int* rbase, int threads, Slot slot) {
         const int k = (int)dag_routes.size() - 1;
         dag_live.resize(dag_routes.size(), 0);
-        std::vector<std::vector<int64_t>> left(threads);   // nets that leave each buffer
+        // nets that leave each buffer
+        std::vector<std::vector<int64_t>> left(threads, std::vector<int64_t>(dag_routes.size(), 0));
+        dag_live[k] += n;
         igr::parallel_ranges(n, threads, [&](int64_t a, int64_t b, int t) {
-            left[t].assign(dag_routes.size(), 0);
             for (int64_t r = a; r < b; r++) {
                 const int net = rnets[r];
                 if (h_rbuf[net] >= 0) left[t][h_rbuf[net]]++;
@@ -149,7 +168,6 @@ struct NetsDev {
                 h_rbuf[net] = k;
             }
         });
-        dag_live[k] += n;
         for (const auto& v : left)
             for (size_t j = 0; j < v.size(); j++) dag_live[j] -= v[j];
         for (size_t j = 0; j < dag_routes.size(); j++)
@@ -195,6 +213,27 @@ struct alignas(16) DagEdge {
 
 struct alignas(16) DagSize {
     int nodes, edges, slots, levels;
+};
+
+// A pass's routes buffer: abandoned unless the pass gets as far as adopt().
+class PassRoutes {
+    NetsDev& nets;
+    hipStream_t s;
+    bool open = true;
+
+public:
+    int* const base;
+    PassRoutes(NetsDev& nets_, hipStream_t s_, int64_t words) : nets(nets_), s(s_), base(nets.new_dag_routes(words)) {}
+    PassRoutes(const PassRoutes&) = delete;
+    PassRoutes& operator=(const PassRoutes&) = delete;
+    ~PassRoutes() {
+        if (open) nets.abandon(s);
+    }
+    template <class Slot>
+    void adopt(const int* rnets, int64_t n, int threads, Slot slot) {
+        nets.adopt(rnets, n, base, threads, slot);
+        open = false;
+    }
 };
 
 // One rip-up-and-reroute pass on the device: DAGs of the rerouted nets in
