@@ -252,7 +252,7 @@ typedef struct igr_tuning {
                            (built-in) */
     int sched_group;    /* lanes per net in the scheduler's claim and viability kernels: 4, 8 or 16 */
     int sched_chunk;    /* scheduler rounds enqueued between host checks, 1..256 */
-    int dag_order;      /* workgroup order of a DAG batch: 1 deepest DAG first, 2 routing order */
+    int dag_order;      /* workgroup order of a DAG batch: 1 deepest DAG first, 2 the order of the net list */
     int dag_waves;      /* waves per net of the DAG kernel, 2 or 4 */
     int track_k;        /* fused track kernel: cells per thread, 4, 8 or 16 */
     int dag_edges;      /* 1 or 2; one kernel prices the DAG edges, the field has no effect */

@@ -6,7 +6,7 @@ results (include/igr.h, igr_tuning):
   sched_group  lanes per net in the scheduler's claim and viability kernels
   sched_chunk  scheduler rounds enqueued between host checks
   graph        one hipGraph per pass for the batch sequence, or stream launches
-  dag_order    workgroup order of a DAG batch (deepest DAG first, or routing order)
+  dag_order    workgroup order of a DAG batch (deepest DAG first, or the order of the net list)
   dag_waves    waves per net of the DAG kernel (2 or 4)
   track_k      cells per thread of the fused track kernel (4, 8, 16)
   sched_kind   scheduler rounds: active-list (work follows the active nets) or release-driven

@@ -592,7 +592,7 @@ __device__ void route_net(const NetArgs& a, int64_t r, uint64_t* K, uint8_t* R, 
 }
 
 // Workgroups pull the batch's nets from its queue (one counter per batch,
-// zero at the pass start) in routing order, deepest DAG first, and exit when the
+// zero at the pass start) in launch order (dag_order), and exit when the
 // counter passes n.
 template <int L, int NW>
 __global__ void __launch_bounds__(64 * NW) k_dag_net(NetArgs a) {

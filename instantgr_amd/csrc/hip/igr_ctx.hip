@@ -702,7 +702,7 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
     const double t1 = now_s();
 
     // Routing order: batch nb-1 first, inside a batch the deepest DAG first
-    // (dag_order 1) or as they come (2).
+    // (dag_order 1) or in list order (2).
     const bool deep_first = (c->tune.dag_order ? c->tune.dag_order : DEF_DAG_ORDER) == 1;
     std::vector<DagBound> bound(nb + 1);
     int any_big = 0;
@@ -740,23 +740,25 @@ void dag_pass_batched(igr_ctx* c, const int* nets, int64_t n, int mode, const ig
         mx_slots = std::max(mx_slots, B.slot1 - B.slot0);
     }
     // IGR_DAG_TRACE=<file>: append one line per batch (nets, nodes, edges,
-    // slots, deepest DAG's levels, largest DAG's nodes).
+    // slots, deepest DAG's levels, largest DAG's nodes, neighbours in the launch
+    // order that are not in the order of the net list).
     if (const char* tp = std::getenv("IGR_DAG_TRACE")) {
         if (FILE* f = std::fopen(tp, "a")) {
-            std::fprintf(f, "# DAG pass: %lld nets, %d batches\nbatch nets nodes edges slots levels max_nodes\n",
+            std::fprintf(f, "# DAG pass: %lld nets, %d batches\nbatch nets nodes edges slots levels max_nodes unordered\n",
                          (long long)n, nb);
             for (int b = 0; b < nb; b++) {
                 const DagBatch& B = batches[b];
                 int64_t mxn = 0;
-                int mxl = 0;
+                int mxl = 0, unordered = 0;
                 for (int64_t r = B.net0; r < B.net1; r++) {
                     const int64_t i = rorder[r];
+                    unordered += r > B.net0 && rorder[r - 1] > i;
                     mxn = std::max(mxn, dg->node_off[i + 1] - dg->node_off[i]);
                     for (int64_t k = dg->node_off[i]; k < dg->node_off[i + 1]; k++) mxl = std::max(mxl, dg->depth[k] + 1);
                 }
-                std::fprintf(f, "%d %lld %lld %lld %lld %d %lld\n", b, (long long)(B.net1 - B.net0),
+                std::fprintf(f, "%d %lld %lld %lld %lld %d %lld %d\n", b, (long long)(B.net1 - B.net0),
                              (long long)(B.node1 - B.node0), (long long)(B.edge1 - B.edge0),
-                             (long long)(B.slot1 - B.slot0), mxl, (long long)mxn);
+                             (long long)(B.slot1 - B.slot0), mxl, (long long)mxn, unordered);
             }
             std::fclose(f);
         }
