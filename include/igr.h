@@ -264,7 +264,9 @@ typedef struct igr_tuning {
                            nets that fit its LDS, which 1 and 2 leave out */
     int presum_k;       /* plain form's prefix-sum kernel: cells per thread, 4, 8 or 16 */
     int dag_grid;       /* DAG kernel: persistent workgroups pulling a batch's nets from its work queue */
-    int lshape_groups;  /* 1, 2 or 4; the pattern DP always takes four nets a wave, the field has no effect */
+    int lshape_groups;  /* plain form: 1 gives the pattern DP a thread per net, the reference's launch structure, for
+                           checks of the row kernel that both forms use otherwise; 2 and 4 have no effect, and none
+                           has any in the batched form */
 } igr_tuning;
 int igr_set_tuning(igr_ctx* ctx, const igr_tuning* t);
 /* The values in force (built-in choices resolved, per-pass choices as 0). */

@@ -15,8 +15,8 @@ results (include/igr.h, igr_tuning):
   dag_grid     persistent workgroups of the DAG kernel pulling nets from the batch's work queue
 
 In the terms of a tile shape: nets per workgroup (dag_grid) and waves per net
-(dag_waves).  dag_edges, dag_seq and lshape_groups have no effect and keep one
-value.
+(dag_waves).  dag_edges and dag_seq have no effect and keep one value, and so
+does lshape_groups, which has one in the plain form only.
 
 `tune` measures them on a design (normally a reduced sample of the production
 design from the same generator) by coordinate descent: each field in turn takes

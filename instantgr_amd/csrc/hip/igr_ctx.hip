@@ -306,21 +306,25 @@ void ensure_scratch(igr_ctx* c, int64_t nodes) {
     c->scratch.lr.alloc(nodes);
 }
 
-// Device work of one plain batch: the reference sequence of launches.
 int largest_net(igr_ctx* c, const int* nets, int64_t n) {
     int64_t m = 1;
     for (int64_t i = 0; i < n; i++) m = std::max(m, c->nets.h_node_off[nets[i] + 1] - c->nets.h_node_off[nets[i]]);
     return (int)m;
 }
 
-// 'nodes': the batch's largest node count.  Up to LSWAVE_MAX_NODES the row
-// kernel takes it (on a 600-net design 47 us a batch, 434 with a thread a net).
+// Device work of one plain batch: the reference sequence of launches.  'nodes':
+// the batch's largest node count.  Up to LSWAVE_MAX_NODES the row kernel takes
+// it (on a 600-net design 47 us a batch, 434 with a thread a net), which the
+// batched form uses too; lshape_groups 1 keeps the reference's thread a net, so
+// that the two forms share no pattern kernel.
 void plain_batch(igr_ctx* c, const int* d_nets, const int64_t* d_off, int64_t n, int nodes, double lbytes = 0) {
     int stamp = ++c->stamp;
     launch_update_cost(c);
     launch_presum(c);
-    if (nodes <= LSWAVE_MAX_NODES) launch_lshape_wave(c, d_nets, n, nodes, stamp, lbytes);
-    else launch_lshape_plain(c, d_nets, d_off, n, stamp, lbytes);
+    if (nodes <= LSWAVE_MAX_NODES && c->tune.lshape_groups != 1)
+        launch_lshape_wave(c, d_nets, n, nodes, stamp, lbytes);
+    else
+        launch_lshape_plain(c, d_nets, d_off, n, stamp, lbytes);
     launch_wire_commit(c, stamp);
     launch_via_commit(c, d_nets, n, stamp, 1);
 }
