@@ -183,11 +183,12 @@ __global__ void __launch_bounds__(TPB) k_lshape_plain(GridDev g, const int* nets
 // (some 1350 instructions): the prefix sums and via costs of the next node and
 // its parent edge are loaded while the current one is worked on.  One launch
 // takes a batch: nets of one wave have similar node counts (the device sorts
-// them), and under 3 KB of LDS a net leaves the waves to the registers.  With
+// them), and at most 3.4 KB of LDS a net (24 nodes, 12 layers; 2.8 with 9)
+// leave the waves to the registers.  With
 // the layer-range tables in LDS (450 bytes a node), the grid read inside the
 // chain and a launch per node-count class, a batch took 295 us on 200x200 (20k
 // nets, 40 batches), 252 us on 800x800 (500k nets, 58 batches) and 315 us on
-// 1237x989 with 11 layers; this kernel takes 41, 68 and 79 us.
+// 1237x989 with 11 layers; this kernel takes 43, 71 and 80 us.
 // ---------------------------------------------------------------------------
 // What a node's step reads from the grid, by lane.
 struct NodeIn {
@@ -198,10 +199,13 @@ struct NodeIn {
 
 // Batches of at most this many nets leave most of the chip's 1024 SIMDs idle
 // with four nets a wave, and a batch then takes as long as its longest net: a
-// wave takes one net, its four rows up to four nodes of a depth level. Batches
-// of 500 nets 56 -> 41 us; with thousands of nets both are bound by the
-// instructions issued, which one net a wave does not reduce.
-constexpr int64_t LSWAVE_WIDE_NETS = 2048;
+// wave takes one net, its four rows up to four nodes of a depth level.  Larger
+// batches are bound by the instructions issued, which one net a wave does not
+// reduce.  Four nets a wave against one, us a launch inside pattern passes with
+// 9 layers, by the batch's nets: up to 512 43 / 32, 513..1024 70 / 49, 1025..2048
+// 76 / 50, 3073..4096 78 / 64, 4097..5120 83 / 76, 5121..6144 86 / 89, 8193..9216
+// 94 / 107; with 11 layers the two meet near 11000.
+constexpr int64_t LSWAVE_WIDE_NETS = 5120;
 __host__ __device__ constexpr int lswave_net_lds(int L, int cap) { return (cap * (8 * L + 12 + 34) + 15) / 16 * 16; }
 
 template <int L, bool WIDE>
