@@ -259,7 +259,7 @@ typedef struct igr_tuning {
     int dag_seq;        /* one kernel runs every DAG level, the field has no effect */
     int sched_kind;     /* scheduler rounds after the first of a batch: 1 active-list (work follows the
                            active nets), 2 release-driven (work follows the released cells); built-in
-                           choice 2 from 150k scheduled nets where 25 of them or more list a cell on
+                           choice 2 from 175k scheduled nets where 28 of them or more list a cell on
                            average, and one workgroup for lists (and last batches) of at most 2048
                            nets that fit its LDS, which 1 and 2 leave out */
     int presum_k;       /* plain form's prefix-sum kernel: cells per thread, 4, 8 or 16 */

@@ -60,12 +60,19 @@ constexpr int TPB = 256;
 constexpr int LTPB = 1024;
 constexpr int ROUNDS = 30;        // rounds per batch (src/database_cuda.hpp:612)
 // Release-driven rounds where the cells' lists hold this many nets on average
-// and the nets are this many, active-list rounds elsewhere.  Scheduler time of
-// the active-list rounds against the release-driven ones, by (nets, list
-// length): (24k, 26) 41 / 55 ms, (125k, 20) 268 / 283, (137k, 51) 140 / 141,
-// (199k, 70) 521 / 473, (321k, 29) 429 / 395, (561k, 34) 282 / 263, (1.59M, 16)
-// 111 / 125, (3.0M, 30) 293 / 281.
-constexpr int64_t SCHED_RELEASE_NETS = 150000, SCHED_RELEASE_LIST = 25;
+// and the nets are this many, active-list rounds elsewhere.  Their rounds cost
+// more each but follow the released cells, so they pay where a congested design
+// needs many batches.  Scheduler ms of the active-list rounds against the
+// release-driven ones, by (nets, list length).  Detour footprints of congested
+// designs: (133k, 43) 285 / 289, (181k, 41) 473 / 439, (207k, 42) 545 / 495,
+// (254k, 40) 678 / 589, (386k, 34) 535 / 463, (390k, 28) 383 / 372, (401k, 46)
+// 929 / 746, (497k, 28) 410 / 393.  Pattern footprints of such designs: (171k, 42)
+// 58 / 68, (225k, 34) 82 / 91, (448k, 37) 213 / 208, (602k, 32) 227 / 223, (604k,
+// 26) 155 / 166, (609k, 28) 170 / 176, (611k, 38) 304 / 281, (716k, 39) 330 / 298,
+// (2.1M, 27) 207 / 209.  Even designs have long lists but few batches and lose a
+// tenth above the line: (314k, 48) 158 / 175, (405k, 43) 63 / 74, (474k, 48) 192 /
+// 212; below it (219k, 24) 73 / 98, (438k, 24) 97 / 122.
+constexpr int64_t SCHED_RELEASE_NETS = 175000, SCHED_RELEASE_LIST = 28;
 
 // control state words (two slots of C_WORDS, then the placed-net counter).
 // C_NU / C_UL: length and buffer of the nets round 0 tests.  Active-list
