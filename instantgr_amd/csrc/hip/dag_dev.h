@@ -1,5 +1,5 @@
-// Device definitions shared by the two forms of the detour-DAG routing
-// kernels (src/Lshape_route_detour.hpp).
+// Device definitions shared by the two forms of the detour-DAG routing kernels
+// (src/Lshape_route_detour.hpp); the pattern kernels take the wire segments'.
 #pragma once
 #include "igr_dev.h"
 

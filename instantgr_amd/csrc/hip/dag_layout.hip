@@ -32,7 +32,7 @@ __global__ void __launch_bounds__(WG) k_dag_layout(DagLayoutArgs a) {
     const int64_t r = blockIdx.x;
     const int lane = threadIdx.x;
     const int64_t i = a.rorder[r];
-    const int64_t b0 = a.node_off[i], e0 = a.par_off[b0];
+    const int64_t b0 = a.node_off[i];
     const int nn = (int)(a.node_off[i + 1] - b0);
     const int64_t g0 = a.nbase[r], ge0 = a.ebase[r];
     const int nl = (int)(a.lbase[r + 1] - a.lbase[r]);

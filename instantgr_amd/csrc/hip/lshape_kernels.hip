@@ -8,6 +8,7 @@
 // reference exactly: FP64 accumulation in the same order (sequential via
 // sums, children added in decreasing node order), strict '<' keeping the
 // first minimum and '<=' in the layer-range prefix minimum.
+#include "dag_dev.h"
 #include "igr_ctx.hpp"
 #include "row.h"
 
@@ -16,25 +17,6 @@ namespace igr_dev {
 namespace {
 
 constexpr int TPB = 256;
-
-__device__ __forceinline__ double wseg(const GridDev& g, int l, int xmin, int xmax, int ymin, int ymax) {
-    return g.presum[gidx(g, l, xmax, ymax)] - g.presum[gidx(g, l, xmin, ymin)];
-}
-
-// Difference-array form of one wire segment (src/graph.hpp:105-117).
-__device__ __forceinline__ void add_segment(const GridDev& g, int l, int minx, int maxx, int miny, int maxy,
-                                            int stamp) {
-    atomicAdd(&g.pre[gidx(g, l, minx, miny)], 1);
-    if (g.dirty) g.dirty[track_id(g, l, minx, miny)] = 1;
-    if (minx == maxx) {
-        atomicAdd(&g.pre[gidx(g, l, minx, maxy)], -1);
-        g.ts[gidx(g, l, minx, maxy)] = stamp;
-    }
-    if (miny == maxy) {
-        atomicAdd(&g.pre[gidx(g, l, maxx, miny)], -1);
-        g.ts[gidx(g, l, maxx, miny)] = stamp;
-    }
-}
 
 template <int L>
 __global__ void __launch_bounds__(TPB) k_lshape_plain(GridDev g, const int* nets, const int64_t* scr_off, int64_t n,
