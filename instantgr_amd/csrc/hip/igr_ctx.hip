@@ -483,18 +483,6 @@ static __global__ void __launch_bounds__(256) k_read_route(const int* src, int r
 
 const int* read_route(igr_ctx* c, const int* src, int64_t rc) {
     Mailbox& m = c->mail;
-    if (!m.word) {
-        int* w = nullptr;
-        void* d = nullptr;
-        HIP_OK(hipHostMalloc(&w, sizeof(int) * (MAIL_HEAD + MAIL_WORDS), hipHostMallocMapped | hipHostMallocCoherent));
-        if (hipHostGetDevicePointer(&d, w, 0) != hipSuccess) {
-            (void)hipHostFree(w);
-            throw std::runtime_error("route mailbox is not visible to the device");
-        }
-        std::memset(w, 0, sizeof(int) * (MAIL_HEAD + MAIL_WORDS));
-        m.word = w;
-        m.dev = static_cast<int*>(d);
-    }
     const int number = m.reads = m.reads == INT_MAX ? 1 : m.reads + 1;
     k_read_route<<<1, 256, 0, c->stream>>>(src, (int)rc, m.dev, number);
     HIP_OK(hipGetLastError());
@@ -520,13 +508,15 @@ int igr_get_route(igr_ctx* c, int net, int* buf, int cap, int* len) {
         };
         // A kernel writes the route into host memory in 9 us; a copy of the
         // slot to pageable memory and a wait took 23.  It stays for a route
-        // larger than the mailbox and for callers on another device (a launch
-        // needs the context's, a copy does not).
+        // larger than the mailbox, for callers on another device (a launch needs
+        // the context's, a copy does not) and where there is no pinned memory.
         int cur = -1;
         if (rc <= MAIL_WORDS && hipGetDevice(&cur) == hipSuccess && cur == c->device) {
             std::lock_guard<std::mutex> lk(c->mail.mu);
-            give(read_route(c, c->nets.h_rptr[net], rc));
-            return;
+            if (c->mail.open()) {
+                give(read_route(c, c->nets.h_rptr[net], rc));
+                return;
+            }
         }
         std::vector<int> tmp(rc);
         HIP_OK(hipMemcpyAsync(tmp.data(), c->nets.h_rptr[net], sizeof(int) * rc, hipMemcpyDeviceToHost, c->stream));

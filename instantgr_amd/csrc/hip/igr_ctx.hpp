@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstring>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -63,22 +64,44 @@ struct Mailbox {
     int* word = nullptr;    // host address
     int* dev = nullptr;     // the same memory to the device
     int reads = 0;
+    bool failed = false;    // no memory for it; not asked for again
     ~Mailbox() {
         if (word) (void)hipHostFree(word);
+    }
+    // Whether there is one (needs mu); without pinned memory there is none, and
+    // routes are copied.
+    bool open() {
+        if (word || failed) return word != nullptr;
+        int* w = nullptr;
+        void* d = nullptr;
+        failed = hipHostMalloc(reinterpret_cast<void**>(&w), sizeof(int) * (MAIL_HEAD + MAIL_WORDS),
+                               hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+                 hipHostGetDevicePointer(&d, w, 0) != hipSuccess;
+        if (failed) {
+            (void)hipGetLastError();
+            if (w) (void)hipHostFree(w);
+            return false;
+        }
+        std::memset(w, 0, sizeof(int) * (MAIL_HEAD + MAIL_WORDS));
+        word = w;
+        dev = static_cast<int*>(d);
+        return true;
     }
 };
 
 // Pinned slots for large copies to and from pageable memory (staging.hip): 16
-// MiB a context, allocated by its first large copy.  'mu' lets one copy at a
-// time use them; done[k] is the last copy through slot k.
+// MiB a context, allocated by its first large copy (where that fails, copies are
+// the runtime's).  'mu' lets one copy at a time use them; done[k] is the last
+// copy through slot k.
 struct Staging {
     static constexpr int SLOTS = 8, THREADS = 4;
     static constexpr int64_t SLOT_BYTES = 2 << 20, MIN_BYTES = 1 << 20;
     std::mutex mu;
     char* mem = nullptr;
+    bool failed = false;    // no pinned memory or events; not asked for again
     hipEvent_t done[SLOTS] = {};
     ~Staging();
-    void open(int device);
+    bool open(int device);
     char* slot(int k) { return mem + k * SLOT_BYTES; }
 };
 
@@ -524,8 +547,8 @@ void launch_pattern_order(igr_ctx* c, const int* d_order, int64_t n, int nb, int
 void launch_dag_measure(igr_ctx* c, int64_t n, int64_t edges, hipStream_t s);
 void launch_dag_order(igr_ctx* c, const int* d_nets, int64_t n, int nb, bool deep_first, DagBound* h_bound, int* h_big);
 // Net's route (rc words of room, at most MAIL_WORDS) from device memory into
-// the context's mailbox, after all work on the stream; returns its host address.
-// Needs c->mail.mu.
+// the context's open mailbox, after all work on the stream; returns its host
+// address.  Needs c->mail.mu.
 const int* read_route(igr_ctx* c, const int* src, int64_t rc);
 inline int host_threads() { return std::max(1, std::min(16, (int)std::thread::hardware_concurrency())); }
 // Copies between the device and pageable memory, after all work on the stream.

@@ -17,21 +17,25 @@ Staging::~Staging() {
     if (mem) (void)hipHostFree(mem);
 }
 
-// The events belong to the context's device, whichever the caller has current.
-void Staging::open(int device) {
-    if (mem) return;
+// Whether the slots are there.  The events belong to the context's device,
+// whichever the caller has current.
+bool Staging::open(int device) {
+    if (mem || failed) return mem != nullptr;
     int cur = -1;
     HIP_OK(hipGetDevice(&cur));
     if (cur != device) HIP_OK(hipSetDevice(device));
     char* m = nullptr;
-    bool ok = hipHostMalloc(&m, (size_t)SLOTS * SLOT_BYTES) == hipSuccess;
+    bool ok = hipHostMalloc(reinterpret_cast<void**>(&m), (size_t)SLOTS * SLOT_BYTES, 0) == hipSuccess;
     for (hipEvent_t& e : done) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
     if (cur != device) (void)hipSetDevice(cur);
-    if (!ok) {
+    failed = !ok;
+    if (failed) {
+        (void)hipGetLastError();
         if (m) (void)hipHostFree(m);
-        throw std::runtime_error("no pinned memory or events for large copies");
+        return false;
     }
     mem = m;
+    return true;
 }
 
 // Chunk k goes through slot k % SLOTS; thread t owns the slots t, t + T, ..,
@@ -51,15 +55,24 @@ static void over_chunks(int device, int64_t bytes, F&& chunk) {
     });
 }
 
+// The slots for a copy of this size, held while the lock lives; none for a small
+// copy and without pinned memory.
+static std::unique_lock<std::mutex> use_slots(igr_ctx* c, int64_t bytes) {
+    Staging& g = c->staging;
+    if (bytes < Staging::MIN_BYTES) return {};
+    std::unique_lock<std::mutex> lk(g.mu);
+    if (!g.open(c->device)) return {};
+    return lk;
+}
+
 void copy_to_host(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipStream_t s) {
     Staging& g = c->staging;
-    if (bytes < Staging::MIN_BYTES) {
+    const auto slots = use_slots(c, bytes);
+    if (!slots) {
         HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         HIP_OK(hipStreamSynchronize(s));
         return;
     }
-    std::lock_guard<std::mutex> lk(g.mu);
-    g.open(c->device);
     const auto start = [&](int slot, int64_t at) {
         HIP_OK(hipMemcpyAsync(g.slot(slot), static_cast<const char*>(src) + at,
                               std::min<int64_t>(Staging::SLOT_BYTES, bytes - at), hipMemcpyDeviceToHost, s));
@@ -79,12 +92,11 @@ void copy_to_host(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipStre
 
 void copy_to_device(igr_ctx* c, void* dst, const void* src, int64_t bytes, hipStream_t s) {
     Staging& g = c->staging;
-    if (bytes < Staging::MIN_BYTES) {
+    const auto slots = use_slots(c, bytes);
+    if (!slots) {
         if (bytes) HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
         return;
     }
-    std::lock_guard<std::mutex> lk(g.mu);
-    g.open(c->device);
     over_chunks(c->device, bytes, [&](int slot, int64_t at, int64_t len) {
         HIP_OK(hipEventSynchronize(g.done[slot]));
         std::memcpy(g.slot(slot), static_cast<const char*>(src) + at, len);
