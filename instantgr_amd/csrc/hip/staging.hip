@@ -46,12 +46,15 @@ static void over_chunks(int device, int64_t bytes, F&& chunk) {
     int T = std::max(1, std::min(std::min(host_threads(), Staging::THREADS), (int)std::min<int64_t>(Staging::SLOTS, chunks)));
     while (Staging::SLOTS % T) T--;
     igr::parallel_ranges(T, T, [&](int64_t a, int64_t b, int) {
-        if (T > 1) HIP_OK(hipSetDevice(device));   // a thread of its own; one chunk is copied by the caller
+        int cur = -1;   // a thread of its own has device 0; the caller keeps the one it has
+        HIP_OK(hipGetDevice(&cur));
+        if (cur != device) HIP_OK(hipSetDevice(device));
         for (int64_t t = a; t < b; t++)
             for (int64_t k = t; k < chunks; k += T) {
                 const int64_t at = k * Staging::SLOT_BYTES;
                 chunk((int)(k % Staging::SLOTS), at, std::min<int64_t>(Staging::SLOT_BYTES, bytes - at));
             }
+        if (cur != device) (void)hipSetDevice(cur);
     });
 }
 
