@@ -67,7 +67,8 @@ int igr_create(const igr_grid_desc* desc, igr_ctx** out);
 void igr_destroy(igr_ctx* ctx);
 const char* igr_last_error(void);
 
-/* Grid state (reference layout on the host side). */
+/* Grid state (reference layout on the host side).  Demand may be any float:
+ * passes add and subtract whole and half tracks in FP32, batch by batch. */
 int igr_set_demand(igr_ctx* ctx, const float* demand);
 int igr_get_demand(igr_ctx* ctx, float* demand);
 int igr_get_timestamp(igr_ctx* ctx, int* ts);

@@ -7,8 +7,8 @@
 // net's rank within it, a scan turns the counts into positions.  Bound by
 // launches and the counters' atomics (0.2-0.3 ms a kernel where half a million
 // nets share a few hundred keys).  On the host the same preparation took 34 ms of
-// a 438k-net DAG pass (205 -> 175 ms in all) and 5 ms of a 500k-net pattern
-// pass (35 -> 31 ms), between the scheduler and the first routing kernel.
+// a 438k-net DAG pass (205 -> 166 ms in all) and 3 ms of a 500k-net pattern
+// pass (35 -> 31.6 ms), between the scheduler and the first routing kernel.
 #include "igr_ctx.hpp"
 
 namespace igr_dev {
