@@ -13,7 +13,7 @@ from test_gpu_lshape_rows import _trees
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("metals,n", [(3, 5119), (3, 5121), (7, 5120), (10, 5120), (10, 5122), (10, 5123), (13, 5121)])
+@pytest.mark.parametrize("metals,n", [(3, 5119), (3, 5121), (7, 5120), (7, 5122), (10, 5120), (10, 5122), (10, 5123), (13, 5121)])
 def test_batch_sizes(metals, n):
     X, Y = 60, 50
     d = Design.custom(layers=metals, xsize=X, ysize=Y, nets=10, pin_cap=4, sigma=6.0, seed=metals).build(2)
